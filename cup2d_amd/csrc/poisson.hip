@@ -14,8 +14,10 @@
 //    scalar (alpha, omega, beta, restart, convergence) lives on the device;
 //    a reduction is finished by its consumer kernel, which re-reduces the
 //    producer's per-workgroup partials (no device-wide fences or atomics);
-//  * iterations are replayed in chunks from a hipGraph; kernels of a
-//    finished solve exit at launch on the device-side `done` flag;
+//  * meshes of up to 16,384 blocks are solved on chip, by one kernel for the
+//    whole solve (team.hip); larger ones (and a solve whose launch on chip
+//    failed) replay iterations in chunks from a hipGraph, whose kernels
+//    exit at launch on the device-side `done` flag once the solve is done;
 //  * mixed precision: FP64 iterative refinement (r = b - A x and x += d in
 //    FP64) around an inner BiCGSTAB with FP32 vectors and SpMV, FP64
 //    accumulation of every inner product, and the block preconditioner as a
@@ -38,6 +40,7 @@
 #include "assembly.h"
 #include "kernels.h"
 #include "flow.h"
+#include "team.h"
 
 using namespace cup2d;
 
@@ -878,6 +881,7 @@ struct cup2d_ps {
   double *d_h = nullptr;                 // cell size per block
   int ell_w = 0;
   long long n_exc = 0;                   // explicit rows
+  int n_codes = 0;                       // entries of etab
   bool has_csr = false;                  // plain CSR copy present (host-assembled meshes)
   int *d_csr_rp = nullptr, *d_csr_col = nullptr;
   double *d_csr_val = nullptr;
@@ -896,7 +900,13 @@ struct cup2d_ps {
   double h_min = 0.0;                    // smallest cell size of the mesh
   double *d_u = nullptr;                 // scalars of the unfused comparator (UScal + constants)
   double *d_p2 = nullptr, *d_p4 = nullptr, *d_p5 = nullptr, *d_pm = nullptr, *d_pfin = nullptr;
-  Scal *h_s = nullptr;                   // pinned copy of the state slots
+  Scal *h_s = nullptr;                   // pinned copy of the state slots, then of the team's control words
+  // the on-chip solve (team.hip): its launch shape for this mesh (-1: the
+  // mesh is too large for it, or a launch failed) and its device words
+  int team_shape = -1;
+  bool team_failed = false;
+  TeamTask team{};
+  unsigned char *d_team = nullptr;
   int G = 1;                             // workgroups of the SpMV / vector kernels
   int Gb = 1;                            // of which the block part of the operator kernels
   int Gp = 1;                            // workgroups of the FP64 preconditioner kernels
@@ -1233,6 +1243,78 @@ int solve_fp64(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   return CUP2D_PS_OK;
 }
 
+// Device words of an on-chip solve: control, phase times, exchange slots.
+constexpr double TEAM_TICK_MS = 1e-5;  // wall_clock64: 100 MHz
+constexpr size_t TEAM_PHASE_AT = 64, TEAM_SLOTS_AT = 128;
+constexpr size_t TEAM_BYTES = TEAM_SLOTS_AT + team_words(TEAM_MAX_WG) * 8;
+
+bool team_on(const cup2d_ps *h) { return h->cfg.schedule == 0 && h->team_shape >= 0 && !h->team_failed; }
+
+// The whole solve on chip (team.hip), in FP64.  A mixed handle's solve takes
+// it too -- vectors that never leave the registers gain nothing from FP32
+// storage -- and keeps its stopping rule: convergence is accepted on the
+// recomputed FP64 residual only.  `done` is false when the launch could not
+// run to its end (the caller falls back to the launch-per-kernel solve).
+int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out, double tol_abs,
+               double tol_rel, int max_restarts, cup2d_ps_stats *st, bool &done) {
+  done = false;
+  Scal m = marker_state(h, tol_abs, tol_rel, max_restarts, h->cfg.max_iter);
+  m.project = m.stall = 0;
+  m.rep_factor = h->mixed ? 1e-300 : 0.0;  // a replacement only where convergence is claimed
+  h->h_s[0] = h->h_s[1] = m;
+  int *ctl = reinterpret_cast<int *>(h->h_s + 2);
+  TeamArgs a{};
+  a.A = view(h);
+  a.fid = h->d_fid;
+  a.pf = h->d_P;
+  a.b = d_b;
+  a.x0 = d_x0;
+  a.out = h->d_x;  // d_out, which may be x0, is written once the launch has succeeded
+  a.halo = h->d_z1;  // z1, z2 and t
+  a.n_codes = h->n_codes;
+  a.xopt = h->d_xopt;
+  a.one = h->team;
+  a.n_tasks = 1;
+  a.n_tickets = h->team.nwg;
+  a.start = h->mixed ? TEAM_ACCEPTS : TEAM_PLAIN;
+  a.gen = h->op.mean_row >= 0 || h->cfg.norm == CUP2D_PS_NORM_INF;
+  a.form_polls = TEAM_POLLS;
+  a.st = h->d_s;
+  a.ctl = reinterpret_cast<int *>(h->d_team);
+  a.phase = h->cfg.profile ? reinterpret_cast<unsigned long long *>(h->d_team + TEAM_PHASE_AT) : nullptr;
+  a.slots = reinterpret_cast<unsigned long long *>(h->d_team + TEAM_SLOTS_AT);
+  HIPCHK(h, hipEventRecord(h->ev0, h->stream));
+  HIPCHK(h, hipMemcpyAsync(h->d_s, h->h_s, sizeof(Scal), hipMemcpyHostToDevice, h->stream));
+  HIPCHK(h, team_launch(a, h->team_shape, team_words(h->team.nwg), h->team.nwg, h->stream));
+  HIPCHK(h, hipEventRecord(h->ev1, h->stream));
+  ptick(h, -1);
+  HIPCHK(h, hipMemcpyAsync(h->h_s, h->d_s, sizeof(Scal), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipMemcpyAsync(ctl, h->d_team, TEAM_SLOTS_AT, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  if (ctl[1]) return CUP2D_PS_OK;
+  done = true;
+  HIPCHK(h, hipMemcpyAsync(d_out, h->d_x, h->op.n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+  const Scal &f = h->h_s[0];
+  if (h->mixed && f.err0 != f.err0) return fail(h, CUP2D_PS_EINVAL, "non-finite residual (NaN/Inf in b or x0)");
+  if (h->cfg.profile) {
+    const auto *ph = reinterpret_cast<const unsigned long long *>(reinterpret_cast<unsigned char *>(ctl) + TEAM_PHASE_AT);
+    for (int k = 0; k < TEAM_PHASES; k++) h->pms[k] += (double)ph[k] * TEAM_TICK_MS;
+  }
+  if (st) {
+    std::memset(st, 0, sizeof(*st));
+    st->iterations = std::max(f.iter, 0);
+    st->restarts = f.restarts;
+    st->converged = f.converged;
+    st->refinements = f.n_rep;
+    st->err_init = f.err0;
+    st->err_final = h->mixed && f.converged && f.n_rep > 0 ? f.err_rep : f.err_opt;
+    float ms = 0;
+    HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
+    st->ms = ms;
+  }
+  return CUP2D_PS_OK;
+}
+
 // FP64 norms of r = b - A x from the k_init partials (host side).
 int outer_residual(cup2d_ps *h, double &err) {
   std::vector<double> part(NQ5 * (size_t)h->G);
@@ -1512,7 +1594,15 @@ int solve_impl(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   HIPCHK(h, hipSetDevice(h->device));
   return guarded(h, [&]() -> int {
     pstart(h);
-    int rc = h->cfg.schedule == 1
+    int rc = CUP2D_PS_OK;
+    bool done = false;
+    if (team_on(h)) {
+      rc = solve_team(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st, done);
+      if (rc) return rc;
+      h->team_failed = !done;
+    }
+    if (!done)
+      rc = h->cfg.schedule == 1
                  ? solve_unfused(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st)
                  : h->mixed ? solve_mixed(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st)
                             : solve_fp64(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st);
@@ -1547,7 +1637,7 @@ int solve_impl(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
 constexpr long long NOALLOC_N = CUP2D_PS_NOALLOC_MAX_N;   // unknowns
 constexpr size_t NOALLOC_GT = MAXG + MAXGE;                 // partial slots per quantity
 constexpr size_t NOALLOC_SCAL = 2 * ((sizeof(Scal) + 255) / 256) * 32;  // doubles: 2 slots, 256-byte aligned
-constexpr size_t NOALLOC_DOUBLES = NOALLOC_SCAL + 9 * (size_t)NOALLOC_N + 17 * NOALLOC_GT + 8;
+constexpr size_t NOALLOC_DOUBLES = NOALLOC_SCAL + 9 * (size_t)NOALLOC_N + 17 * NOALLOC_GT + 8 + TEAM_BYTES / 8;
 static_assert(NOALLOC_N % 64 == 0, "the work vectors are whole blocks");
 
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
@@ -1574,15 +1664,16 @@ int scratch_address(int dev, double *&out) {
 struct WorkBufs {
   double *x, *xopt, *r, *rhat, *p, *nu, *z1, *z2, *t, *p2, *p4, *p5, *pm, *pfin;
   Scal *s;
+  unsigned char *team;
 };
 WorkBufs get_bufs(const cup2d_ps *h) {
   return WorkBufs{h->d_x, h->d_xopt, h->d_r, h->d_rhat, h->d_p, h->d_nu, h->d_z1, h->d_z2, h->d_t,
-                  h->d_p2, h->d_p4, h->d_p5, h->d_pm, h->d_pfin, h->d_s};
+                  h->d_p2, h->d_p4, h->d_p5, h->d_pm, h->d_pfin, h->d_s, h->d_team};
 }
 void set_bufs(cup2d_ps *h, const WorkBufs &b) {
   h->d_x = b.x; h->d_xopt = b.xopt; h->d_r = b.r; h->d_rhat = b.rhat; h->d_p = b.p;
   h->d_nu = b.nu; h->d_z1 = b.z1; h->d_z2 = b.z2; h->d_t = b.t; h->d_p2 = b.p2; h->d_p4 = b.p4;
-  h->d_p5 = b.p5; h->d_pm = b.pm; h->d_pfin = b.pfin; h->d_s = b.s;
+  h->d_p5 = b.p5; h->d_pm = b.pm; h->d_pfin = b.pfin; h->d_s = b.s; h->d_team = b.team;
 }
 // The same buffers carved out of the scratch array for n unknowns.
 WorkBufs scratch_bufs(double *base, size_t n) {
@@ -1599,6 +1690,7 @@ WorkBufs scratch_bufs(double *base, size_t n) {
   b.p5 = b.p4 + 4 * NOALLOC_GT;
   b.pm = b.p5 + NQ5 * NOALLOC_GT;
   b.pfin = b.pm + NOALLOC_GT;
+  b.team = reinterpret_cast<unsigned char *>(b.pfin + 4 * NOALLOC_GT);
   return b;
 }
 
@@ -1630,7 +1722,11 @@ int solve_noalloc_body(cup2d_ps *h, const double *d_b, double *d_x, double tol_a
   h->cfg.use_graph = 0;
   h->cfg.profile = 0;
   int rc = guarded(h, [&]() -> int {
-    int r = solve_fp64(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st);
+    bool done = false;
+    int r = team_on(h) ? solve_team(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st, done) : CUP2D_PS_OK;
+    if (r) return r;
+    if (team_on(h)) h->team_failed = !done;
+    if (!done) r = solve_fp64(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st);
     if (r) return r;
     // true residual of the returned x: partials of |r|^2, |r|_inf, |b|^2,
     // |b|_inf, each reduced by one workgroup into scratch
@@ -1707,7 +1803,7 @@ static int create_body(const cup2d_ps_config *cfg, cup2d_ps **out) {
     return fail(nullptr, CUP2D_PS_EHIP, "hipGetSymbolAddress of the work space failed");
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess ||
-      hipHostMalloc((void **)&h->h_s, 2 * sizeof(Scal), hipHostMallocDefault) != hipSuccess) {
+      hipHostMalloc((void **)&h->h_s, 2 * sizeof(Scal) + TEAM_SLOTS_AT, hipHostMallocDefault) != hipSuccess) {
     cup2d_ps_destroy(h.release());  // releases whichever of them were made
     return fail(nullptr, CUP2D_PS_EHIP, "stream/event/pinned allocation failed");
   }
@@ -1785,9 +1881,32 @@ static int set_mesh_body(cup2d_ps *h, const cup2d_mesh_desc *m) {
       (rc = upload(h, &h->d_csr_col, op.col)) || (rc = upload(h, &h->d_csr_val, op.val)))
     return rc;
   h->n_exc = (long long)n_exc;
+  h->n_codes = (int)ell.values.size();
   h->has_csr = true;
   if ((rc = upload_h(h, m))) return rc;
   return finish_mesh(h);
+}
+
+// The on-chip solve's team for the mesh: the fewest blocks per workgroup
+// whose workgroups all fit on the device at once -- an iteration of a uniform
+// mesh took 14.2 us with 16 blocks per workgroup, 14.9 with 32 and 19.5 with
+// 64 on 1536 blocks, 18.4 with 32 and 21.6 with 64 on 8192 -- but 16 blocks
+// only up to 192 workgroups: on 3072 blocks 16 and 32 were alike (15.9), on
+// 4096 32 was faster (16.1 against 17.0), the larger team's sums taking longer
+// than the shorter product saves.
+constexpr int TEAM_16_MOST = 192;
+static void plan_team(cup2d_ps *h) {
+  h->team_shape = -1;
+  for (int s = 0; s < TEAM_SHAPES; s++) {
+    TeamTask t{};
+    team_split((int)std::min<long long>(h->op.nb, 1 << 30), team_blocks(s), t);
+    if (t.nwg > std::min(s == TEAM_16 ? TEAM_16_MOST : TEAM_MAX_WG, team_resident(s))) continue;
+    t.e1 = (int)h->n_exc;
+    t.mean_row = (int)h->op.mean_row;
+    h->team = t;
+    h->team_shape = s;
+    return;
+  }
 }
 
 // The block preconditioner, the work vectors and the launch shapes: the part
@@ -1801,18 +1920,22 @@ static int finish_mesh(cup2d_ps *h) {
   if ((rc = upload(h, &h->d_P, pf64)) || (rc = dalloc(h, &h->d_pf, 8 * 64))) return rc;
   HIPCHK(h, hipMemcpy(h->d_pf, pf.data(), pf.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
   const size_t n = op.n;
-  double **vecs[] = {&h->d_x, &h->d_xopt, &h->d_r, &h->d_rhat, &h->d_p, &h->d_nu,
-                     &h->d_z1, &h->d_z2, &h->d_t, &h->d_b, &h->d_xio};
+  double **vecs[] = {&h->d_x, &h->d_xopt, &h->d_r, &h->d_rhat, &h->d_p, &h->d_nu, &h->d_b, &h->d_xio};
   for (double **v : vecs)
     if ((rc = dalloc(h, v, n))) return rc;
+  if ((rc = dalloc(h, &h->d_z1, 3 * n))) return rc;  // one buffer: the on-chip solve's halo takes all three
+  h->d_z2 = h->d_z1 + n;
+  h->d_t = h->d_z2 + n;
   float **fvecs[] = {&h->f_r, &h->f_rhat, &h->f_p, &h->f_nu, &h->f_z1, &h->f_z2, &h->f_t};
   for (float **v : fvecs)
     if ((rc = dalloc(h, v, h->mixed ? n : 64))) return rc;
   const size_t GT = MAXG + MAXGE;
   if ((rc = dalloc(h, &h->d_s, 2)) || (rc = dalloc(h, &h->d_u, 16)) || (rc = dalloc(h, &h->d_p2, 2 * GT)) ||
       (rc = dalloc(h, &h->d_p4, 4 * GT)) || (rc = dalloc(h, &h->d_p5, NQ5 * GT)) ||
-      (rc = dalloc(h, &h->d_pm, GT)) || (rc = dalloc(h, &h->d_pfin, 4 * GT)))
+      (rc = dalloc(h, &h->d_pm, GT)) || (rc = dalloc(h, &h->d_pfin, 4 * GT)) ||
+      (rc = dalloc(h, &h->d_team, TEAM_BYTES)))
     return rc;
+  plan_team(h);
   HIPCHK(h, hipMemset(h->d_s, 0, 2 * sizeof(Scal)));
   const long long waves = (op.nb + SPMV_U - 1) / SPMV_U;
   h->Gb = (int)std::max<long long>(1, std::min<long long>(MAXG, (waves + WAVES - 1) / WAVES));
@@ -1873,6 +1996,7 @@ static int set_mesh_on_device_body(cup2d_ps *h, const cup2d_mesh_desc *m) {
   h->d_ewid = D.ewid;
   h->ell_w = D.ell_w;
   h->n_exc = D.n_exc;
+  h->n_codes = D.n_codes;
   h->has_csr = false;
   if (const int hr = upload_h(h, m)) return hr;
   h->d_csr_rp = h->d_csr_col = nullptr;

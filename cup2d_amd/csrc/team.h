@@ -1,0 +1,90 @@
+// team.h -- the on-chip solve: one kernel runs whole FP64 BiCGSTAB solves
+// with the vectors held in registers (team.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <string>
+#include <vector>
+
+#include "kernels.h"
+
+namespace cup2d {
+
+// One solve of a launch: blocks b0 .. b0 + nb - 1 of the operator, taken by a
+// team of nwg workgroups of bpw consecutive blocks each (the last one fewer).
+struct TeamTask {
+  int b0, nb;
+  int nwg, bpw;
+  int ticket0;        // first ticket of the team: workgroup `rank` holds ticket0 + rank
+  int slot0;          // first of the team's exchange words, in units of TEAM_SLOT_WORDS
+  int e0, e1;         // explicit rows (ELL slots) of these blocks
+  int mean_row;       // replaced row, or -1
+  int pad;
+};
+
+constexpr int TEAM_MAX_WG = 256;        // workgroups of a team: at most one per CU
+constexpr int TEAM_MAX_BLOCKS = 64 * TEAM_MAX_WG;  // largest mesh solved on chip
+constexpr int TEAM_PHASES = 5;          // cup2d_ps_phase
+
+// Words of the exchange area per workgroup slot (see team.hip).
+constexpr int TEAM_NQ = 4;              // quantities of one exchange
+constexpr int TEAM_SLOT_WORDS = 2 * 2 * TEAM_NQ;
+// Copies of the exchange words: one per 32 workgroups.
+__host__ __device__ constexpr int team_copies(int nwg) { return (nwg + 31) / 32; }
+// Exchange words of a team.
+constexpr size_t team_words(int nwg) { return (size_t)nwg * TEAM_SLOT_WORDS * team_copies(nwg); }
+
+struct TeamArgs {
+  OpView A;
+  const int2 *fid;
+  const double *pf;                     // FP64 MFMA fragments of P_inv
+  const double *b, *x0;
+  double *out;
+  double *halo;                         // [3 n] what the workgroups read of each other
+  double *xopt;                         // [n] work vector
+  int n_codes;                          // entries of A.etab
+  const TeamTask *task;                 // [n_tasks], or null: the one task `one`
+  TeamTask one;
+  int n_tasks, n_tickets;
+  int start;                            // TeamStart
+  int gen;                              // a mean row or the infinity norm among the tasks
+  int form_polls;                       // polls before the wait for a team to form fails
+  Scal *st;                             // [n_tasks] marker state in, final state out
+  unsigned long long *slots;            // exchange words of all teams, zero at launch
+  int *ctl;                             // {next ticket, failure}, zero at launch
+  unsigned long long *phase;            // [n_tasks][TEAM_PHASES] ticks of 10 ns, or null
+};
+
+// What the start of a solve (and of a residual replacement) also decides.
+enum TeamStart {
+  TEAM_PLAIN = 0,     // nothing (the FP64 single solve: evaluate alone)
+  TEAM_CHECKED = 1,   // a non-finite residual ends the solve, a zero one is convergence
+  TEAM_ACCEPTS = 2,   // ... and a start within the tolerance is convergence too
+};
+
+// Blocks per workgroup of a launch shape.
+enum TeamShape { TEAM_16 = 0, TEAM_32 = 1, TEAM_64 = 2, TEAM_SHAPES = 3 };
+inline int team_blocks(int shape) { return shape == TEAM_16 ? 16 : shape == TEAM_32 ? 32 : 64; }
+
+// Polls (0.5 us and more each) before a wait inside a team fails.
+constexpr int TEAM_POLLS = 1 << 21;
+
+// Workgroups of a shape that this device runs at once (0: unknown; the
+// kernels' LDS size is allowed here, so a shape is asked for before its launch).
+int team_resident(int shape);
+
+// Splits nb blocks over a team of workgroups of at most `most` blocks.
+inline void team_split(int nb, int most, TeamTask &t) {
+  t.nb = nb;
+  t.nwg = (nb + most - 1) / most;
+  t.bpw = (nb + t.nwg - 1) / t.nwg;
+  t.nwg = (nb + t.bpw - 1) / t.bpw;
+}
+
+// Launches the solves on `stream` with `grid` workgroups, no more than
+// team_resident and no fewer than any task's team (the exchange words and ctl
+// are cleared first).  Nothing is allocated.
+hipError_t team_launch(const TeamArgs &a, int shape, size_t n_words, int grid, hipStream_t stream);
+
+}  // namespace cup2d

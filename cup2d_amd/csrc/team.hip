@@ -1,0 +1,874 @@
+// team.hip -- whole FP64 BiCGSTAB solves in one kernel.
+//
+// The iteration of BiCGSTAB.cu:412-620 (restart, best iterate, stopping
+// norms) with the vectors r, rhat, p, nu, z, t and x of a workgroup's blocks in
+// its registers for the whole solve.  A team of co-resident workgroups
+// advances one mesh; the only data that leave a workgroup are the cells of
+// z = P v that another workgroup's rows read (the operator's halo) and the
+// partial sums of the dot products.
+//
+// What bounds it: an iteration has five points where the workgroups wait for
+// each other (z's halo twice, (rhat, nu), omega's two sums, the update's sums),
+// each one store and one load past the L2s, which are not coherent between
+// the XCDs: 0.7-1 us for a halo, 1.0 us (8 workgroups) to 2 us (250) for sums.
+// A fence that writes an L2 back costs more than a kernel boundary; here every
+// shared word is written and read by relaxed agent-scope accesses, and a
+// waiting workgroup polls the data themselves: partial sums carry the
+// exchange's number in the upper half of each word, and a halo word holds a
+// NaN that no arithmetic returns until its value arrives.  Between the waits a
+// wave's instructions count (one or two waves per SIMD): the loop is one copy
+// of the code for both halves of an iteration (the instruction cache), its
+// branches are uniform, and everything an explicit row needs lies in LDS.
+//
+// Measured (us per iteration to a relative residual of 1e-10, against five
+// kernels per iteration replayed from a graph): 128 blocks 11.9 against 24.0,
+// 1448 blocks 14.5 against 27.9, 8348 blocks 23.7 against 49.9, 16,229 blocks
+// 29.2 against 64.8.  On 16k blocks the products (2 x 8192 flop per block at
+// the 72 TFLOP/s of a large FP64 matrix product) are 3.7 us of it.
+//
+// Teams form by tickets: a workgroup takes the next ticket, which names its
+// task and its rank, and when its task is solved takes another.  Tickets are
+// taken in order by running workgroups, so the lowest unfinished task always
+// has or gets its whole team (a cooperative launch: no more workgroups than
+// fit) and every wait ends; a wait beyond its limit marks the launch as
+// failed and every workgroup leaves.
+
+#include "team.h"
+
+#include <atomic>
+
+namespace cup2d {
+namespace {
+
+typedef unsigned long long u64;
+
+constexpr int ZS = 66;                    // LDS row of a block: 16-byte aligned, 16 blocks over all banks
+constexpr int TEAM_MAX_CONFIRM = 64;      // residual confirmations of a mixed solve
+
+__device__ __forceinline__ u64 ld_agent(const u64 *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(u64 *p, u64 v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// N pairs of words (16 bytes each, past the caches), the wait included.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void ld_pairs(const u64 *p0, u32x4 &v0) {
+  asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v0) : "v"(p0) : "memory");
+}
+__device__ __forceinline__ void ld_pairs(const u64 *p0, const u64 *p1, u32x4 &v0, u32x4 &v1) {
+  asm volatile(
+      "global_load_dwordx4 %0, %2, off sc1\n\tglobal_load_dwordx4 %1, %3, off sc1\n\ts_waitcnt vmcnt(0)"
+      : "=&v"(v0), "=&v"(v1)
+      : "v"(p0), "v"(p1)
+      : "memory");
+}
+__device__ __forceinline__ void ld_pairs(const u64 *p0, const u64 *p1, const u64 *p2, const u64 *p3, u32x4 &v0,
+                                         u32x4 &v1, u32x4 &v2, u32x4 &v3) {
+  asm volatile(
+      "global_load_dwordx4 %0, %4, off sc1\n\tglobal_load_dwordx4 %1, %5, off sc1\n\t"
+      "global_load_dwordx4 %2, %6, off sc1\n\tglobal_load_dwordx4 %3, %7, off sc1\n\ts_waitcnt vmcnt(0)"
+      : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
+      : "v"(p0), "v"(p1), "v"(p2), "v"(p3)
+      : "memory");
+}
+
+// A value that is the same in every lane, as the compiler sees it too: the
+// branches on it then keep one copy of the registers either side updates.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uni(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = uni((int)b), hi = uni((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Wave reductions by DPP (row shifts, then row broadcasts; the total in lane
+// 63): a step is two register moves and an add, where a shuffle through LDS
+// takes its latency.  Lanes without a source add 0; the maxima are of
+// absolute values, so 0 serves there too.
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <bool MAX>
+__device__ __forceinline__ double dpp_total(double v) {
+  auto op = [](double a, double b) { return MAX ? nmax(a, b) : a + b; };
+  v = op(v, dpp<0x111>(v));  // row_shr 1, 2, 4, 8
+  v = op(v, dpp<0x112>(v));
+  v = op(v, dpp<0x114>(v));
+  v = op(v, dpp<0x118>(v));
+  v = op(v, dpp<0x142>(v));  // row_bcast 15, 31
+  v = op(v, dpp<0x143>(v));
+  return v;
+}
+
+// A word of z that has not arrived: a signalling NaN, which no arithmetic
+// returns (an x0 that holds this very one fails the launch, not the solve:
+// the launch-per-kernel path takes over).
+constexpr u64 EMPTY = 0x7ff4c2d0a11c0de5ull;
+
+constexpr int face_rows(int blocks) { return blocks * 28; }  // a block has 28 cells on its faces
+constexpr int ENT = 14;                                      // entries of an explicit row kept in LDS (13 occur)
+constexpr int TAB = 256;                                     // coefficients kept in LDS
+
+template <int WGS, int T>
+struct Shared {
+  static constexpr int BPW = WGS / 256 * T * TILE, NW = WGS / 64;
+  static constexpr int GHOST0 = BPW * ZS, GHOSTS = BPW * 40;  // first, most cells of other workgroups
+  static constexpr int ITEMS = BPW * 12;                      // a block's 4 faces and 8 rows
+  static constexpr int ROWS = BPW == 64 ? 512 : face_rows(BPW);  // explicit rows kept in LDS
+  double z[GHOST0 + GHOSTS];        // the workgroup's blocks (product inputs, then z), then the ghosts
+  double2 pf[T == 1 ? 1 : 4 * 8 * 64];  // P_inv's fragments, two K steps a word
+  double ye[face_rows(BPW)];        // A z of the explicit rows
+  double tab[TAB];
+  double red[TEAM_NQ][NW], tot[TEAM_NQ];  // a wave per quantity: TEAM_NQ <= NW
+  u64 mask[BPW];
+  double h2[BPW];
+  int4 face[BPW];                   // where z across each face lies (Xm, Xp, Ym, Yp); the block's own cells
+                                    // where no plain neighbour does (a wall's term vanishes)
+  int ghost[GHOSTS];                // where in the halo buffer each ghost comes
+  unsigned ent[ENT][ROWS];          // entries of the explicit rows: LDS index, coefficient << 16
+  int erow[face_rows(BPW)];         // ELL slot of each explicit row
+  int eoff[BPW + 1];                // first explicit row of each block
+  unsigned char ewid[face_rows(BPW)];  // entries, | 128 when they are read from memory
+  int2 item[ITEMS];                 // what other workgroups read, 8 cells each: {first LDS index | stride 8 (bit
+                                    // 16), place in the halo buffer}
+  int ng, ni, ticket, bad;
+};
+
+// The running workgroup: what its functions share.
+template <int WGS, int T>
+struct Ctx {
+  typedef Shared<WGS, T> S;
+  const TeamArgs &a;
+  S &s;
+  int tid, lane, w, q, j, grp, c0;  // wave within its tile, MFMA column / k slot, first cell
+  TeamTask t;
+  int rank, b0, nb;                 // first block, blocks
+  u64 *slots;
+  int copies, copy, slab;           // copies of the exchange words, the one read here, words of a copy
+  unsigned ep, zp;                  // number of the exchange, parity of z's buffer
+  bool dead;
+
+  __device__ __forceinline__ Ctx(const TeamArgs &aa, S &ss) : a(aa), s(ss), dead(false) { place(); }
+
+  // The thread's place, computed anew: kept out of the compiler's sight, so
+  // that the dozens of addresses that follow from it are recomputed where
+  // they are used and don't hold registers through the loop (with T = 2 they
+  // pushed the vectors out to memory).
+  __device__ __forceinline__ void place() {
+    tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    lane = tid & 63;
+    q = lane >> 4;
+    j = lane & 15;
+    const int wv = uni(tid >> 6);
+    w = wv & 3;
+    grp = wv >> 2;
+    c0 = 16 * w + 4 * q;
+  }
+
+  __device__ __forceinline__ int lb(int tt) const { return (grp * T + tt) * TILE + j; }
+  __device__ __forceinline__ bool ok(int tt) const { return lb(tt) < nb; }
+  __device__ __forceinline__ long cell(int tt) const { return (long)(b0 + (ok(tt) ? lb(tt) : 0)) * 64 + c0; }
+  // the halo buffer of this z: the faces of every block (8 cells each, Xm, Xp,
+  // Ym, Yp), then every block whole; 64 bytes that one workgroup writes and
+  // another reads lie together
+  __device__ __forceinline__ double *halo() const { return a.halo + (zp ? 96l * a.A.nb : 0); }
+
+  // every 1024 polls: whether to give up (the launch failed, or the limit)
+  __device__ __forceinline__ bool give_up(int &n, int limit) {
+    if (((++n) & 1023) != 0) return false;
+    if (n < limit && !__hip_atomic_load(a.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
+    __hip_atomic_store(a.ctl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s.bad = 1;
+    return true;
+  }
+
+  // z at a cell of another workgroup, once it has arrived; v: a first look
+  __device__ __forceinline__ double remote(const double *p, u64 v, int limit) {
+    const u64 *w64 = reinterpret_cast<const u64 *>(p);
+    int n = 0;
+    while (v == EMPTY && !dead && !give_up(n, limit)) v = ld_agent(w64);
+    return __longlong_as_double((long long)v);
+  }
+
+  // The cells that others read go to the halo buffer (from LDS), or are
+  // emptied there.
+  template <bool EMPTIES>
+  __device__ __forceinline__ void publish(double *buf) {
+    const int n = 8 * uni(s.ni);
+    for (int i = tid; i < n; i += WGS) {
+      const int2 it = s.item[i >> 3];
+      const int c = i & 7;
+      u64 v = EMPTY;
+      if (!EMPTIES) v = (u64)__double_as_longlong(s.z[(it.x & 0xffff) + (it.x >> 16 ? 8 * c : c)]);
+      st_agent(reinterpret_cast<u64 *>(buf + 8 * (long)it.y + c), v);
+    }
+  }
+
+  // After the pass's last exchange everyone has read its z: the words are
+  // emptied (that is complete before the next exchange, which lies before
+  // their next use) and the other buffer is next.
+  __device__ __forceinline__ void clear() {
+    publish<true>(halo());
+    zp ^= 1;
+  }
+
+  // Sums (the last one a maximum with MAXLAST) of the NQ quantities over
+  // the team, in a fixed order, so that every workgroup holds the same totals:
+  // lanes, waves, ranks.  The totals are in s.tot.  A wave per quantity
+  // publishes the workgroup's sum and gathers the team's.
+  template <int NQ, bool MAXLAST>
+  __device__ __forceinline__ void exchange(double (&v)[NQ], int limit) {
+    const int wv = uni(tid >> 6);
+#pragma unroll
+    for (int k = 0; k < NQ; k++) v[k] = MAXLAST && k == NQ - 1 ? dpp_total<true>(v[k]) : dpp_total<false>(v[k]);
+    if (lane == 63)
+#pragma unroll
+      for (int k = 0; k < NQ; k++) s.red[k][wv] = v[k];
+    // what this workgroup emptied is empty before it says that it is here
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    ep++;
+    if (wv < NQ) {
+      const bool mx = MAXLAST && wv == NQ - 1;
+      auto op = [mx](double x, double y) { return MAXLAST && mx ? nmax(x, y) : x + y; };
+      const double2 *rp = reinterpret_cast<const double2 *>(s.red[wv]);
+      double r = 0.0;
+#pragma unroll
+      for (int i = 0; i < S::NW / 2; i++) {
+        const double2 u = rp[i];
+        r = op(op(r, u.x), u.y);
+      }
+      const int n = t.nwg;
+      if (n > 1) {
+        u64 *base = slots + ((ep & 1) ? slab * copies : 0) + 2 * wv * n;
+        const u64 b = (u64)__double_as_longlong(r), tag = (u64)ep << 32;
+        // Large teams write their sums in several copies, each read by some of
+        // the workgroups: a line that 250 workgroups poll is slow to reach.
+        if (lane < 2 * copies)
+          st_agent(base + (lane >> 1) * slab + 2 * rank + (lane & 1), tag | ((lane & 1) ? b >> 32 : b & 0xffffffffull));
+        const u64 *sk = base + copy * slab;
+        constexpr int NS = TEAM_MAX_WG / 64;
+        const u64 *p[NS];
+        u32x4 w4[NS];
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+          p[i] = sk + 2 * min(i * 64 + lane, n - 1);
+          w4[i] = u32x4{0, ep, 0, ep};
+        }
+        unsigned off;
+        int polls = 0;
+        do {
+          if (n > 128) ld_pairs(p[0], p[1], p[2], p[3], w4[0], w4[1], w4[2], w4[3]);
+          else if (n > 64) ld_pairs(p[0], p[1], w4[0], w4[1]);
+          else ld_pairs(p[0], w4[0]);
+          off = 0;
+#pragma unroll
+          for (int i = 0; i < NS; i++) off |= (w4[i].y ^ ep) | (w4[i].w ^ ep);
+        } while (off && !dead && !give_up(polls, limit));
+        r = 0.0;
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+          const double d = __longlong_as_double((long long)w4[i].z << 32 | w4[i].x);
+          r = op(r, i * 64 + lane < n ? d : 0.0);
+        }
+        r = MAXLAST && mx ? dpp_total<true>(r) : dpp_total<false>(r);
+      }
+      if (lane == 63) s.tot[wv] = r;
+    }
+    __syncthreads();
+    dead = dead || uni(s.bad) != 0;
+  }
+
+  __device__ __forceinline__ void to_lds(const double (&z)[T][4]) {
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+      double2 *d = reinterpret_cast<double2 *>(s.z + lb(tt) * ZS + c0);
+      d[0] = make_double2(z[tt][0], z[tt][1]);
+      d[1] = make_double2(z[tt][2], z[tt][3]);
+    }
+  }
+  __device__ __forceinline__ void from_lds(int i, double (&v)[4]) const {
+    const double2 *d = reinterpret_cast<const double2 *>(s.z + i);
+    const double2 u0 = d[0], u1 = d[1];
+    v[0] = u0.x; v[1] = u0.y; v[2] = u1.x; v[3] = u1.y;
+  }
+
+  // z = P z of the thread's cells.  The fragments of P are read while the
+  // inputs go through LDS, and the inputs of every tile before the first
+  // product: the 16 dependent products of a tile then wait on no load
+  // (read four at a time between the products, the LDS latency was paid
+  // four times a tile and the product took twice as long).
+  __device__ __forceinline__ void prec(const PFrag64 &F, double (&z)[T][4]) {
+    double2 f[8], u[8], un[8];
+    to_lds(z);
+#pragma unroll
+    for (int k = 0; k < 8; k++) f[k] = T == 1 ? make_double2(F.a[2 * k], F.a[2 * k + 1]) : s.pf[(w * 8 + k) * 64 + lane];
+    __syncthreads();
+    auto input = [&](int tt, double2 (&v)[8]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) v[k] = reinterpret_cast<const double2 *>(s.z + lb(tt) * ZS + 16 * q)[k];
+    };
+    input(0, u);
+    f64x4 acc[T];
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+      if (tt + 1 < T) input(tt + 1, un);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[tt] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].x, u[k].x, acc[tt], 0, 0, 0);
+        acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].y, u[k].y, acc[tt], 0, 0, 0);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++) u[k] = un[k];
+    }
+    // The product's results are read 20 and more cycles after the last
+    // instruction: said here, because the compiler's own count once let the
+    // high half of the first result be read early (the product was kept in
+    // accumulation registers then).
+    if constexpr (T == 1) asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]));
+    else asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[T - 1]));
+#pragma unroll
+    for (int tt = 0; tt < T; tt++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) z[tt][k] = acc[tt][k];
+    __syncthreads();  // the inputs are overwritten by z
+  }
+
+  // y = A z of the thread's cells (0 past the last block, where z is 0)
+  __device__ __forceinline__ void spmv(const double (&z)[T][4], double (&y)[T][4], int limit) {
+    const double *zb = halo();
+    to_lds(z);
+    __syncthreads();
+    publish<false>(halo());
+    const int ng = uni(s.ng);
+    for (int g = tid; g < ng; g += 2 * WGS) {  // two at a time: one round trip for most teams
+      const int g1 = g + WGS < ng ? g + WGS : g;
+      const double *p0 = zb + s.ghost[g], *p1 = zb + s.ghost[g1];
+      const u64 v0 = ld_agent(reinterpret_cast<const u64 *>(p0)), v1 = ld_agent(reinterpret_cast<const u64 *>(p1));
+      s.z[S::GHOST0 + g] = remote(p0, v0, limit);
+      s.z[S::GHOST0 + g1] = remote(p1, v1, limit);
+    }
+    __syncthreads();
+    const int ne = uni(s.eoff[nb]);
+    if (ne > 0) {
+      for (int k = tid; k < ne; k += WGS) {  // a thread per explicit row
+        const int width = s.ewid[k];
+        double sum = 0.0;
+        if (width < 128) {
+          for (int w0 = 0; w0 < width; w0 += ENT / 2) {
+            unsigned en[ENT / 2];
+#pragma unroll
+            for (int i = 0; i < ENT / 2; i++) en[i] = s.ent[w0 + i][k];
+#pragma unroll
+            for (int i = 0; i < ENT / 2; i++) sum += s.tab[en[i] >> 16] * s.z[en[i] & 0xffffu];
+          }
+        } else {
+          const int e = s.erow[k];
+          for (int i = 0; i < width - 128; i++) {
+            const long at = (long)i * a.A.n_exc + e;
+            const int col = a.A.ecol[at], l = (col >> 6) - b0;
+            const double v = (l >= 0 && l < nb) ? s.z[l * ZS + (col & 63)] : remote(zb + place_of(a.A.erow[e] >> 6, col), EMPTY, limit);
+            sum += a.A.etab[a.A.ecode[at]] * v;
+          }
+        }
+        s.ye[k] = sum;
+      }
+      __syncthreads();
+    }
+    const int row = 2 * w + (q >> 1), ix0 = 4 * (q & 1);
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+      const int base = lb(tt) * ZS;
+      const int4 f = s.face[lb(tt)];
+      const int fx = ix0 == 0 ? f.x : f.y;
+      const double mid = s.z[base + row * 8 + (ix0 == 0 ? 4 : 3)];  // across the middle of the row
+      const double hx = s.z[fx + (fx < S::GHOST0 ? 8 * row : row)];
+      double dn[4], up[4];
+      from_lds((row > 0 ? base + (row - 1) * 8 : f.z) + ix0, dn);
+      from_lds((row < 7 ? base + (row + 1) * 8 : f.w) + ix0, up);
+      const double lo = ix0 == 0 ? hx : mid, hi = ix0 == 0 ? mid : hx;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {  // face order Ym, Xm, Xp, Yp as the other operator kernels
+        const double xl = k > 0 ? z[tt][k > 0 ? k - 1 : 0] : lo;
+        const double xr = k < 3 ? z[tt][k < 3 ? k + 1 : 3] : hi;
+        y[tt][k] = ((dn[k] + xl) + xr) + up[k] - 4.0 * z[tt][k];
+      }
+      const u64 m = s.mask[lb(tt)];
+      const unsigned em = (unsigned)(m >> c0) & 15u;
+      if (em) {  // the block's explicit rows come in the order of its mask's bits
+        int at = s.eoff[lb(tt)] + __popcll(m & ((1ull << c0) - 1));
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          if ((em >> k) & 1u) y[tt][k] = s.ye[at++];
+      }
+    }
+  }
+
+  // Where in the halo buffer a cell of another workgroup comes, for a row of
+  // block b: with the face that a same-level neighbour shows b (the only
+  // cells of it that b's rows read), or with the whole block.
+  __device__ __forceinline__ int place_of(int b, int col) const {
+    const int4 n4 = a.A.nbr[b];
+    const int blk = col >> 6, ix = col & 7, iy = (col >> 3) & 7;
+    if (n4.x == blk && ix == 7) return (4 * blk + 1) * 8 + iy;
+    if (n4.y == blk && ix == 0) return (4 * blk + 0) * 8 + iy;
+    if (n4.z == blk && iy == 7) return (4 * blk + 3) * 8 + ix;
+    if (n4.w == blk && iy == 0) return (4 * blk + 2) * 8 + ix;
+    return 32 * a.A.nb + col;
+  }
+
+  // Headers, ghosts and explicit rows of the workgroup's blocks.
+  __device__ __forceinline__ void lay_out() {
+    if (tid == 0) s.ng = s.ni = 0;
+    __syncthreads();
+    // LDS index of 8 cells of another workgroup, from `first` of the halo buffer on
+    auto ghosts = [&](int first) -> int {
+      const int g = atomicAdd(&s.ng, 8);
+#pragma unroll 1
+      for (int i = 0; i < 8; i++) s.ghost[g + i] = first + i;
+      return S::GHOST0 + g;
+    };
+#pragma unroll 1
+    for (int l = tid; l < S::BPW; l += WGS) {
+      const bool in = l < nb;
+      const int b = b0 + (in ? l : 0);
+      const int4 n4 = a.A.nbr[b];
+      s.mask[l] = in ? a.A.mask[b] : 0ull;
+      s.h2[l] = in ? a.A.h2[b] : 0.0;
+      int at[4];
+      bool whole = false;
+      auto offer = [&](int base, bool column, int to) {
+        s.item[atomicAdd(&s.ni, 1)] = make_int2(l * ZS + base | (column ? 1 << 16 : 0), to);
+      };
+#pragma unroll 1
+      for (int f = 0; f < 4; f++) {
+        const int nv = f == 0 ? n4.x : f == 1 ? n4.y : f == 2 ? n4.z : n4.w;
+        at[f] = l * ZS + (f == 1 ? 7 : f == 3 ? 56 : 0);
+        if (!in) continue;
+        if (nv >= 0) {
+          if (nv >= b0 && nv < b0 + nb) {
+            at[f] = (nv - b0) * ZS + (f == 0 ? 7 : f == 2 ? 56 : 0);  // the neighbour's facing row
+          } else {
+            at[f] = ghosts((4 * nv + (f ^ 1)) * 8);
+            offer(f == 1 ? 7 : f == 3 ? 56 : 0, f < 2, 4 * b + f);
+          }
+        } else if (nv == -2) {
+          const int2 fd = a.fid[4 * (long)b + f];
+          // the rows beside a coarse-fine face read up to three cells deep
+          whole = whole || fd.x < b0 || fd.x >= b0 + nb || (fd.y >= 0 && (fd.y < b0 || fd.y >= b0 + nb));
+        }
+      }
+      if (whole)
+#pragma unroll 1
+        for (int i = 0; i < 8; i++) offer(8 * i, false, 4 * a.A.nb + 8 * b + i);
+      s.face[l] = make_int4(at[0], at[1], at[2], at[3]);
+    }
+    __syncthreads();
+    if (tid == 0) {
+      int n = 0;
+#pragma unroll 1
+      for (int l = 0; l <= S::BPW; l++) {
+        s.eoff[l] = n;
+        if (l < S::BPW) n += __popcll(s.mask[l]);
+      }
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int e = t.e0 + tid; e < t.e1; e += WGS) {
+      const int row = a.A.erow[e], l = (row >> 6) - b0;
+      if (l < 0 || l >= nb) continue;
+      const int k = s.eoff[l] + __popcll(s.mask[l] & ((1ull << (row & 63)) - 1));
+      s.erow[k] = e;
+      int width = 0;
+      bool fits = k < S::ROWS && a.A.ell_w <= ENT;
+#pragma unroll 1
+      for (int i = 0; i < a.A.ell_w; i++) {
+        const long at = (long)i * a.A.n_exc + e;
+        const unsigned code = a.A.ecode[at];
+        if (code) width = i + 1;
+        fits = fits && code < TAB;
+      }
+#pragma unroll 1
+      for (int i = 0; i < ENT && fits; i++) {  // entries past the row's end: 0.0 times its own value
+        const long at = (long)i * a.A.n_exc + e;
+        const unsigned code = i < width ? a.A.ecode[at] : 0;
+        const int col = i < width ? a.A.ecol[at] : row, lc = (col >> 6) - b0;
+        unsigned idx;
+        if (lc >= 0 && lc < nb) {
+          idx = lc * ZS + (col & 63);
+        } else {
+          const int g = atomicAdd(&s.ng, 1);
+          fits = g < S::GHOSTS;
+          if (fits) s.ghost[g] = place_of(row >> 6, col);
+          idx = S::GHOST0 + g;
+        }
+        if (fits) s.ent[i][k] = idx | code << 16;
+      }
+      s.ewid[k] = (unsigned char)(fits ? width : 128 + width);
+    }
+    __syncthreads();
+    if (tid == 0 && s.ng > S::GHOSTS) s.ng = S::GHOSTS;
+  }
+};
+
+#define CELLS                             \
+  _Pragma("unroll") for (int tt = 0; tt < T; tt++) _Pragma("unroll") for (int k = 0; k < 4; k++)
+
+// GEN: with the mean row and the infinity norm; without, the two sums of the
+// 2-norm on the operator's plain form.
+// Two waves' worth of registers at least are left to each wave (256): with
+// more, the compiler keeps products in the accumulation registers.
+template <int WGS, int T, bool GEN>
+__global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  typedef Shared<WGS, T> S;
+  static_assert(sizeof(S) <= 160 * 1024, "LDS of a CU");
+  static_assert(S::GHOST0 + S::GHOSTS <= 65536 && S::GHOSTS >= S::BPW * 32, "LDS indices");
+  S &s = *reinterpret_cast<S *>(smem);
+  Ctx<WGS, T> c(a, s);
+  const int &tid = c.tid;
+  PFrag64 F;  // one tile per wave: the fragments stay in registers; more: in LDS
+  if (T == 1)
+    load_pfrag64(F, a.pf, c.w, c.lane);
+  else
+    for (int i = tid; i < 4 * 8 * 64; i += WGS) {  // fragments (w, ks), lane -> (w, ks / 2), lane
+    const int at = (i >> 6) * 2 * 64 + (i & 63);
+    s.pf[i] = make_double2(a.pf[at], a.pf[at + 64]);
+  }
+  for (int i = tid; i < TAB; i += WGS) s.tab[i] = i < a.n_codes ? a.A.etab[i] : 0.0;
+  if (tid == 0) s.bad = 0;
+  auto tot = [&](int k) __attribute__((always_inline)) { return uni(s.tot[k]); };
+  for (;;) {
+    if (tid == 0)
+      s.ticket = __hip_atomic_fetch_add(a.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int tk = uni(s.ticket);
+    if (tk >= a.n_tickets || c.dead) break;
+    int id = 0;
+    if (a.task) {
+      int hi = a.n_tasks;  // the last task whose first ticket is not beyond this one
+      while (hi - id > 1) {
+        const int mid = (id + hi) >> 1;
+        if (a.task[mid].ticket0 <= tk) id = mid;
+        else hi = mid;
+      }
+      c.t = a.task[id];
+    } else {
+      c.t = a.one;
+    }
+    const TeamTask &t = c.t;
+    c.rank = tk - t.ticket0;
+    c.b0 = t.b0 + c.rank * t.bpw;
+    c.nb = min(t.bpw, t.nb - c.rank * t.bpw);
+    c.slots = a.slots + (size_t)t.slot0 * TEAM_SLOT_WORDS;
+    c.copies = team_copies(t.nwg);
+    c.copy = c.rank % c.copies;
+    c.slab = 2 * TEAM_NQ * t.nwg;
+    c.ep = c.zp = 0;
+    c.lay_out();
+
+    const bool mr = GEN && t.mean_row >= 0;
+    // the state's constants, and the state itself (every thread keeps and
+    // advances it from the same totals)
+    const Scal *st = a.st + id;
+    const bool l2 = !GEN || st->norm;
+    const int max_iter = st->max_iter, max_restarts = st->max_restarts;
+    const bool confirm = st->rep_factor > 0.0;
+    const double eps = st->eps, tol_abs = st->tol_abs, tol_rel = st->tol_rel, bd_tol = st->bd_tol;
+    double err = 0.0, err0 = 0.0, size_opt = 0.0, err_rep = 0.0, rho = 0.0, target = 0.0;
+    int iter = 0, restarts = 0, n_rep = 0;
+    bool done = false, converged = false, improved = false;
+
+    double r[T][4], rhat[T][4], p[T][4], nu[T][4], x[T][4];
+    double hh = 0.0, alpha = 0.0, omega = 1.0, mean = 0.0;
+    u64 tick = 0, ph[TEAM_PHASES] = {0, 0, 0, 0, 0};
+    const bool prof = a.phase && c.rank == 0 && wave_id() == 0;
+    auto lap = [&](int k) __attribute__((always_inline)) {
+      if (prof) {
+        const u64 now = wall_clock64();
+        ph[k] += now - tick;
+        tick = now;
+      }
+    };
+    if (prof) tick = wall_clock64();
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) x[tt][k] = a.x0[c.cell(tt) + k];  // the caller's arrays: 8-byte aligned
+      if (c.ok(tt)) st4(a.xopt, c.cell(tt), x[tt]);
+      else x[tt][0] = x[tt][1] = x[tt][2] = x[tt][3] = 0.0;
+    }
+    CELLS r[tt][k] = rhat[tt][k] = p[tt][k] = nu[tt][k] = 0.0;
+    {  // the whole team is here and its words of z are empty before any is awaited
+      c.clear();
+      c.clear();
+      double v[2] = {0.0, 0.0};
+      c.template exchange<2, false>(v, a.form_polls);
+    }
+
+    // A pass of this loop is one application of the operator and what hangs
+    // on it: the residual r = b - A x (at the start and to confirm
+    // convergence), nu = A P p with alpha, or t = A P s with omega -- one
+    // copy of the code for all three, which keeps the loop in the
+    // instruction cache -- or the mean of the returned iterate.
+    enum { RES, NU, TS, FIN };
+    int mode = RES;
+    bool replaced = false;
+    while (!c.dead) {
+      c.place();
+      double z[T][4], y[T][4];
+      double v[GEN ? 4 : 2] = {};
+      if (mode != FIN) {
+        if (mode == NU) {
+          CELLS z[tt][k] = p[tt][k];
+        } else if (mode == TS) {
+          CELLS z[tt][k] = r[tt][k];
+        } else {
+          CELLS z[tt][k] = x[tt][k];
+        }
+        if (mode != RES) {
+          c.prec(F, z);
+          lap(1);
+        }
+        c.place();
+        c.spmv(z, y, TEAM_POLLS);
+        if constexpr (GEN)
+          if (mr) CELLS {  // the mean row: sum h^2 z, and the other factor's value there
+            v[2] += s.h2[c.lb(tt)] * z[tt][k];
+            if (c.ok(tt) && c.cell(tt) + k == t.mean_row) {
+              y[tt][k] = 0.0;
+              v[3] = mode == NU ? rhat[tt][k] : r[tt][k];
+            }
+          }
+        if (mode == NU) {
+          CELLS v[0] += y[tt][k] * rhat[tt][k];
+        } else {
+          CELLS {
+            v[0] += y[tt][k] * r[tt][k];
+            v[1] += y[tt][k] * y[tt][k];
+          }
+        }
+        lap(0);
+      } else {
+        CELLS {
+          const double w2 = s.h2[c.lb(tt)];
+          v[0] += x[tt][k] * w2;
+          v[1] += w2;
+        }
+      }
+      c.place();
+      c.template exchange<GEN ? 4 : 2, false>(v, TEAM_POLLS);
+      if (c.dead) break;
+      if (mode == FIN) {  // the h^2-weighted mean removed (ExpAMRSolver.cpp:383-415)
+        mean = tot(0) / tot(1);
+#pragma unroll
+        for (int tt = 0; tt < T; tt++)
+          if (c.ok(tt))
+#pragma unroll
+            for (int k = 0; k < 4; k++) a.out[c.cell(tt) + k] = x[tt][k] - mean;
+        break;
+      }
+      if (mr) CELLS if (c.ok(tt) && c.cell(tt) + k == t.mean_row) y[tt][k] = tot(2);
+      double coef;
+      if (mode == NU) {
+        alpha = coef = uni(rho / (tot(0) + (mr ? tot(3) * tot(2) : 0.0) + eps));
+      } else {
+        const double ts = tot(0) + (mr ? tot(2) * tot(3) : 0.0);
+        const double tq = tot(1) + (mr ? tot(2) * tot(2) : 0.0);
+        omega = coef = uni(ts / (tq + eps));
+      }
+      if (mode != RES) {  // s = r - alpha nu, or r = s - omega t; x follows
+        CELLS {
+          x[tt][k] = x[tt][k] + coef * z[tt][k];
+          r[tt][k] = r[tt][k] - coef * y[tt][k];
+        }
+        if (mode == NU) {
+          c.clear();
+          CELLS nu[tt][k] = y[tt][k];
+          mode = TS;
+          lap(3);
+          continue;
+        }
+      } else {
+        omega = 1.0;
+#pragma unroll
+        for (int tt = 0; tt < T; tt++) {
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            const double bb = a.b[c.cell(tt) + k];
+            const bool row0 = mr && c.cell(tt) + k == t.mean_row;  // b = 0 there (ExpAMRSolver.cpp:340-345)
+            const double ri = c.ok(tt) ? (row0 ? 0.0 : bb) - y[tt][k] : 0.0;
+            r[tt][k] = rhat[tt][k] = ri;
+            p[tt][k] = nu[tt][k] = 0.0;
+          }
+        }
+      }
+      double f[GEN ? 3 : 2] = {};
+      CELLS {
+        const double rd = r[tt][k];
+        f[0] += rd * rd;
+        f[1] += rhat[tt][k] * rd;
+        if constexpr (GEN) f[2] = nmax(f[2], fabs(rd));
+      }
+      const double aow = alpha / (omega + eps);  // of beta, before the wait
+      lap(2);
+      c.place();
+      c.template exchange<GEN ? 3 : 2, GEN>(f, TEAM_POLLS);
+      if (c.dead) break;
+      // the state at the top of the iteration (kernels.h evaluate: the same
+      // rules, without the projection and the stall window)
+      const double rr = tot(0), rhr = tot(1);
+      bool restart = false, replace = false;
+      double beta = 0.0;
+      // the size of the residual as it is compared: |r|^2 or |r|_inf
+      const double size = l2 ? rr : tot(2);
+      auto norm_of = [l2](double v) { return l2 ? sqrt(v) : v; };
+      if (mode == RES) {
+        err = uni(norm_of(size));
+        if (replaced) {
+          n_rep++;
+        } else {
+          err0 = err;
+          // sizes above this have not converged (the test itself is exact)
+          const double most = fmax(tol_abs, tol_rel * err0) * (1.0 + 1e-9);
+          target = uni(l2 ? most * most : most);
+        }
+        size_opt = size;
+        err_rep = err;
+        hh = rho = rr;
+        improved = replaced;
+        done = err == 0.0 || iter >= max_iter;
+        if (replaced && (err <= tol_abs || err / err0 <= tol_rel)) converged = done = true;
+        if (a.start != TEAM_PLAIN) {
+          if (err != err || err > 1.79e308) {
+            done = true;
+            converged = false;
+          } else if (!replaced && (err == 0.0 || (a.start == TEAM_ACCEPTS && (err <= tol_abs || tol_rel >= 1.0)))) {
+            converged = done = true;
+          }
+        }
+        if (n_rep >= TEAM_MAX_CONFIRM) done = true;
+      } else {
+        iter++;
+        improved = false;
+        if (size < size_opt) {
+          improved = true;
+          size_opt = size;
+          if (size <= target && ((err = uni(norm_of(size))) <= tol_abs || err / err0 <= tol_rel)) {
+            if (confirm) replace = true;  // the recurrence says converged: confirm it on the residual itself
+            else converged = done = true;
+          }
+        }
+        if (iter >= max_iter) done = true;
+        beta = uni((rhr / (rho + eps)) * aow);
+        rho = rhr;
+        const bool breakdown = rhr * rhr < bd_tol * rr * hh || !(fabs(beta) < 1e30);
+        if (!done && !replace && breakdown && max_restarts > 0) {
+          restarts++;
+          if (restarts >= max_restarts) {
+            done = true;
+          } else {
+            restart = true;
+            hh = rho = rr;  // rhat = r
+          }
+        }
+        replace = replace && !done;
+      }
+      c.clear();
+      lap(mode == RES ? 4 : 3);
+      replaced = replace;
+      if (improved) {
+        if (!done && !replace)  // the iterate is the best so far
+#pragma unroll
+          for (int tt = 0; tt < T; tt++)
+            if (c.ok(tt)) st4(a.xopt, c.cell(tt), x[tt]);
+      } else if (done || replace) {  // go on with the best one
+#pragma unroll
+        for (int tt = 0; tt < T; tt++)
+          if (c.ok(tt)) ld4(a.xopt, c.cell(tt), x[tt]);
+      }
+      if (done || replace) {
+        mode = done ? FIN : RES;
+        continue;
+      }
+      if (restart) {
+        CELLS rhat[tt][k] = p[tt][k] = r[tt][k];
+      } else {
+        CELLS p[tt][k] = r[tt][k] + beta * (p[tt][k] - omega * nu[tt][k]);
+      }
+      mode = NU;
+    }
+    if (c.dead) break;
+    lap(4);
+    if (c.rank == 0 && tid == 0) {
+      Scal *o = a.st + id;
+      o->iter = iter;
+      o->restarts = restarts;
+      o->n_rep = n_rep;
+      o->converged = converged;
+      o->improved = improved;
+      o->done = o->idle = 1;
+      o->err0 = err0;
+      o->err = o->err_opt = l2 ? sqrt(size_opt) : size_opt;
+      o->err_rep = err_rep;
+      o->mean = mean;
+      if (prof)
+        for (int k = 0; k < TEAM_PHASES; k++) a.phase[(size_t)id * TEAM_PHASES + k] = ph[k];
+    }
+    __syncthreads();  // the shared state is rewritten by the next task
+  }
+}
+
+template <bool GEN>
+const void *shape_kernel(int shape) {
+  return shape == TEAM_16   ? reinterpret_cast<const void *>(&k_team<256, 1, GEN>)
+         : shape == TEAM_32 ? reinterpret_cast<const void *>(&k_team<512, 1, GEN>)
+                            : reinterpret_cast<const void *>(&k_team<512, 2, GEN>);
+}
+const void *shape_kernel(int shape, bool gen) { return gen ? shape_kernel<true>(shape) : shape_kernel<false>(shape); }
+int shape_threads(int shape) { return shape == TEAM_16 ? 256 : 512; }
+size_t shape_lds(int shape) {
+  return shape == TEAM_16 ? sizeof(Shared<256, 1>) : shape == TEAM_32 ? sizeof(Shared<512, 1>) : sizeof(Shared<512, 2>);
+}
+
+}  // namespace
+
+int team_resident(int shape) {
+  static std::atomic<int> known[64][TEAM_SHAPES];  // per device: looked up once (0: not yet)
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (const int n = known[dev][shape].load()) return n;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  int least = 1 << 30;
+  for (const bool gen : {false, true}) {
+    const void *k = shape_kernel(shape, gen);
+    int per = 0;
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape_lds(shape)) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, shape_threads(shape), shape_lds(shape)) != hipSuccess)
+      return 0;
+    least = per < least ? per : least;
+  }
+  known[dev][shape] = cus * least;
+  return cus * least;
+}
+
+hipError_t team_launch(const TeamArgs &a, int shape, size_t n_words, int grid, hipStream_t stream) {
+  TeamArgs args = a;
+  hipError_t e = hipMemsetAsync(a.slots, 0, n_words * sizeof(u64), stream);
+  if (e == hipSuccess) e = hipMemsetAsync(a.ctl, 0, 2 * sizeof(int), stream);
+  if (e != hipSuccess) return e;
+  void *params[] = {&args};
+  return hipLaunchCooperativeKernel(shape_kernel(shape, a.gen), dim3(grid), dim3(shape_threads(shape)),
+                                    params, (unsigned)shape_lds(shape), stream);
+}
+
+}  // namespace cup2d

@@ -62,12 +62,14 @@ typedef struct {
   int norm;               /* stopping norm: CUP2D_PS_NORM_INF as BiCGSTAB.cu:572-587, or
                              CUP2D_PS_NORM_L2 as AMRSolver.cpp:466-471 */
   int max_iter;           /* iteration cap (reference GPU: 1000, BiCGSTAB.cu:468) */
-  int chunk;              /* iterations per captured graph launch; 0 = automatic */
+  int chunk;              /* iterations per captured graph launch; 0 = automatic (meshes that are
+                             not solved on chip, as use_graph) */
   int use_graph;          /* 1 = replay iteration chunks as a hipGraph */
   int profile;            /* 1 = per-phase device timers (the reference's DeviceProfiler,
-                             DeviceProfiler.cuh:26-107, used at BiCGSTAB.cu:191-619): kernels are
-                             launched one by one between HIP events and the phase times are
-                             returned in cup2d_ps_stats.ms_phase; 0 = off (graph replay) */
+                             DeviceProfiler.cuh:26-107, used at BiCGSTAB.cu:191-619), returned in
+                             cup2d_ps_stats.ms_phase: read inside the kernel of an on-chip solve,
+                             elsewhere kernels are launched one by one between HIP events;
+                             0 = off */
   int item_blocks;        /* batch handles: blocks per work item, 1..256; 0 = the value tuned in
                              this process for the batch's shape, else 8 */
   int schedule;           /* 0 = fused kernels (default); 1 = one operation per launch with a
@@ -157,7 +159,7 @@ int cup2d_ps_solve_device(cup2d_ps *h, const double *d_b, double *d_x, double to
  * graph instantiation in the call.  No counterpart in the reference; it is
  * for callers that cannot allocate (serving loops, harnesses that forbid
  * allocation).  The work vectors, partial sums and solver state live in a
- * fixed per-device array of the library (about 9.5 MB, held until the
+ * fixed per-device array of the library (about 10 MB, held until the
  * process ends) instead of the handle's buffers, so: FP64 handles with the
  * fused schedule only, meshes of at most CUP2D_PS_NOALLOC_MAX_N unknowns
  * (CUP2D_PS_EINVAL beyond), d_b must not alias d_x, and calls that overlap
