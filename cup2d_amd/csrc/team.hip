@@ -134,10 +134,10 @@ struct Shared {
   unsigned ent[ENT][ROWS];          // entries of the explicit rows: LDS index, coefficient << 16
   int erow[face_rows(BPW)];         // ELL slot of each explicit row
   int eoff[BPW + 1];                // first explicit row of each block
-  unsigned char ewid[face_rows(BPW)];  // entries, | 128 when they are read from memory
+  unsigned char ewid[face_rows(BPW)];  // entries, | 64 with ghosts among them, | 192 read from memory
   int2 item[ITEMS];                 // what other workgroups read, 8 cells each: {first LDS index | stride 8 (bit
                                     // 16), place in the halo buffer}
-  int ng, ni, ticket, bad;
+  int ng, ni, nf, ticket, bad;      // ghosts, items, explicit rows with ghosts
 };
 
 // The running workgroup: what its functions share.
@@ -343,45 +343,61 @@ struct Ctx {
     __syncthreads();  // the inputs are overwritten by z
   }
 
+  // ye = A z of the explicit rows whose kind (0: all entries in LDS from the
+  // start, 64: some are ghosts, or the row is read from memory) is this: a
+  // thread per row.
+  __device__ __forceinline__ void explicit_rows(int kind, const double *zb, int limit) {
+    const int ne = uni(s.eoff[nb]);
+    for (int k = tid; k < ne; k += WGS) {
+      const int how = s.ewid[k], width = how & 63;
+      if ((how & 64) != kind) continue;
+      double sum = 0.0;
+      if (how < 128) {
+        for (int w0 = 0; w0 < width; w0 += ENT / 2) {
+          unsigned en[ENT / 2];
+#pragma unroll
+          for (int i = 0; i < ENT / 2; i++) en[i] = s.ent[w0 + i][k];
+#pragma unroll
+          for (int i = 0; i < ENT / 2; i++) sum += s.tab[en[i] >> 16] * s.z[en[i] & 0xffffu];
+        }
+      } else {
+        const int e = s.erow[k];
+        for (int i = 0; i < width; i++) {
+          const long at = (long)i * a.A.n_exc + e;
+          const int col = a.A.ecol[at], l = (col >> 6) - b0;
+          const double v =
+              (l >= 0 && l < nb) ? s.z[l * ZS + (col & 63)] : remote(zb + place_of(a.A.erow[e] >> 6, col), EMPTY, limit);
+          sum += a.A.etab[a.A.ecode[at]] * v;
+        }
+      }
+      s.ye[k] = sum;
+    }
+  }
+
   // y = A z of the thread's cells (0 past the last block, where z is 0)
   __device__ __forceinline__ void spmv(const double (&z)[T][4], double (&y)[T][4], int limit) {
     const double *zb = halo();
     to_lds(z);
     __syncthreads();
     publish<false>(halo());
+    // The ghosts are asked for, the explicit rows without any are computed
+    // while they travel, and the others follow.
     const int ng = uni(s.ng);
-    for (int g = tid; g < ng; g += 2 * WGS) {  // two at a time: one round trip for most teams
-      const int g1 = g + WGS < ng ? g + WGS : g;
-      const double *p0 = zb + s.ghost[g], *p1 = zb + s.ghost[g1];
-      const u64 v0 = ld_agent(reinterpret_cast<const u64 *>(p0)), v1 = ld_agent(reinterpret_cast<const u64 *>(p1));
-      s.z[S::GHOST0 + g] = remote(p0, v0, limit);
-      s.z[S::GHOST0 + g1] = remote(p1, v1, limit);
+    const int g0 = min(tid, ng - 1), g1 = min(tid + WGS, ng - 1);
+    u64 v0 = 0, v1 = 0;
+    if (ng > 0) {
+      v0 = ld_agent(reinterpret_cast<const u64 *>(zb + s.ghost[g0]));
+      v1 = ld_agent(reinterpret_cast<const u64 *>(zb + s.ghost[g1]));
+    }
+    explicit_rows(0, zb, limit);
+    if (ng > 0) {
+      s.z[S::GHOST0 + g0] = remote(zb + s.ghost[g0], v0, limit);
+      s.z[S::GHOST0 + g1] = remote(zb + s.ghost[g1], v1, limit);
+      for (int g = tid + 2 * WGS; g < ng; g += WGS) s.z[S::GHOST0 + g] = remote(zb + s.ghost[g], EMPTY, limit);
     }
     __syncthreads();
-    const int ne = uni(s.eoff[nb]);
-    if (ne > 0) {
-      for (int k = tid; k < ne; k += WGS) {  // a thread per explicit row
-        const int width = s.ewid[k];
-        double sum = 0.0;
-        if (width < 128) {
-          for (int w0 = 0; w0 < width; w0 += ENT / 2) {
-            unsigned en[ENT / 2];
-#pragma unroll
-            for (int i = 0; i < ENT / 2; i++) en[i] = s.ent[w0 + i][k];
-#pragma unroll
-            for (int i = 0; i < ENT / 2; i++) sum += s.tab[en[i] >> 16] * s.z[en[i] & 0xffffu];
-          }
-        } else {
-          const int e = s.erow[k];
-          for (int i = 0; i < width - 128; i++) {
-            const long at = (long)i * a.A.n_exc + e;
-            const int col = a.A.ecol[at], l = (col >> 6) - b0;
-            const double v = (l >= 0 && l < nb) ? s.z[l * ZS + (col & 63)] : remote(zb + place_of(a.A.erow[e] >> 6, col), EMPTY, limit);
-            sum += a.A.etab[a.A.ecode[at]] * v;
-          }
-        }
-        s.ye[k] = sum;
-      }
+    if (uni(s.nf) > 0) {
+      explicit_rows(64, zb, limit);
       __syncthreads();
     }
     const int row = 2 * w + (q >> 1), ix0 = 4 * (q & 1);
@@ -428,7 +444,7 @@ struct Ctx {
 
   // Headers, ghosts and explicit rows of the workgroup's blocks.
   __device__ __forceinline__ void lay_out() {
-    if (tid == 0) s.ng = s.ni = 0;
+    if (tid == 0) s.ng = s.ni = s.nf = 0;
     __syncthreads();
     // LDS index of 8 cells of another workgroup, from `first` of the halo buffer on
     auto ghosts = [&](int first) -> int {
@@ -489,7 +505,7 @@ struct Ctx {
       const int k = s.eoff[l] + __popcll(s.mask[l] & ((1ull << (row & 63)) - 1));
       s.erow[k] = e;
       int width = 0;
-      bool fits = k < S::ROWS && a.A.ell_w <= ENT;
+      bool fits = k < S::ROWS && a.A.ell_w <= ENT, far = false;
 #pragma unroll 1
       for (int i = 0; i < a.A.ell_w; i++) {
         const long at = (long)i * a.A.n_exc + e;
@@ -507,13 +523,15 @@ struct Ctx {
           idx = lc * ZS + (col & 63);
         } else {
           const int g = atomicAdd(&s.ng, 1);
+          far = true;
           fits = g < S::GHOSTS;
           if (fits) s.ghost[g] = place_of(row >> 6, col);
           idx = S::GHOST0 + g;
         }
         if (fits) s.ent[i][k] = idx | code << 16;
       }
-      s.ewid[k] = (unsigned char)(fits ? width : 128 + width);
+      if (far || !fits) atomicAdd(&s.nf, 1);
+      s.ewid[k] = (unsigned char)(fits ? (far ? 64 : 0) + width : 192 + width);
     }
     __syncthreads();
     if (tid == 0 && s.ng > S::GHOSTS) s.ng = S::GHOSTS;
