@@ -3,8 +3,18 @@
 // Each instance is the solve of ExpAMRSolver::solve (ExpAMRSolver.cpp:354-416)
 // on its own mesh: BiCGSTAB (BiCGSTAB.cu:412-620) with the 64x64 block
 // preconditioner and h^2-weighted mean removal.  The instances' blocks are
-// concatenated into one block-diagonal operator and every iteration advances
-// all unfinished instances at once:
+// concatenated into one block-diagonal operator.
+//
+// Where every instance has at most 16,384 blocks, each is solved on chip by a
+// team of workgroups (team.hip), all in one launch: an iteration touches memory
+// for its halo and its sums only, and an instance ends when it converges, its
+// workgroups taking the next.  64 instances of 512-8,192 blocks (13.9 million
+// cells) to 1e-12: 424 ms, by the item kernels 915 ms; 9 small ones in mixed
+// precision 23.2 ms against 53.4 ms.  What bounds it: the workgroups' own work
+// (25 us an iteration on 64 blocks; 3,389 workgroups' worth of instances on 256).
+//
+// A batch with a larger instance takes the item kernels, which advance all
+// unfinished instances at once:
 //
 //  * work units: "items" (a run of up to `ib` blocks of one instance) for the
 //    SpMV and vector kernels, a workgroup per item; "tiles" (16 blocks of one
@@ -20,9 +30,10 @@
 //  * the item size `ib` is picked by a timing autotuner and cached per
 //    batch shape.
 //
-// Precisions: FP64, or FP32-stored Krylov vectors with FP64 arithmetic and
-// the BF16 MFMA preconditioner inside per-instance FP64 iterative refinement
-// (the scheme of the single-solve mixed path).
+// Precisions of the item kernels: FP64, or FP32-stored Krylov vectors with
+// FP64 arithmetic and the BF16 MFMA preconditioner inside per-instance FP64
+// iterative refinement (the scheme of the single-solve mixed path).  On chip
+// both are FP64, the mixed handle with its own stopping rule.
 
 #include <hip/hip_runtime.h>
 
@@ -42,6 +53,7 @@
 #include "assemble_device.h"
 #include "assembly.h"
 #include "kernels.h"
+#include "team.h"
 
 using namespace cup2d;
 
@@ -1162,6 +1174,18 @@ struct cup2d_psb {
   void *v_r = nullptr, *v_rhat = nullptr, *v_p = nullptr, *v_nu = nullptr, *v_z1 = nullptr,
        *v_z2 = nullptr, *v_t = nullptr;  // Krylov vectors, FP64 or FP32
   Scal *d_st = nullptr;
+  // the on-chip solve (team.hip): its launch shape (-1: a mesh of the batch is
+  // too large for it), the instances' teams in launch order, device words
+  int team_shape = -1;
+  bool team_failed = false;
+  int n_codes = 0;                  // entries of etab
+  std::vector<TeamTask> team;
+  std::vector<int> team_inst;       // instance of each task
+  size_t team_words = 0;            // exchange words
+  int team_grid = 0, n_tickets = 0;
+  TeamTask *d_task = nullptr;
+  unsigned char *d_team = nullptr;  // control words, phase times [K], exchange words
+  double *d_halo = nullptr;         // [3 n]
   int *d_all_done = nullptr;
   int *h_all_done = nullptr;        // pinned
   std::vector<Scal> h_st;
@@ -1591,7 +1615,76 @@ int run_pass(cup2d_psb *h, const double *d_b, int max_iter, int max_chunks) {
   return CUP2D_PS_OK;
 }
 
-// One BiCGSTAB run per instance from r0 = b - A x0 (FP64).  Mixed precision:
+// Device words of the on-chip solve: control words, then [K] phase times, then
+// the exchange words.
+constexpr size_t TEAM_PHASE_AT = 64;
+size_t team_slots_at(int K) {
+  return (TEAM_PHASE_AT + (size_t)K * TEAM_PHASES * sizeof(unsigned long long) + 127) / 128 * 128;
+}
+bool team_on(const cup2d_psb *h) { return h->team_shape >= 0 && !h->team_failed; }
+
+// Every instance solved on chip (team.hip), a team of workgroups each, in one
+// launch: in start_order, the next instance as workgroups come free.
+// FP64 throughout; a mixed handle keeps its stopping rule (convergence is
+// accepted on the recomputed FP64 residual).  h_st holds the marker states
+// (instance order) and receives the final ones; the mean-free solutions go to
+// h->d_x.  `done` is false when the launch could not run to its end.
+int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done) {
+  done = false;
+  const int K = h->K;
+  std::vector<Scal> st(K);
+  for (int i = 0; i < K; i++) {
+    Scal s = h->h_st[h->team_inst[i]];
+    s.project = s.stall = 0;
+    s.rep_factor = h->mixed ? 1e-300 : 0.0;  // a replacement only where convergence is claimed
+    st[i] = s;
+  }
+  TeamArgs a{};
+  a.A = bview(h).A;
+  a.fid = h->d_fid;
+  a.pf = h->d_P;
+  a.b = d_b;
+  a.x0 = d_x0;
+  a.out = h->d_x;
+  a.halo = h->d_halo;
+  a.xopt = h->d_xopt;
+  a.n_codes = h->n_codes;
+  a.task = h->d_task;
+  a.n_tasks = K;
+  a.n_tickets = h->n_tickets;
+  a.start = h->mixed ? TEAM_ACCEPTS : TEAM_CHECKED;
+  a.gen = h->cfg.mean_constraint != 0 || h->cfg.norm == CUP2D_PS_NORM_INF;
+  a.form_polls = TEAM_POLLS << 5;  // a team forms when earlier tasks end
+  a.st = h->d_st;
+  a.ctl = reinterpret_cast<int *>(h->d_team);
+  a.phase = h->cfg.profile ? reinterpret_cast<unsigned long long *>(h->d_team + TEAM_PHASE_AT) : nullptr;
+  a.slots = reinterpret_cast<unsigned long long *>(h->d_team + team_slots_at(K));
+  BCHK(h, hipMemcpyAsync(h->d_st, st.data(), K * sizeof(Scal), hipMemcpyHostToDevice, h->stream));
+  BCHK(h, team_launch(a, h->team_shape, h->team_words, h->team_grid, h->stream));
+  std::vector<unsigned char> words(team_slots_at(K));
+  BCHK(h, hipMemcpyAsync(st.data(), h->d_st, K * sizeof(Scal), hipMemcpyDeviceToHost, h->stream));
+  BCHK(h, hipMemcpyAsync(words.data(), h->d_team, words.size(), hipMemcpyDeviceToHost, h->stream));
+  BCHK(h, hipStreamSynchronize(h->stream));
+  if (reinterpret_cast<const int *>(words.data())[1]) return CUP2D_PS_OK;
+  done = true;
+  for (int i = 0; i < K; i++) h->h_st[h->team_inst[i]] = st[i];
+  if (h->cfg.profile) {
+    // the launch's time, split as its teams spent theirs
+    bptick(h, -1);
+    BCHK(h, hipEventRecord(h->ev1, h->stream));
+    BCHK(h, hipEventSynchronize(h->ev1));
+    float ms = 0;
+    BCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
+    const auto *ph = reinterpret_cast<const unsigned long long *>(words.data() + TEAM_PHASE_AT);
+    double all = 0.0;
+    for (int i = 0; i < K * TEAM_PHASES; i++) all += (double)ph[i];
+    for (int i = 0; i < K * TEAM_PHASES && all > 0; i++) h->pms[i % TEAM_PHASES] += ms * (double)ph[i] / all;
+  }
+  return CUP2D_PS_OK;
+}
+
+// One BiCGSTAB run per instance from r0 = b - A x0 (FP64): on chip, or, where
+// a mesh is too large for that, by the item kernels.  There, mixed precision:
 // FP32-stored Krylov vectors with FP64 residual replacement and restart
 // (launch_replacement_b at the start of every chunk), so the stopping test is
 // met on an FP64 residual.
@@ -1604,14 +1697,25 @@ int solve_b_body(cup2d_psb *h, const double *d_b, const double *d_x0, double *d_
   h->pused = 0;
   bptick(h, -1);
   BCHK(h, hipEventRecord(h->ev0, h->stream));
-  BCHK(h, hipMemcpyAsync(h->d_x, d_x0, h->n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
-  if (d_b != h->d_b)  // the replacement step of the captured graph reads the handle's copy
-    BCHK(h, hipMemcpyAsync(h->d_b, d_b, h->n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
   std::vector<int> iters(K, 0), restarts(K, 0), reps(K, 0), conv(K, 0);
   std::vector<double> err0(K, -1.0), errf(K, 0.0);
   for (int k = 0; k < K; k++) h->h_st[k] = marker_b(h, k, tol_abs, tol_rel, max_restarts, max_iter);
-  int rc = h->mixed ? run_pass<float>(h, h->d_b, max_iter, -1) : run_pass<double>(h, h->d_b, max_iter, -1);
-  if (rc) return rc;
+  int rc = CUP2D_PS_OK;
+  bool done = false;
+  if (team_on(h)) {
+    if ((rc = solve_b_team(h, d_b, d_x0, done))) return rc;
+    h->team_failed = !done;
+  }
+  const bool on_chip = done;
+  if (on_chip) {
+    BCHK(h, hipMemcpyAsync(d_out, h->d_x, h->n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+  } else {
+    BCHK(h, hipMemcpyAsync(h->d_x, d_x0, h->n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+    if (d_b != h->d_b)  // the replacement step of the captured graph reads the handle's copy
+      BCHK(h, hipMemcpyAsync(h->d_b, d_b, h->n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+    rc = h->mixed ? run_pass<float>(h, h->d_b, max_iter, -1) : run_pass<double>(h, h->d_b, max_iter, -1);
+    if (rc) return rc;
+  }
   for (int k = 0; k < K; k++) {
     const Scal &s = h->h_st[k];
     iters[k] = std::max(s.iter, 0);
@@ -1625,9 +1729,11 @@ int solve_b_body(cup2d_psb *h, const double *d_b, const double *d_x0, double *d_
   }
   const BView V = bview(h);
   const int Gi = grid_items(h);
-  kb_fmean<<<Gi, WG, 0, h->stream>>>(V, h->d_x, h->d_pm);
-  kb_mean<<<K, WG, 0, h->stream>>>(V, h->d_st, h->d_pm);
-  kb_fwrite<<<Gi, WG, 0, h->stream>>>(V, h->d_x, d_out, h->d_st);
+  if (!on_chip) {
+    kb_fmean<<<Gi, WG, 0, h->stream>>>(V, h->d_x, h->d_pm);
+    kb_mean<<<K, WG, 0, h->stream>>>(V, h->d_st, h->d_pm);
+    kb_fwrite<<<Gi, WG, 0, h->stream>>>(V, h->d_x, d_out, h->d_st);
+  }
   BCHK(h, hipGetLastError());
   BCHK(h, hipEventRecord(h->ev1, h->stream));
   // the returned solutions' true residuals, recomputed in FP64 (x_opt is
@@ -1872,6 +1978,7 @@ static int build_host(cup2d_psb *h, int n_inst, const cup2d_mesh_desc *meshes) {
   }
   h->ell_w = W;
   h->elen = std::move(ell.len);
+  h->n_codes = (int)ell.values.size();
   ops.clear();
   auto &pool = h->allocs;
   int rc;
@@ -1919,6 +2026,7 @@ static int build_device(cup2d_psb *h, int n_inst, const cup2d_mesh_desc *meshes)
   h->ell_w = D.ell_w;
   h->eoff = D.eoff;
   h->elen = std::move(D.elen);
+  h->n_codes = D.n_codes;
   h->h_mean_row = D.mean_rows;
   h->d_nbr = D.nbr;
   h->d_fid = D.fid;
@@ -1928,6 +2036,100 @@ static int build_device(cup2d_psb *h, int n_inst, const cup2d_mesh_desc *meshes)
   h->d_ecol = D.ecol;
   h->d_ecode = D.ecode;
   h->d_etab = D.etab;
+  return CUP2D_PS_OK;
+}
+
+// The order in which instances of n[k] workgroups start on `grid` of them:
+// whenever workgroups come free, the longest instance that fits.  Durations are
+// taken to grow as blocks^(3/4) (iterations grow with the size, an iteration's
+// time hardly does); the tickets then go in this order.  On the 64-instance
+// batch this leaves the workgroups idle for 3 % of the time against 14 % with
+// the largest instances first.
+static std::vector<int> start_order(const std::vector<int> &n, int grid) {
+  const int K = (int)n.size();
+  std::vector<int> left(K), order;
+  for (int k = 0; k < K; k++) left[k] = k;
+  std::stable_sort(left.begin(), left.end(), [&](int a, int b) { return n[a] > n[b]; });
+  std::multimap<double, int> running;  // end of an instance, its workgroups
+  double t = 0.0;
+  int free = grid;
+  while (!left.empty()) {
+    size_t kept = 0;
+    for (size_t i = 0; i < left.size(); i++) {
+      const int k = left[i];
+      if (n[k] <= free) {
+        free -= n[k];
+        running.emplace(t + std::pow((double)n[k], 0.75), n[k]);
+        order.push_back(k);
+      } else {
+        left[kept++] = k;
+      }
+      if (free == 0) {
+        for (i++; i < left.size(); i++) left[kept++] = left[i];
+      }
+    }
+    left.resize(kept);
+    if (running.empty()) break;  // an instance wider than the grid: the caller has ruled it out
+    t = running.begin()->first;
+    free += running.begin()->second;
+    running.erase(running.begin());
+  }
+  return order;
+}
+
+// The on-chip solve's teams: the fewest blocks per workgroup with which all
+// instances run at once, because a team's iteration is the shorter the fewer
+// blocks its workgroups hold (16: 11.7 us, 32: 15, 64: 23); else 64 blocks per
+// workgroup in start_order, which keep the most instances running (64 blocks in
+// 23-25 us against 32 in 18).
+static int plan_teams(cup2d_psb *h) {
+  h->team_shape = -1;
+  const int K = h->K;
+  long long most = 0;
+  for (int k = 0; k < K; k++) most = std::max(most, h->boff[k + 1] - h->boff[k]);
+  if (most > TEAM_MAX_BLOCKS) return CUP2D_PS_OK;
+  for (int s = 0; s < TEAM_SHAPES && h->team_shape < 0; s++) {
+    const int grid = std::min(TEAM_MAX_WG, team_resident(s));
+    std::vector<int> wide(K);
+    int tickets = 0, widest = 0;
+    for (int k = 0; k < K; k++) {
+      TeamTask t{};
+      team_split((int)(h->boff[k + 1] - h->boff[k]), team_blocks(s), t);
+      wide[k] = t.nwg;
+      widest = std::max(widest, t.nwg);
+      tickets = std::min(tickets + t.nwg, 1 << 30);
+    }
+    if (widest > grid || (tickets > grid && s + 1 < TEAM_SHAPES)) continue;
+    const std::vector<int> order = start_order(wide, grid);
+    std::vector<TeamTask> team;
+    size_t words = 0;
+    tickets = 0;
+    for (int k : order) {
+      TeamTask t{};
+      team_split((int)(h->boff[k + 1] - h->boff[k]), team_blocks(s), t);
+      t.b0 = (int)h->boff[k];
+      t.ticket0 = tickets;
+      t.slot0 = (int)(words / TEAM_SLOT_WORDS);
+      t.e0 = (int)h->eoff[k];
+      t.e1 = (int)h->eoff[k + 1];
+      t.mean_row = (int)h->h_mean_row[k];
+      tickets += t.nwg;
+      words += team_words(t.nwg);
+      team.push_back(t);
+    }
+    h->team_shape = s;
+    h->team = std::move(team);
+    h->team_inst = order;
+    h->team_words = words;
+    h->n_tickets = tickets;
+    h->team_grid = std::min(grid, tickets);
+  }
+  if (h->team_shape < 0) return CUP2D_PS_OK;
+  int rc;
+  if ((rc = bupload(h, h->allocs, &h->d_task, h->team)) ||
+      (rc = balloc(h, h->allocs, &h->d_team, team_slots_at(K) + h->team_words * sizeof(unsigned long long))) ||
+      (rc = balloc(h, h->allocs, &h->d_halo, 3 * (size_t)h->n)))
+    return rc;
   return CUP2D_PS_OK;
 }
 
@@ -1957,6 +2159,7 @@ static int finish_meshes(cup2d_psb *h, int n_inst) {
       (rc = balloc(h, pool, &h->d_rt, 4 * (size_t)n_inst)))
     return rc;
   h->h_st.assign(n_inst, Scal{});
+  if ((rc = plan_teams(h))) return rc;
   int ib = h->cfg.item_blocks;
   {
     std::lock_guard<std::mutex> lock(g_tuned_mu);
