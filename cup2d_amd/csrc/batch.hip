@@ -9,9 +9,10 @@
 // team of workgroups (team.hip), all in one launch: an iteration touches memory
 // for its halo and its sums only, and an instance ends when it converges, its
 // workgroups taking the next.  64 instances of 512-8,192 blocks (13.9 million
-// cells) to 1e-12: 424 ms, by the item kernels 915 ms; 9 small ones in mixed
-// precision 23.2 ms against 53.4 ms.  What bounds it: the workgroups' own work
-// (25 us an iteration on 64 blocks; 3,389 workgroups' worth of instances on 256).
+// cells) to 1e-12: 361 ms, by the item kernels 915 ms; 9 small ones in mixed
+// precision 22 ms against 53.4 ms.  What bounds it: the workgroups' own work and
+// the waits of a team (18 us an iteration on 64 blocks; 3,389 workgroups' worth
+// of instances on 256).
 //
 // A batch with a larger instance takes the item kernels, which advance all
 // unfinished instances at once:
@@ -1653,7 +1654,8 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   a.n_tasks = K;
   a.n_tickets = h->n_tickets;
   a.start = h->mixed ? TEAM_ACCEPTS : TEAM_CHECKED;
-  a.gen = h->cfg.mean_constraint != 0 || h->cfg.norm == CUP2D_PS_NORM_INF;
+  a.mean_rows = h->cfg.mean_constraint != 0;
+  a.norm_max = h->cfg.norm == CUP2D_PS_NORM_INF;
   a.form_polls = TEAM_POLLS << 5;  // a team forms when earlier tasks end
   a.st = h->d_st;
   a.ctl = reinterpret_cast<int *>(h->d_team);
@@ -2079,9 +2081,9 @@ static std::vector<int> start_order(const std::vector<int> &n, int grid) {
 
 // The on-chip solve's teams: the fewest blocks per workgroup with which all
 // instances run at once, because a team's iteration is the shorter the fewer
-// blocks its workgroups hold (16: 11.7 us, 32: 15, 64: 23); else 64 blocks per
-// workgroup in start_order, which keep the most instances running (64 blocks in
-// 23-25 us against 32 in 18).
+// blocks its workgroups hold (16: 8-10 us, 32: 11, 48: 13, 64: 14); else 64
+// blocks per workgroup in start_order, which keep the most instances running
+// (the 64-instance batch in 361 ms, with 48 in 412, with 32 in 515).
 static int plan_teams(cup2d_psb *h) {
   h->team_shape = -1;
   const int K = h->K;

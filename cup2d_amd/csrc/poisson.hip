@@ -1277,7 +1277,8 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   a.n_tasks = 1;
   a.n_tickets = h->team.nwg;
   a.start = h->mixed ? TEAM_ACCEPTS : TEAM_PLAIN;
-  a.gen = h->op.mean_row >= 0 || h->cfg.norm == CUP2D_PS_NORM_INF;
+  a.mean_rows = h->op.mean_row >= 0;
+  a.norm_max = h->cfg.norm == CUP2D_PS_NORM_INF;
   a.form_polls = TEAM_POLLS;
   a.st = h->d_s;
   a.ctl = reinterpret_cast<int *>(h->d_team);
@@ -1889,11 +1890,12 @@ static int set_mesh_body(cup2d_ps *h, const cup2d_mesh_desc *m) {
 
 // The on-chip solve's team for the mesh: the fewest blocks per workgroup
 // whose workgroups all fit on the device at once -- an iteration of a uniform
-// mesh took 14.2 us with 16 blocks per workgroup, 14.9 with 32 and 19.5 with
-// 64 on 1536 blocks, 18.4 with 32 and 21.6 with 64 on 8192 -- but 16 blocks
-// only up to 192 workgroups: on 3072 blocks 16 and 32 were alike (15.9), on
-// 4096 32 was faster (16.1 against 17.0), the larger team's sums taking longer
-// than the shorter product saves.
+// mesh took 9.9 us with 16 blocks per workgroup, 10.9 with 32, 12.7 with 48 and
+// 13.8 with 64 on 1536 blocks, 14.5 / 15.0 / 15.5 with 32 / 48 / 64 on 8190, and
+// on a graded mesh of 8348 blocks 16.4 with 48 and 17.3 with 64 -- but 16 blocks
+// only up to 192 workgroups: on 3072 blocks 16 and 32 took 11.2 and 11.6, on
+// 4096 12.5 and 12.0, the larger team's sums taking longer than the shorter
+// product saves.
 constexpr int TEAM_16_MOST = 192;
 static void plan_team(cup2d_ps *h) {
   h->team_shape = -1;

@@ -48,7 +48,7 @@ struct TeamArgs {
   TeamTask one;
   int n_tasks, n_tickets;
   int start;                            // TeamStart
-  int gen;                              // a mean row or the infinity norm among the tasks
+  int mean_rows, norm_max;              // a mean row among the tasks, the infinity norm
   int form_polls;                       // polls before the wait for a team to form fails
   Scal *st;                             // [n_tasks] marker state in, final state out
   unsigned long long *slots;            // exchange words of all teams, zero at launch
@@ -64,8 +64,8 @@ enum TeamStart {
 };
 
 // Blocks per workgroup of a launch shape.
-enum TeamShape { TEAM_16 = 0, TEAM_32 = 1, TEAM_64 = 2, TEAM_SHAPES = 3 };
-inline int team_blocks(int shape) { return shape == TEAM_16 ? 16 : shape == TEAM_32 ? 32 : 64; }
+enum TeamShape { TEAM_16 = 0, TEAM_32 = 1, TEAM_48 = 2, TEAM_64 = 3, TEAM_SHAPES = 4 };
+inline int team_blocks(int shape) { return shape == TEAM_64 ? 64 : 16 * (shape + 1); }
 
 // Polls (0.5 us and more each) before a wait inside a team fails.
 constexpr int TEAM_POLLS = 1 << 21;

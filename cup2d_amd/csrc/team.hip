@@ -7,24 +7,29 @@
 // z = P v that another workgroup's rows read (the operator's halo) and the
 // partial sums of the dot products.
 //
-// What bounds it: an iteration has five points where the workgroups wait for
-// each other (z's halo twice, (rhat, nu), omega's two sums, the update's sums),
-// each one store and one load past the L2s, which are not coherent between
-// the XCDs: 0.7-1 us for a halo, 1.0 us (8 workgroups) to 2 us (250) for sums.
-// A fence that writes an L2 back costs more than a kernel boundary; here every
-// shared word is written and read by relaxed agent-scope accesses, and a
-// waiting workgroup polls the data themselves: partial sums carry the
-// exchange's number in the upper half of each word, and a halo word holds a
-// NaN that no arithmetic returns until its value arrives.  Between the waits a
-// wave's instructions count (one or two waves per SIMD): the loop is one copy
-// of the code for both halves of an iteration (the instruction cache), its
-// branches are uniform, and everything an explicit row needs lies in LDS.
+// What bounds it: an iteration has four points where the workgroups wait for
+// each other (z's halo twice, (rhat, nu) with the size of the r before, and
+// omega's sums with those of the next rho), each one store and one load past
+// the L2s, which are not coherent between the XCDs: 0.7-1 us for a halo, 1.0 us
+// (8 workgroups) to 2-3 us (250) for sums.  A fence that writes an L2 back
+// costs more than a kernel boundary; here every shared word is written and
+// read by relaxed agent-scope accesses, and a waiting workgroup polls the data
+// themselves: partial sums carry the exchange's number in the upper half of
+// each word, and a halo word holds a NaN that no arithmetic returns until its
+// value arrives.  Between the waits a wave's instructions count (one to three
+// waves per SIMD), above all the taken branches and the chains of LDS reads:
+// the two halves of an iteration are one straight line (as one body with the
+// mode as a variable they took 10.6 us on 128 blocks, 8.0 so), everything an
+// explicit row needs lies in LDS, and the addresses of a thread's halo words
+// in registers.  What is the same in every lane is kept in scalar registers
+// (uni): in vector ones the vectors were spilled to memory (64 blocks per
+// workgroup: 20.5 us on 16,384 blocks, 17.6 without).
 //
-// Measured (us per iteration to a relative residual of 1e-10, against five
-// kernels per iteration replayed from a graph): 128 blocks 11.9 against 24.0,
-// 1448 blocks 14.5 against 27.9, 8348 blocks 23.7 against 49.9, 16,229 blocks
-// 29.2 against 64.8.  On 16k blocks the products (2 x 8192 flop per block at
-// the 72 TFLOP/s of a large FP64 matrix product) are 3.7 us of it.
+// Measured (us per iteration to a relative residual of 1e-12, against five
+// kernels per iteration replayed from a graph): 128 blocks 8.0 against 24.0,
+// 1448 blocks 11.5 against 27.9, 8348 blocks 16.4 against 49.9, 16,229 blocks
+// 20 against 64.8.  On 16k blocks the products (2 x 8192 flop per block at the
+// 72 TFLOP/s of a large FP64 matrix product) are 3.7 us of it.
 //
 // Teams form by tickets: a workgroup takes the next ticket, which names its
 // task and its rank, and when its task is solved takes another.  Tickets are
@@ -118,11 +123,12 @@ constexpr int TAB = 256;                                     // coefficients kep
 template <int WGS, int T>
 struct Shared {
   static constexpr int BPW = WGS / 256 * T * TILE, NW = WGS / 64;
+  static constexpr bool PF = BPW > 32;                        // P_inv in LDS, else in registers
   static constexpr int GHOST0 = BPW * ZS, GHOSTS = BPW * 40;  // first, most cells of other workgroups
   static constexpr int ITEMS = BPW * 12;                      // a block's 4 faces and 8 rows
-  static constexpr int ROWS = BPW == 64 ? 512 : face_rows(BPW);  // explicit rows kept in LDS
+  static constexpr int ROWS = BPW == 64 ? 512 : BPW == 48 ? 768 : face_rows(BPW);  // explicit rows kept in LDS
   double z[GHOST0 + GHOSTS];        // the workgroup's blocks (product inputs, then z), then the ghosts
-  double2 pf[T == 1 ? 1 : 4 * 8 * 64];  // P_inv's fragments, two K steps a word
+  double2 pf[PF ? 4 * 8 * 64 : 1];  // P_inv's fragments, two K steps a word
   double ye[face_rows(BPW)];        // A z of the explicit rows
   double tab[TAB];
   double red[TEAM_NQ][NW], tot[TEAM_NQ];  // a wave per quantity: TEAM_NQ <= NW
@@ -137,6 +143,7 @@ struct Shared {
   unsigned char ewid[face_rows(BPW)];  // entries, | 64 with ghosts among them, | 192 read from memory
   int2 item[ITEMS];                 // what other workgroups read, 8 cells each: {first LDS index | stride 8 (bit
                                     // 16), place in the halo buffer}
+  u64 tick, phase[TEAM_PHASES];     // of the profile: not in registers, which the loop needs
   int ng, ni, nf, ticket, bad;      // ghosts, items, explicit rows with ghosts
 };
 
@@ -152,6 +159,8 @@ struct Ctx {
   u64 *slots;
   int copies, copy, slab;           // copies of the exchange words, the one read here, words of a copy
   unsigned ep, zp;                  // number of the exchange, parity of z's buffer
+  int ni8, ng, nf;                  // words that others read, ghosts, explicit rows with ghosts
+  int iz, io, ig;                   // the thread's first such word (LDS index, place), its first ghost's place
   bool dead;
 
   __device__ __forceinline__ Ctx(const TeamArgs &aa, S &ss) : a(aa), s(ss), dead(false) { place(); }
@@ -201,14 +210,20 @@ struct Ctx {
   // emptied there.
   template <bool EMPTIES>
   __device__ __forceinline__ void publish(double *buf) {
-    const int n = 8 * uni(s.ni);
-    for (int i = tid; i < n; i += WGS) {
-      const int2 it = s.item[i >> 3];
-      const int c = i & 7;
-      u64 v = EMPTY;
-      if (!EMPTIES) v = (u64)__double_as_longlong(s.z[(it.x & 0xffff) + (it.x >> 16 ? 8 * c : c)]);
-      st_agent(reinterpret_cast<u64 *>(buf + 8 * (long)it.y + c), v);
+    if (tid < ni8)
+      st_agent(reinterpret_cast<u64 *>(buf + io), EMPTIES ? EMPTY : (u64)__double_as_longlong(s.z[iz]));
+#pragma unroll 1
+    for (int i = tid + WGS; i < ni8; i += WGS) {
+      int at, to;
+      word(i, at, to);
+      st_agent(reinterpret_cast<u64 *>(buf + to), EMPTIES ? EMPTY : (u64)__double_as_longlong(s.z[at]));
     }
+  }
+  // word i of those that others read: its LDS index and its place in the halo buffer
+  __device__ __forceinline__ void word(int i, int &at, int &to) const {
+    const int2 it = s.item[i >> 3];
+    at = (it.x & 0xffff) + (it.x >> 16 ? 8 * (i & 7) : i & 7);
+    to = 8 * it.y + (i & 7);
   }
 
   // After the pass's last exchange everyone has read its z: the words are
@@ -227,7 +242,8 @@ struct Ctx {
   __device__ __forceinline__ void exchange(double (&v)[NQ], int limit) {
     const int wv = uni(tid >> 6);
 #pragma unroll
-    for (int k = 0; k < NQ; k++) v[k] = MAXLAST && k == NQ - 1 ? dpp_total<true>(v[k]) : dpp_total<false>(v[k]);
+    for (int k = 0; k < NQ; k++)
+      v[k] = MAXLAST && k == NQ - 1 ? dpp_total<true>(v[k]) : dpp_total<false>(v[k]);
     if (lane == 63)
 #pragma unroll
       for (int k = 0; k < NQ; k++) s.red[k][wv] = v[k];
@@ -300,35 +316,37 @@ struct Ctx {
     v[0] = u0.x; v[1] = u0.y; v[2] = u1.x; v[3] = u1.y;
   }
 
-  // z = P z of the thread's cells.  The fragments of P are read while the
-  // inputs go through LDS, and the inputs of every tile before the first
-  // product: the 16 dependent products of a tile then wait on no load
-  // (read four at a time between the products, the LDS latency was paid
-  // four times a tile and the product took twice as long).
+  // z = P z of the thread's cells.  One tile per wave with the fragments of P
+  // in registers (up to 32 blocks): all inputs are read before the first
+  // product, the 16 dependent products then wait on no load (read four at a
+  // time between the products, the LDS latency was paid four times and the
+  // product took twice as long).  Fragments in LDS (48 and 64 blocks): half of
+  // the operands at a time, for the registers; the SIMD's other waves fill in.
   __device__ __forceinline__ void prec(const PFrag64 &F, double (&z)[T][4]) {
-    double2 f[8], u[8], un[8];
     to_lds(z);
-#pragma unroll
-    for (int k = 0; k < 8; k++) f[k] = T == 1 ? make_double2(F.a[2 * k], F.a[2 * k + 1]) : s.pf[(w * 8 + k) * 64 + lane];
     __syncthreads();
-    auto input = [&](int tt, double2 (&v)[8]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int k = 0; k < 8; k++) v[k] = reinterpret_cast<const double2 *>(s.z + lb(tt) * ZS + 16 * q)[k];
-    };
-    input(0, u);
+    constexpr int H = S::PF ? 2 : 1, N = 8 / H;
     f64x4 acc[T];
 #pragma unroll
-    for (int tt = 0; tt < T; tt++) {
-      if (tt + 1 < T) input(tt + 1, un);
+    for (int tt = 0; tt < T; tt++) acc[tt] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+      double2 f[N], u[T][N];
+#pragma unroll
+      for (int k = 0; k < N; k++)
+        f[k] = S::PF ? s.pf[(w * 8 + h * N + k) * 64 + lane] : make_double2(F.a[2 * k], F.a[2 * k + 1]);
+#pragma unroll
+      for (int tt = 0; tt < T; tt++)
+#pragma unroll
+        for (int k = 0; k < N; k++) u[tt][k] = reinterpret_cast<const double2 *>(s.z + lb(tt) * ZS + 16 * q)[h * N + k];
       __builtin_amdgcn_sched_barrier(0);
-      acc[tt] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int k = 0; k < 8; k++) {
-        acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].x, u[k].x, acc[tt], 0, 0, 0);
-        acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].y, u[k].y, acc[tt], 0, 0, 0);
+      for (int k = 0; k < N; k++) {
+#pragma unroll
+        for (int tt = 0; tt < T; tt++) acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].x, u[tt][k].x, acc[tt], 0, 0, 0);
+#pragma unroll
+        for (int tt = 0; tt < T; tt++) acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].y, u[tt][k].y, acc[tt], 0, 0, 0);
       }
-#pragma unroll
-      for (int k = 0; k < 8; k++) u[k] = un[k];
     }
     // The product's results are read 20 and more cycles after the last
     // instruction: said here, because the compiler's own count once let the
@@ -378,25 +396,27 @@ struct Ctx {
   __device__ __forceinline__ void spmv(const double (&z)[T][4], double (&y)[T][4], int limit) {
     const double *zb = halo();
     to_lds(z);
+    int4 face[T];
+    u64 mask[T];
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+      face[tt] = s.face[lb(tt)];
+      mask[tt] = s.mask[lb(tt)];
+    }
     __syncthreads();
     publish<false>(halo());
     // The ghosts are asked for, the explicit rows without any are computed
     // while they travel, and the others follow.
-    const int ng = uni(s.ng);
-    const int g0 = min(tid, ng - 1), g1 = min(tid + WGS, ng - 1);
-    u64 v0 = 0, v1 = 0;
-    if (ng > 0) {
-      v0 = ld_agent(reinterpret_cast<const u64 *>(zb + s.ghost[g0]));
-      v1 = ld_agent(reinterpret_cast<const u64 *>(zb + s.ghost[g1]));
-    }
+    u64 v0 = 0;
+    if (tid < ng) v0 = ld_agent(reinterpret_cast<const u64 *>(zb + ig));
     explicit_rows(0, zb, limit);
-    if (ng > 0) {
-      s.z[S::GHOST0 + g0] = remote(zb + s.ghost[g0], v0, limit);
-      s.z[S::GHOST0 + g1] = remote(zb + s.ghost[g1], v1, limit);
-      for (int g = tid + 2 * WGS; g < ng; g += WGS) s.z[S::GHOST0 + g] = remote(zb + s.ghost[g], EMPTY, limit);
+    if (tid < ng) {
+      s.z[S::GHOST0 + tid] = remote(zb + ig, v0, limit);
+#pragma unroll 1
+      for (int g = tid + WGS; g < ng; g += WGS) s.z[S::GHOST0 + g] = remote(zb + s.ghost[g], EMPTY, limit);
     }
     __syncthreads();
-    if (uni(s.nf) > 0) {
+    if (nf > 0) {
       explicit_rows(64, zb, limit);
       __syncthreads();
     }
@@ -404,7 +424,7 @@ struct Ctx {
 #pragma unroll
     for (int tt = 0; tt < T; tt++) {
       const int base = lb(tt) * ZS;
-      const int4 f = s.face[lb(tt)];
+      const int4 f = face[tt];
       const int fx = ix0 == 0 ? f.x : f.y;
       const double mid = s.z[base + row * 8 + (ix0 == 0 ? 4 : 3)];  // across the middle of the row
       const double hx = s.z[fx + (fx < S::GHOST0 ? 8 * row : row)];
@@ -418,7 +438,7 @@ struct Ctx {
         const double xr = k < 3 ? z[tt][k < 3 ? k + 1 : 3] : hi;
         y[tt][k] = ((dn[k] + xl) + xr) + up[k] - 4.0 * z[tt][k];
       }
-      const u64 m = s.mask[lb(tt)];
+      const u64 m = mask[tt];
       const unsigned em = (unsigned)(m >> c0) & 15u;
       if (em) {  // the block's explicit rows come in the order of its mask's bits
         int at = s.eoff[lb(tt)] + __popcll(m & ((1ull << c0) - 1));
@@ -534,19 +554,26 @@ struct Ctx {
       s.ewid[k] = (unsigned char)(fits ? (far ? 64 : 0) + width : 192 + width);
     }
     __syncthreads();
-    if (tid == 0 && s.ng > S::GHOSTS) s.ng = S::GHOSTS;
+    ni8 = 8 * uni(s.ni);
+    ng = min(uni(s.ng), S::GHOSTS);
+    nf = uni(s.nf);
+    iz = io = 0;
+    if (tid < ni8) word(tid, iz, io);
+    ig = s.ghost[min(tid, max(ng - 1, 0))];
   }
 };
 
 #define CELLS                             \
   _Pragma("unroll") for (int tt = 0; tt < T; tt++) _Pragma("unroll") for (int k = 0; k < 4; k++)
 
-// GEN: with the mean row and the infinity norm; without, the two sums of the
-// 2-norm on the operator's plain form.
+// What a task may ask for: the 2-norm on the operator's plain form, the
+// infinity norm on it, or the mean row with either.
+enum { PLAIN, NORM_MAX, MEAN_ROW, KINDS };
+
 // Two waves' worth of registers at least are left to each wave (256): with
 // more, the compiler keeps products in the accumulation registers.
-template <int WGS, int T, bool GEN>
-__global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
+template <int WGS, int T, int KIND>
+__global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   typedef Shared<WGS, T> S;
   static_assert(sizeof(S) <= 160 * 1024, "LDS of a CU");
@@ -555,7 +582,7 @@ __global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
   Ctx<WGS, T> c(a, s);
   const int &tid = c.tid;
   PFrag64 F;  // one tile per wave: the fragments stay in registers; more: in LDS
-  if (T == 1)
+  if (!S::PF)
     load_pfrag64(F, a.pf, c.w, c.lane);
   else
     for (int i = tid; i < 4 * 8 * 64; i += WGS) {  // fragments (w, ks), lane -> (w, ks / 2), lane
@@ -576,10 +603,13 @@ __global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
       int hi = a.n_tasks;  // the last task whose first ticket is not beyond this one
       while (hi - id > 1) {
         const int mid = (id + hi) >> 1;
-        if (a.task[mid].ticket0 <= tk) id = mid;
+        if (uni(a.task[mid].ticket0) <= tk) id = mid;
         else hi = mid;
       }
-      c.t = a.task[id];
+      const int *f = reinterpret_cast<const int *>(a.task + id);
+      int *to = reinterpret_cast<int *>(&c.t);
+#pragma unroll
+      for (int i = 0; i < (int)(sizeof(TeamTask) / sizeof(int)); i++) to[i] = uni(f[i]);
     } else {
       c.t = a.one;
     }
@@ -594,30 +624,32 @@ __global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
     c.ep = c.zp = 0;
     c.lay_out();
 
-    const bool mr = GEN && t.mean_row >= 0;
+    const bool mr = KIND == MEAN_ROW && t.mean_row >= 0;
     // the state's constants, and the state itself (every thread keeps and
     // advances it from the same totals)
     const Scal *st = a.st + id;
-    const bool l2 = !GEN || st->norm;
-    const int max_iter = st->max_iter, max_restarts = st->max_restarts;
-    const bool confirm = st->rep_factor > 0.0;
-    const double eps = st->eps, tol_abs = st->tol_abs, tol_rel = st->tol_rel, bd_tol = st->bd_tol;
+    const bool l2 = KIND == PLAIN || (KIND == MEAN_ROW && uni(st->norm));
+    const int max_iter = uni(st->max_iter), max_restarts = uni(st->max_restarts);
+    const bool confirm = uni(st->rep_factor) > 0.0;
+    const double eps = uni(st->eps), tol_abs = uni(st->tol_abs), tol_rel = uni(st->tol_rel), bd_tol = uni(st->bd_tol);
     double err = 0.0, err0 = 0.0, size_opt = 0.0, err_rep = 0.0, rho = 0.0, target = 0.0;
     int iter = 0, restarts = 0, n_rep = 0;
     bool done = false, converged = false, improved = false;
 
     double r[T][4], rhat[T][4], p[T][4], nu[T][4], x[T][4];
     double hh = 0.0, alpha = 0.0, omega = 1.0, mean = 0.0;
-    u64 tick = 0, ph[TEAM_PHASES] = {0, 0, 0, 0, 0};
     const bool prof = a.phase && c.rank == 0 && wave_id() == 0;
     auto lap = [&](int k) __attribute__((always_inline)) {
-      if (prof) {
+      if (__builtin_expect(prof, 0) && tid == 0) {
         const u64 now = wall_clock64();
-        ph[k] += now - tick;
-        tick = now;
+        s.phase[k] += now - s.tick;
+        s.tick = now;
       }
     };
-    if (prof) tick = wall_clock64();
+    if (prof && tid == 0) {
+      for (int k = 0; k < TEAM_PHASES; k++) s.phase[k] = 0;
+      s.tick = wall_clock64();
+    }
 #pragma unroll
     for (int tt = 0; tt < T; tt++) {
 #pragma unroll
@@ -633,91 +665,80 @@ __global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
       c.template exchange<2, false>(v, a.form_polls);
     }
 
-    // A pass of this loop is one application of the operator and what hangs
-    // on it: the residual r = b - A x (at the start and to confirm
-    // convergence), nu = A P p with alpha, or t = A P s with omega -- one
-    // copy of the code for all three, which keeps the loop in the
-    // instruction cache -- or the mean of the returned iterate.
-    enum { RES, NU, TS, FIN };
-    int mode = RES;
-    bool replaced = false;
-    while (!c.dead) {
-      c.place();
-      double z[T][4], y[T][4];
-      double v[GEN ? 4 : 2] = {};
-      if (mode != FIN) {
-        if (mode == NU) {
-          CELLS z[tt][k] = p[tt][k];
-        } else if (mode == TS) {
-          CELLS z[tt][k] = r[tt][k];
-        } else {
-          CELLS z[tt][k] = x[tt][k];
-        }
-        if (mode != RES) {
-          c.prec(F, z);
-          lap(1);
-        }
-        c.place();
-        c.spmv(z, y, TEAM_POLLS);
-        if constexpr (GEN)
-          if (mr) CELLS {  // the mean row: sum h^2 z, and the other factor's value there
-            v[2] += s.h2[c.lb(tt)] * z[tt][k];
-            if (c.ok(tt) && c.cell(tt) + k == t.mean_row) {
-              y[tt][k] = 0.0;
-              v[3] = mode == NU ? rhat[tt][k] : r[tt][k];
-            }
-          }
-        if (mode == NU) {
-          CELLS v[0] += y[tt][k] * rhat[tt][k];
-        } else {
-          CELLS {
-            v[0] += y[tt][k] * r[tt][k];
-            v[1] += y[tt][k] * y[tt][k];
+    // y = A z; the mean row: sum h^2 z in v[2], the other factor's value there in v[3]
+    double z[T][4], y[T][4];
+    auto mean_row = [&](double (&v)[4], const double (&other)[T][4]) __attribute__((always_inline)) {
+      if constexpr (KIND == MEAN_ROW)
+        if (mr) CELLS {
+          v[2] += s.h2[c.lb(tt)] * z[tt][k];
+          if (c.ok(tt) && c.cell(tt) + k == t.mean_row) {
+            y[tt][k] = 0.0;
+            v[3] = other[tt][k];
           }
         }
-        lap(0);
-      } else {
-        CELLS {
-          const double w2 = s.h2[c.lb(tt)];
-          v[0] += x[tt][k] * w2;
-          v[1] += w2;
-        }
-      }
-      c.place();
-      c.template exchange<GEN ? 4 : 2, false>(v, TEAM_POLLS);
-      if (c.dead) break;
-      if (mode == FIN) {  // the h^2-weighted mean removed (ExpAMRSolver.cpp:383-415)
-        mean = tot(0) / tot(1);
-#pragma unroll
-        for (int tt = 0; tt < T; tt++)
-          if (c.ok(tt))
-#pragma unroll
-            for (int k = 0; k < 4; k++) a.out[c.cell(tt) + k] = x[tt][k] - mean;
-        break;
-      }
+    };
+    auto put_mean_row = [&]() __attribute__((always_inline)) {
       if (mr) CELLS if (c.ok(tt) && c.cell(tt) + k == t.mean_row) y[tt][k] = tot(2);
-      double coef;
-      if (mode == NU) {
-        alpha = coef = uni(rho / (tot(0) + (mr ? tot(3) * tot(2) : 0.0) + eps));
-      } else {
-        const double ts = tot(0) + (mr ? tot(2) * tot(3) : 0.0);
-        const double tq = tot(1) + (mr ? tot(2) * tot(2) : 0.0);
-        omega = coef = uni(ts / (tq + eps));
+    };
+    auto keep = [&]() __attribute__((always_inline)) {  // the iterate is the best so far
+#pragma unroll
+      for (int tt = 0; tt < T; tt++)
+        if (c.ok(tt)) st4(a.xopt, c.cell(tt), x[tt]);
+    };
+    auto recall = [&]() __attribute__((always_inline)) {  // go on with the best one
+#pragma unroll
+      for (int tt = 0; tt < T; tt++)
+        if (c.ok(tt)) ld4(a.xopt, c.cell(tt), x[tt]);
+    };
+    // the size of the residual as it is compared: |r|^2 or |r|_inf
+    auto norm_of = [l2](double v) { return l2 ? sqrt(v) : v; };
+    double beta = 0.0;
+    bool restart = false, replace = false;
+    // The state at the top of an iteration (kernels.h evaluate: the same
+    // rules, without the projection and the stall window); rho and beta are
+    // the new ones.
+    auto judge = [&](double rr, double size) __attribute__((always_inline)) {
+      iter++;
+      improved = size < size_opt;
+      restart = replace = false;
+      if (improved) size_opt = size;
+      if (__builtin_expect(improved && size <= target, 0)) {
+        err = uni(norm_of(size));
+        if (err <= tol_abs || err / err0 <= tol_rel) {
+          if (confirm) replace = true;  // the recurrence says converged: confirm it on the residual itself
+          else converged = done = true;
+        }
       }
-      if (mode != RES) {  // s = r - alpha nu, or r = s - omega t; x follows
-        CELLS {
-          x[tt][k] = x[tt][k] + coef * z[tt][k];
-          r[tt][k] = r[tt][k] - coef * y[tt][k];
+      if (iter >= max_iter) done = true;
+      const bool breakdown = rho * rho < bd_tol * rr * hh || !(fabs(beta) < 1e30);
+      if (__builtin_expect(breakdown && !done && !replace && max_restarts > 0, 0)) {
+        restarts++;
+        if (restarts >= max_restarts) {
+          done = true;
+        } else {
+          restart = true;
+          hh = rho = rr;  // rhat = r
         }
-        if (mode == NU) {
-          c.clear();
-          CELLS nu[tt][k] = y[tt][k];
-          mode = TS;
-          lap(3);
-          continue;
-        }
-      } else {
-        omega = 1.0;
+      }
+      replace = replace && !done;
+    };
+
+    // Residuals r = b - A x (the start, and the confirmations of a mixed
+    // solve), each followed by iterations.
+    for (;;) {
+      c.place();
+      CELLS z[tt][k] = x[tt][k];
+      c.spmv(z, y, TEAM_POLLS);
+      lap(0);
+      if constexpr (KIND == MEAN_ROW) {
+        double v[4] = {};
+        mean_row(v, z);
+        c.template exchange<4, false>(v, TEAM_POLLS);
+        if (c.dead) break;
+        put_mean_row();
+      }
+      {
+        double f[KIND == PLAIN ? 1 : 2] = {};
 #pragma unroll
         for (int tt = 0; tt < T; tt++) {
 #pragma unroll
@@ -725,105 +746,185 @@ __global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
             const double bb = a.b[c.cell(tt) + k];
             const bool row0 = mr && c.cell(tt) + k == t.mean_row;  // b = 0 there (ExpAMRSolver.cpp:340-345)
             const double ri = c.ok(tt) ? (row0 ? 0.0 : bb) - y[tt][k] : 0.0;
-            r[tt][k] = rhat[tt][k] = ri;
-            p[tt][k] = nu[tt][k] = 0.0;
+            r[tt][k] = rhat[tt][k] = p[tt][k] = ri;
+            f[0] += ri * ri;
+            if constexpr (KIND != PLAIN) f[1] = nmax(f[1], fabs(ri));
           }
         }
+        c.place();
+        c.template exchange<KIND == PLAIN ? 1 : 2, KIND != PLAIN>(f, TEAM_POLLS);
       }
-      double f[GEN ? 3 : 2] = {};
-      CELLS {
-        const double rd = r[tt][k];
-        f[0] += rd * rd;
-        f[1] += rhat[tt][k] * rd;
-        if constexpr (GEN) f[2] = nmax(f[2], fabs(rd));
-      }
-      const double aow = alpha / (omega + eps);  // of beta, before the wait
-      lap(2);
-      c.place();
-      c.template exchange<GEN ? 3 : 2, GEN>(f, TEAM_POLLS);
       if (c.dead) break;
-      // the state at the top of the iteration (kernels.h evaluate: the same
-      // rules, without the projection and the stall window)
-      const double rr = tot(0), rhr = tot(1);
-      bool restart = false, replace = false;
-      double beta = 0.0;
-      // the size of the residual as it is compared: |r|^2 or |r|_inf
-      const double size = l2 ? rr : tot(2);
-      auto norm_of = [l2](double v) { return l2 ? sqrt(v) : v; };
-      if (mode == RES) {
-        err = uni(norm_of(size));
-        if (replaced) {
-          n_rep++;
-        } else {
-          err0 = err;
-          // sizes above this have not converged (the test itself is exact)
-          const double most = fmax(tol_abs, tol_rel * err0) * (1.0 + 1e-9);
-          target = uni(l2 ? most * most : most);
-        }
-        size_opt = size;
-        err_rep = err;
-        hh = rho = rr;
-        improved = replaced;
-        done = err == 0.0 || iter >= max_iter;
-        if (replaced && (err <= tol_abs || err / err0 <= tol_rel)) converged = done = true;
-        if (a.start != TEAM_PLAIN) {
-          if (err != err || err > 1.79e308) {
-            done = true;
-            converged = false;
-          } else if (!replaced && (err == 0.0 || (a.start == TEAM_ACCEPTS && (err <= tol_abs || tol_rel >= 1.0)))) {
-            converged = done = true;
-          }
-        }
-        if (n_rep >= TEAM_MAX_CONFIRM) done = true;
-      } else {
-        iter++;
-        improved = false;
-        if (size < size_opt) {
-          improved = true;
-          size_opt = size;
-          if (size <= target && ((err = uni(norm_of(size))) <= tol_abs || err / err0 <= tol_rel)) {
-            if (confirm) replace = true;  // the recurrence says converged: confirm it on the residual itself
-            else converged = done = true;
-          }
-        }
-        if (iter >= max_iter) done = true;
-        beta = uni((rhr / (rho + eps)) * aow);
-        rho = rhr;
-        const bool breakdown = rhr * rhr < bd_tol * rr * hh || !(fabs(beta) < 1e30);
-        if (!done && !replace && breakdown && max_restarts > 0) {
-          restarts++;
-          if (restarts >= max_restarts) {
-            done = true;
-          } else {
-            restart = true;
-            hh = rho = rr;  // rhat = r
-          }
-        }
-        replace = replace && !done;
-      }
       c.clear();
-      lap(mode == RES ? 4 : 3);
-      replaced = replace;
-      if (improved) {
-        if (!done && !replace)  // the iterate is the best so far
-#pragma unroll
-          for (int tt = 0; tt < T; tt++)
-            if (c.ok(tt)) st4(a.xopt, c.cell(tt), x[tt]);
-      } else if (done || replace) {  // go on with the best one
-#pragma unroll
-        for (int tt = 0; tt < T; tt++)
-          if (c.ok(tt)) ld4(a.xopt, c.cell(tt), x[tt]);
-      }
-      if (done || replace) {
-        mode = done ? FIN : RES;
-        continue;
-      }
-      if (restart) {
-        CELLS rhat[tt][k] = p[tt][k] = r[tt][k];
+      const double size = l2 ? tot(0) : tot(1);
+      err = uni(norm_of(size));
+      if (replace) {
+        n_rep++;
       } else {
-        CELLS p[tt][k] = r[tt][k] + beta * (p[tt][k] - omega * nu[tt][k]);
+        err0 = err;
+        // sizes above this have not converged (the test itself is exact)
+        const double most = fmax(tol_abs, tol_rel * err0) * (1.0 + 1e-9);
+        target = uni(l2 ? most * most : most);
       }
-      mode = NU;
+      size_opt = size;
+      err_rep = err;
+      hh = rho = tot(0);
+      improved = replace;
+      done = err == 0.0 || iter >= max_iter;
+      if (replace && (err <= tol_abs || err / err0 <= tol_rel)) converged = done = true;
+      if (a.start != TEAM_PLAIN) {
+        if (err != err || err > 1.79e308) {
+          done = true;
+          converged = false;
+        } else if (!replace && (err == 0.0 || (a.start == TEAM_ACCEPTS && (err <= tol_abs || tol_rel >= 1.0)))) {
+          converged = done = true;
+        }
+      }
+      if (n_rep >= TEAM_MAX_CONFIRM) done = true;
+      if (!done && improved) keep();
+      if (done && !improved) recall();
+      lap(4);
+      if (done) break;
+      beta = 0.0;
+      bool pending = false;  // the last iteration's r is yet to be judged
+      for (;;) {
+        // nu = A P p and alpha.  The size of r, by which the iteration before
+        // is judged, is summed with (rhat, nu), one exchange an iteration
+        // less; the mean row's own sums take its place there.
+        c.place();
+        CELLS z[tt][k] = p[tt][k];
+        c.prec(F, z);
+        lap(1);
+        c.place();
+        c.spmv(z, y, TEAM_POLLS);
+        double coef, by_row = 0.0;
+        {
+          double v[KIND == PLAIN ? 2 : KIND == NORM_MAX ? 3 : 4] = {};
+          if constexpr (KIND == MEAN_ROW) mean_row(v, rhat);
+          CELLS {
+            v[0] += y[tt][k] * rhat[tt][k];
+            if constexpr (KIND != MEAN_ROW) v[1] += r[tt][k] * r[tt][k];
+            if constexpr (KIND == NORM_MAX) v[2] = nmax(v[2], fabs(r[tt][k]));
+          }
+          lap(0);
+          c.place();
+          c.template exchange<KIND == PLAIN ? 2 : KIND == NORM_MAX ? 3 : 4, KIND == NORM_MAX>(v, TEAM_POLLS);
+        }
+        if (c.dead) break;
+        if constexpr (KIND == MEAN_ROW) {
+          if (mr) by_row = tot(3) * tot(2);
+          put_mean_row();
+        } else if (pending) {
+          judge(tot(1), tot(l2 ? 1 : 2));
+          if (__builtin_expect(done || replace || restart, 0)) {  // nothing of this pass is kept
+            c.clear();
+            if (!restart) {
+              if (!improved) recall();
+              break;
+            }
+            if (improved) keep();
+            CELLS rhat[tt][k] = p[tt][k] = r[tt][k];
+            pending = false;
+            continue;
+          }
+          if (improved) keep();
+        }
+        alpha = coef = uni(rho / (tot(0) + by_row + eps));
+        CELLS {  // s = r - alpha nu; x follows
+          x[tt][k] = x[tt][k] + coef * z[tt][k];
+          r[tt][k] = r[tt][k] - coef * y[tt][k];
+          nu[tt][k] = y[tt][k];
+        }
+        c.clear();
+        lap(3);
+        // t = A P s and omega
+        c.place();
+        CELLS z[tt][k] = r[tt][k];
+        c.prec(F, z);
+        lap(1);
+        c.place();
+        c.spmv(z, y, TEAM_POLLS);
+        {
+          double v[4] = {};
+          if constexpr (KIND == MEAN_ROW) mean_row(v, r);
+          CELLS {
+            v[0] += y[tt][k] * r[tt][k];
+            v[1] += y[tt][k] * y[tt][k];
+            if constexpr (KIND != MEAN_ROW) {
+              v[2] += y[tt][k] * rhat[tt][k];
+              v[3] += r[tt][k] * rhat[tt][k];
+            }
+          }
+          lap(0);
+          c.place();
+          c.template exchange<4, false>(v, TEAM_POLLS);
+        }
+        if (c.dead) break;
+        double ts = tot(0), tq = tot(1);
+        if constexpr (KIND == MEAN_ROW) {
+          if (mr) {
+            ts += tot(2) * tot(3);
+            tq += tot(2) * tot(2);
+          }
+          put_mean_row();
+        }
+        omega = coef = uni(ts / (tq + eps));
+        CELLS {  // r = s - omega t
+          x[tt][k] = x[tt][k] + coef * z[tt][k];
+          r[tt][k] = r[tt][k] - coef * y[tt][k];
+        }
+        const double aow = alpha / (omega + eps);
+        if constexpr (KIND == MEAN_ROW) {
+          double f[3] = {};
+          CELLS {
+            const double rd = r[tt][k];
+            f[0] += rd * rd;
+            f[1] += rhat[tt][k] * rd;
+            f[2] = nmax(f[2], fabs(rd));
+          }
+          lap(2);
+          c.place();
+          c.template exchange<3, true>(f, TEAM_POLLS);
+          if (c.dead) break;
+          beta = uni((tot(1) / (rho + eps)) * aow);
+          rho = tot(1);
+          judge(tot(0), tot(l2 ? 0 : 2));
+          c.clear();
+          if (improved && !done && !replace) keep();
+          if (!improved && (done || replace)) recall();
+          if (done || replace) break;
+          if (restart) {
+            CELLS rhat[tt][k] = p[tt][k] = r[tt][k];
+            continue;
+          }
+        } else {
+          // rhat r of r = s - omega t, from this exchange's sums
+          const double rhr = tot(3) - omega * tot(2);
+          beta = uni((rhr / (rho + eps)) * aow);
+          rho = uni(rhr);
+          pending = true;
+          c.clear();
+        }
+        CELLS p[tt][k] = r[tt][k] + beta * (p[tt][k] - omega * nu[tt][k]);
+        lap(3);
+      }
+      if (c.dead || done) break;
+    }
+    if (!c.dead) {  // the h^2-weighted mean removed (ExpAMRSolver.cpp:383-415)
+      double v[2] = {};
+      CELLS {
+        const double w2 = s.h2[c.lb(tt)];
+        v[0] += x[tt][k] * w2;
+        v[1] += w2;
+      }
+      c.place();
+      c.template exchange<2, false>(v, TEAM_POLLS);
+      mean = tot(0) / tot(1);
+#pragma unroll
+      for (int tt = 0; tt < T; tt++)
+        if (c.ok(tt) && !c.dead)
+#pragma unroll
+          for (int k = 0; k < 4; k++) a.out[c.cell(tt) + k] = x[tt][k] - mean;
     }
     if (c.dead) break;
     lap(4);
@@ -840,22 +941,25 @@ __global__ __launch_bounds__(WGS, 2) void k_team(TeamArgs a) {
       o->err_rep = err_rep;
       o->mean = mean;
       if (prof)
-        for (int k = 0; k < TEAM_PHASES; k++) a.phase[(size_t)id * TEAM_PHASES + k] = ph[k];
+        for (int k = 0; k < TEAM_PHASES; k++) a.phase[(size_t)id * TEAM_PHASES + k] = s.phase[k];
     }
     __syncthreads();  // the shared state is rewritten by the next task
   }
 }
 
-template <bool GEN>
+template <int KIND>
 const void *shape_kernel(int shape) {
-  return shape == TEAM_16   ? reinterpret_cast<const void *>(&k_team<256, 1, GEN>)
-         : shape == TEAM_32 ? reinterpret_cast<const void *>(&k_team<512, 1, GEN>)
-                            : reinterpret_cast<const void *>(&k_team<512, 2, GEN>);
+  return shape == TEAM_16   ? reinterpret_cast<const void *>(&k_team<256, 1, KIND>)
+         : shape == TEAM_32 ? reinterpret_cast<const void *>(&k_team<512, 1, KIND>)
+         : shape == TEAM_48 ? reinterpret_cast<const void *>(&k_team<768, 1, KIND>)
+                            : reinterpret_cast<const void *>(&k_team<512, 2, KIND>);
 }
-const void *shape_kernel(int shape, bool gen) { return gen ? shape_kernel<true>(shape) : shape_kernel<false>(shape); }
-int shape_threads(int shape) { return shape == TEAM_16 ? 256 : 512; }
+const void *shape_kernel(int shape, int kind) {
+  return kind == PLAIN ? shape_kernel<PLAIN>(shape) : kind == NORM_MAX ? shape_kernel<NORM_MAX>(shape) : shape_kernel<MEAN_ROW>(shape);
+}
+int shape_threads(int shape) { return shape == TEAM_64 ? 512 : 16 * team_blocks(shape); }
 size_t shape_lds(int shape) {
-  return shape == TEAM_16 ? sizeof(Shared<256, 1>) : shape == TEAM_32 ? sizeof(Shared<512, 1>) : sizeof(Shared<512, 2>);
+  return shape == TEAM_16 ? sizeof(Shared<256, 1>) : shape == TEAM_32 ? sizeof(Shared<512, 1>) : shape == TEAM_48 ? sizeof(Shared<768, 1>) : sizeof(Shared<512, 2>);
 }
 
 }  // namespace
@@ -867,8 +971,8 @@ int team_resident(int shape) {
   if (const int n = known[dev][shape].load()) return n;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
   int least = 1 << 30;
-  for (const bool gen : {false, true}) {
-    const void *k = shape_kernel(shape, gen);
+  for (int kind = 0; kind < KINDS; kind++) {
+    const void *k = shape_kernel(shape, kind);
     int per = 0;
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape_lds(shape)) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, shape_threads(shape), shape_lds(shape)) != hipSuccess)
@@ -885,7 +989,7 @@ hipError_t team_launch(const TeamArgs &a, int shape, size_t n_words, int grid, h
   if (e == hipSuccess) e = hipMemsetAsync(a.ctl, 0, 2 * sizeof(int), stream);
   if (e != hipSuccess) return e;
   void *params[] = {&args};
-  return hipLaunchCooperativeKernel(shape_kernel(shape, a.gen), dim3(grid), dim3(shape_threads(shape)),
+  return hipLaunchCooperativeKernel(shape_kernel(shape, a.mean_rows ? MEAN_ROW : a.norm_max ? NORM_MAX : PLAIN), dim3(grid), dim3(shape_threads(shape)),
                                     params, (unsigned)shape_lds(shape), stream);
 }
 

@@ -1,6 +1,6 @@
 """The on-chip solve (csrc/team.hip) at the edges of its work split: one
-workgroup, the first and last meshes of each launch shape (16, 32 and 64 blocks
-per workgroup, 256 workgroups), the first mesh beyond it, remainders, block
+workgroup, the first and last meshes of each launch shape (16, 32, 48 and 64
+blocks per workgroup, 256 workgroups), the first mesh beyond it, remainders, block
 orders in which every neighbour lies in another workgroup, and explicit rows on
 both sides of a workgroup's edge.
 
@@ -26,7 +26,7 @@ def _shuffled(m, seed):
                          m.periodic_y)
 
 
-GRIDS = [(1, 1), (2, 1), (5, 3), (4, 4), (17, 1), (11, 3), (13, 5), (64, 64), (241, 17), (91, 90), (331, 25), (128, 128),
+GRIDS = [(1, 1), (2, 1), (5, 3), (4, 4), (17, 1), (11, 3), (13, 5), (64, 64), (241, 17), (91, 90), (331, 25), (128, 96), (25, 492), (128, 128),
          (331, 50)]
 
 
@@ -70,6 +70,23 @@ def test_block_orders_and_coarse_fine_rows(oracle, name, mc):
         bm[A.mean_row] = 0.0
     tr = oracle.true_residual(A, bm, x1, mean_mode=mc, h2v=oracle.h2(m))
     assert abs(tr["rel2"] - s1["true_rel2"]) <= 1e-9 * tr["rel2"]
+
+
+@pytest.mark.parametrize("norm,mc", [(PS.NORM_L2, 0), (PS.NORM_INF, 0), (PS.NORM_L2, 1)])
+@pytest.mark.parametrize("max_iter,breakdown_tol,max_restarts", [(1, 1e-14, 100), (2, 1e-14, 100), (3, 1e-14, 100),
+                                                                 (12, 0.3, 100), (12, 0.3, 3), (12, 0.9, 100)])
+def test_last_iterations_and_restarts(norm, mc, max_iter, breakdown_tol, max_restarts):
+    """An iteration is judged when the next one's first sums arrive: the last one, and those that restart (a large
+    breakdown tolerance: nearly all), end as the one-operation-per-launch solver's do."""
+    m = W.graded_disk_mesh()
+    b = W.vortex_rhs(m, 3)
+    cfg = dict(norm=norm, max_iter=max_iter, mean_constraint=mc, breakdown_tol=breakdown_tol)
+    x1, s1 = PS.Solver(**cfg).set_mesh(m, on_device=True).solve(b, rel_tol=1e-30, max_restarts=max_restarts)
+    x2, s2 = PS.Solver(schedule=1, **cfg).set_mesh(m).solve(b, rel_tol=1e-30, max_restarts=max_restarts)
+    assert (s1["iterations"], s1["restarts"]) == (s2["iterations"], s2["restarts"])
+    assert s2["restarts"] >= (2 if breakdown_tol > 0.1 else 0)
+    assert np.linalg.norm(x1 - x2) <= 1e-10 * np.linalg.norm(x2)
+    assert abs(s1["err_final"] - s2["err_final"]) <= 1e-10 * s2["err_final"]
 
 
 @pytest.mark.parametrize("precision", [PS.FP64, PS.MIXED])
