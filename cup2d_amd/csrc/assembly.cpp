@@ -456,4 +456,24 @@ std::vector<double> make_pfrag64(const std::vector<double> &P) {
   return f;
 }
 
+// P commutes with the reflections of the block, so it maps the part of a
+// field that is even or odd in x and in y to a part of the same kind, which
+// its quadrant (16 cells) determines: four 16 x 16 products in place of one of
+// 64 x 64.  Class c (odd in x: c & 1, odd in y: c & 2), output and input cell
+// of the quadrant: the sum of P over the input's mirror images with their
+// signs, and the 1/4 of the parts' sum.
+std::vector<double> make_pclass64(const std::vector<double> &P) {
+  std::vector<double> f(4 * 4 * 64);
+  for (int c = 0; c < 4; c++)
+    for (int ks = 0; ks < 4; ks++)
+      for (int l = 0; l < 64; l++) {
+        const int m = l & 15, row = 8 * (m & 3) + (m >> 2), y = l >> 4, x = ks;
+        const long double sx = c & 1 ? -1 : 1, sy = c & 2 ? -1 : 1;
+        const long double v = P[row * 64 + 8 * y + x] + sx * P[row * 64 + 8 * y + 7 - x] +
+                              sy * (P[row * 64 + 8 * (7 - y) + x] + sx * P[row * 64 + 8 * (7 - y) + 7 - x]);
+        f[(c * 4 + ks) * 64 + l] = (double)(0.25L * v);
+      }
+  return f;
+}
+
 }  // namespace cup2d

@@ -118,4 +118,8 @@ std::vector<uint16_t> make_pfrag(const std::vector<double> &P);
 // registers of a lane four consecutive cells (see tile_prec64).
 std::vector<double> make_pfrag64(const std::vector<double> &P);
 
+// P on the parts of a block that are even or odd in x and y, as A operands of
+// v_mfma_f64_16x16x4_f64: class c, K step ks, lane l.
+std::vector<double> make_pclass64(const std::vector<double> &P);
+
 }  // namespace cup2d

@@ -1160,6 +1160,7 @@ struct cup2d_psb {
   int *d_erow = nullptr, *d_ecol = nullptr;
   uint16_t *d_ecode = nullptr;
   double *d_etab = nullptr, *d_h2 = nullptr, *d_P = nullptr;
+  double *d_pc = nullptr;           // MFMA fragments of P_inv's classes (make_pclass64)
   std::vector<uint8_t> elen;        // [n_exc] entries of each explicit row
   int ell_w = 0;
   bf16x8 *d_pfrag = nullptr;
@@ -1643,7 +1644,7 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   TeamArgs a{};
   a.A = bview(h).A;
   a.fid = h->d_fid;
-  a.pf = h->d_P;
+  a.pc = h->d_pc;
   a.b = d_b;
   a.x0 = d_x0;
   a.out = h->d_x;
@@ -2142,8 +2143,8 @@ static int finish_meshes(cup2d_psb *h, int n_inst) {
   int rc;
   static const std::vector<double> P = make_pinv();  // the same for every mesh
   static const std::vector<uint16_t> pf = make_pfrag(P);
-  static const std::vector<double> pf64 = make_pfrag64(P);
-  if ((rc = bupload(h, pool, &h->d_P, pf64)) || (rc = bupload(h, pool, &h->d_mean_row, h->h_mean_row)))
+  static const std::vector<double> pf64 = make_pfrag64(P), pc64 = make_pclass64(P);
+  if ((rc = bupload(h, pool, &h->d_P, pf64)) || (rc = bupload(h, pool, &h->d_pc, pc64)) || (rc = bupload(h, pool, &h->d_mean_row, h->h_mean_row)))
     return rc;
   if ((rc = balloc(h, pool, &h->d_pfrag, pf.size() / 8))) return rc;
   BCHK(h, hipMemcpy(h->d_pfrag, pf.data(), pf.size() * sizeof(uint16_t), hipMemcpyHostToDevice));

@@ -886,6 +886,7 @@ struct cup2d_ps {
   int *d_csr_rp = nullptr, *d_csr_col = nullptr;
   double *d_csr_val = nullptr;
   double *d_P = nullptr;                 // FP64 MFMA fragments of P_inv (make_pfrag64)
+  double *d_pc = nullptr;                // of its classes (make_pclass64)
   bf16x8 *d_pf = nullptr;                // BF16 MFMA fragments of P_inv
   // FP64 work vectors (x is the solution in both precisions)
   double *d_x = nullptr, *d_xopt = nullptr, *d_r = nullptr, *d_rhat = nullptr, *d_p = nullptr,
@@ -1266,7 +1267,7 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   TeamArgs a{};
   a.A = view(h);
   a.fid = h->d_fid;
-  a.pf = h->d_P;
+  a.pc = h->d_pc;
   a.b = d_b;
   a.x0 = d_x0;
   a.out = h->d_x;  // d_out, which may be x0, is written once the launch has succeeded
@@ -1918,8 +1919,8 @@ static int finish_mesh(cup2d_ps *h) {
   int rc = 0;
   static const std::vector<double> P = make_pinv();  // the same for every mesh
   static const std::vector<uint16_t> pf = make_pfrag(P);
-  static const std::vector<double> pf64 = make_pfrag64(P);
-  if ((rc = upload(h, &h->d_P, pf64)) || (rc = dalloc(h, &h->d_pf, 8 * 64))) return rc;
+  static const std::vector<double> pf64 = make_pfrag64(P), pc64 = make_pclass64(P);
+  if ((rc = upload(h, &h->d_P, pf64)) || (rc = upload(h, &h->d_pc, pc64)) || (rc = dalloc(h, &h->d_pf, 8 * 64))) return rc;
   HIPCHK(h, hipMemcpy(h->d_pf, pf.data(), pf.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
   const size_t n = op.n;
   double **vecs[] = {&h->d_x, &h->d_xopt, &h->d_r, &h->d_rhat, &h->d_p, &h->d_nu, &h->d_b, &h->d_xio};

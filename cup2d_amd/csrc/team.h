@@ -38,7 +38,7 @@ constexpr size_t team_words(int nwg) { return (size_t)nwg * TEAM_SLOT_WORDS * te
 struct TeamArgs {
   OpView A;
   const int2 *fid;
-  const double *pf;                     // FP64 MFMA fragments of P_inv
+  const double *pc;                     // FP64 MFMA fragments of P_inv's classes
   const double *b, *x0;
   double *out;
   double *halo;                         // [3 n] what the workgroups read of each other

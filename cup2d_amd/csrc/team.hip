@@ -123,12 +123,11 @@ constexpr int TAB = 256;                                     // coefficients kep
 template <int WGS, int T>
 struct Shared {
   static constexpr int BPW = WGS / 256 * T * TILE, NW = WGS / 64;
-  static constexpr bool PF = BPW > 32;                        // P_inv in LDS, else in registers
   static constexpr int GHOST0 = BPW * ZS, GHOSTS = BPW * 40;  // first, most cells of other workgroups
   static constexpr int ITEMS = BPW * 12;                      // a block's 4 faces and 8 rows
   static constexpr int ROWS = BPW == 64 ? 512 : BPW == 48 ? 768 : face_rows(BPW);  // explicit rows kept in LDS
   double z[GHOST0 + GHOSTS];        // the workgroup's blocks (product inputs, then z), then the ghosts
-  double2 pf[PF ? 4 * 8 * 64 : 1];  // P_inv's fragments, two K steps a word
+  double part[GHOST0];              // P v of the blocks, by class
   double ye[face_rows(BPW)];        // A z of the explicit rows
   double tab[TAB];
   double red[TEAM_NQ][NW], tot[TEAM_NQ];  // a wave per quantity: TEAM_NQ <= NW
@@ -316,37 +315,29 @@ struct Ctx {
     v[0] = u0.x; v[1] = u0.y; v[2] = u1.x; v[3] = u1.y;
   }
 
-  // z = P z of the thread's cells.  One tile per wave with the fragments of P
-  // in registers (up to 32 blocks): all inputs are read before the first
-  // product, the 16 dependent products then wait on no load (read four at a
-  // time between the products, the LDS latency was paid four times and the
-  // product took twice as long).  Fragments in LDS (48 and 64 blocks): half of
-  // the operands at a time, for the registers; the SIMD's other waves fill in.
-  __device__ __forceinline__ void prec(const PFrag64 &F, double (&z)[T][4]) {
+  // z = P z of the thread's cells, by parts that are even or odd in x and y
+  // (make_pclass64): the tile's wave w forms the quadrant of part w, 4
+  // products in place of 16, and the parts are put together through LDS.
+  // Against the 64 x 64 product, whose operands took as many LDS reads:
+  // us an iteration @@
+  __device__ __forceinline__ void prec(const double (&F)[4], double (&z)[T][4]) {
     to_lds(z);
     __syncthreads();
-    constexpr int H = S::PF ? 2 : 1, N = 8 / H;
+    const double sx = w & 1 ? -1.0 : 1.0, sy = w & 2 ? -1.0 : 1.0;
     f64x4 acc[T];
 #pragma unroll
-    for (int tt = 0; tt < T; tt++) acc[tt] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int tt = 0; tt < T; tt++) {
+      double lo[2][4], hi[2][4], in[4];  // rows q and 7 - q
+      from_lds(lb(tt) * ZS + 8 * q, lo[0]);
+      from_lds(lb(tt) * ZS + 8 * q + 4, lo[1]);
+      from_lds(lb(tt) * ZS + 8 * (7 - q), hi[0]);
+      from_lds(lb(tt) * ZS + 8 * (7 - q) + 4, hi[1]);
 #pragma unroll
-    for (int h = 0; h < H; h++) {
-      double2 f[N], u[T][N];
+      for (int k = 0; k < 4; k++)
+        in[k] = fma(sy, fma(sx, hi[1][3 - k], hi[0][k]), fma(sx, lo[1][3 - k], lo[0][k]));
+      acc[tt] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int k = 0; k < N; k++)
-        f[k] = S::PF ? s.pf[(w * 8 + h * N + k) * 64 + lane] : make_double2(F.a[2 * k], F.a[2 * k + 1]);
-#pragma unroll
-      for (int tt = 0; tt < T; tt++)
-#pragma unroll
-        for (int k = 0; k < N; k++) u[tt][k] = reinterpret_cast<const double2 *>(s.z + lb(tt) * ZS + 16 * q)[h * N + k];
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-#pragma unroll
-        for (int tt = 0; tt < T; tt++) acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].x, u[tt][k].x, acc[tt], 0, 0, 0);
-#pragma unroll
-        for (int tt = 0; tt < T; tt++) acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[k].y, u[tt][k].y, acc[tt], 0, 0, 0);
-      }
+      for (int k = 0; k < 4; k++) acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(F[k], in[k], acc[tt], 0, 0, 0);
     }
     // The product's results are read 20 and more cycles after the last
     // instruction: said here, because the compiler's own count once let the
@@ -355,10 +346,30 @@ struct Ctx {
     if constexpr (T == 1) asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]));
     else asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[T - 1]));
 #pragma unroll
-    for (int tt = 0; tt < T; tt++)
+    for (int tt = 0; tt < T; tt++) {
+      double2 *d = reinterpret_cast<double2 *>(s.part + lb(tt) * ZS + c0);
+      d[0] = make_double2(acc[tt][0], acc[tt][1]);
+      d[1] = make_double2(acc[tt][2], acc[tt][3]);
+    }
+    __syncthreads();
+    const int row = 2 * w + (q >> 1), yq = row < 4 ? row : 7 - row;
+    const bool right = q & 1;  // the row's right half: the quadrant's mirror image
+    const double s2 = w < 2 ? 1.0 : -1.0, s1 = right ? -1.0 : 1.0;
 #pragma unroll
-      for (int k = 0; k < 4; k++) z[tt][k] = acc[tt][k];
-    __syncthreads();  // the inputs are overwritten by z
+    for (int tt = 0; tt < T; tt++) {
+      double v[4][4];
+#pragma unroll
+      for (int cl = 0; cl < 4; cl++) {
+        const double2 *d = reinterpret_cast<const double2 *>(s.part + lb(tt) * ZS + 16 * cl + 4 * yq);
+        const double2 u0 = d[0], u1 = d[1];
+        v[cl][0] = u0.x; v[cl][1] = u0.y; v[cl][2] = u1.x; v[cl][3] = u1.y;
+      }
+      double o[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) o[k] = fma(s1, fma(s2, v[3][k], v[1][k]), fma(s2, v[2][k], v[0][k]));
+#pragma unroll
+      for (int k = 0; k < 4; k++) z[tt][k] = right ? o[3 - k] : o[k];
+    }
   }
 
   // ye = A z of the explicit rows whose kind (0: all entries in LDS from the
@@ -581,14 +592,9 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
   S &s = *reinterpret_cast<S *>(smem);
   Ctx<WGS, T> c(a, s);
   const int &tid = c.tid;
-  PFrag64 F;  // one tile per wave: the fragments stay in registers; more: in LDS
-  if (!S::PF)
-    load_pfrag64(F, a.pf, c.w, c.lane);
-  else
-    for (int i = tid; i < 4 * 8 * 64; i += WGS) {  // fragments (w, ks), lane -> (w, ks / 2), lane
-    const int at = (i >> 6) * 2 * 64 + (i & 63);
-    s.pf[i] = make_double2(a.pf[at], a.pf[at + 64]);
-  }
+  double F[4];  // the wave's class of P_inv
+#pragma unroll
+  for (int k = 0; k < 4; k++) F[k] = a.pc[(c.w * 4 + k) * 64 + c.lane];
   for (int i = tid; i < TAB; i += WGS) s.tab[i] = i < a.n_codes ? a.A.etab[i] : 0.0;
   if (tid == 0) s.bad = 0;
   auto tot = [&](int k) __attribute__((always_inline)) { return uni(s.tot[k]); };
