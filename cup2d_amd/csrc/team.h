@@ -30,8 +30,11 @@ constexpr int TEAM_PHASES = 5;          // cup2d_ps_phase
 // Words of the exchange area per workgroup slot (see team.hip).
 constexpr int TEAM_NQ = 4;              // quantities of one exchange
 constexpr int TEAM_SLOT_WORDS = 2 * 2 * TEAM_NQ;
-// Copies of the exchange words: one per 32 workgroups.
-__host__ __device__ constexpr int team_copies(int nwg) { return (nwg + 31) / 32; }
+// Copies of the exchange words, each read by some of the workgroups: one up to
+// 64 workgroups, then one per 32 (a line that 250 workgroups poll is slow to
+// reach).  Sums by groups of 16 and then over the groups, two waits with 16
+// values each, took 1-2 us an iteration more on 96-256 workgroups.
+__host__ __device__ constexpr int team_copies(int nwg) { return nwg <= 64 ? 1 : (nwg + 31) / 32; }
 // Exchange words of a team.
 constexpr size_t team_words(int nwg) { return (size_t)nwg * TEAM_SLOT_WORDS * team_copies(nwg); }
 

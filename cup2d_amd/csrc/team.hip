@@ -26,10 +26,10 @@
 // workgroup: 20.5 us on 16,384 blocks, 17.6 without).
 //
 // Measured (us per iteration to a relative residual of 1e-12, against five
-// kernels per iteration replayed from a graph): 128 blocks 8.0 against 24.0,
-// 1448 blocks 11.5 against 27.9, 8348 blocks 16.4 against 49.9, 16,229 blocks
-// 20 against 64.8.  On 16k blocks the products (2 x 8192 flop per block at the
-// 72 TFLOP/s of a large FP64 matrix product) are 3.7 us of it.
+// kernels per iteration replayed from a graph): 128 blocks 7.7 against 24.0,
+// 1448 blocks 10.8 against 27.9, 8348 blocks 15.5 against 49.9, 16,229 blocks
+// 19.4 against 64.8.  One workgroup of 64 blocks alone takes 7.4 us, of 16 4.3 us:
+// the rest is the waits and the slowest of the workgroups.
 //
 // Teams form by tickets: a workgroup takes the next ticket, which names its
 // task and its rank, and when its task is solved takes another.  Tickets are
@@ -59,23 +59,22 @@ __device__ __forceinline__ void st_agent(u64 *p, u64 v) {
 
 // N pairs of words (16 bytes each, past the caches), the wait included.
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void ld_pairs(const u64 *p0, u32x4 &v0) {
-  asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v0) : "v"(p0) : "memory");
+__device__ __forceinline__ void ld_pairs(const u64 *const (&p)[1], u32x4 (&v)[1]) {
+  asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v[0]) : "v"(p[0]) : "memory");
 }
-__device__ __forceinline__ void ld_pairs(const u64 *p0, const u64 *p1, u32x4 &v0, u32x4 &v1) {
+__device__ __forceinline__ void ld_pairs(const u64 *const (&p)[2], u32x4 (&v)[2]) {
   asm volatile(
       "global_load_dwordx4 %0, %2, off sc1\n\tglobal_load_dwordx4 %1, %3, off sc1\n\ts_waitcnt vmcnt(0)"
-      : "=&v"(v0), "=&v"(v1)
-      : "v"(p0), "v"(p1)
+      : "=&v"(v[0]), "=&v"(v[1])
+      : "v"(p[0]), "v"(p[1])
       : "memory");
 }
-__device__ __forceinline__ void ld_pairs(const u64 *p0, const u64 *p1, const u64 *p2, const u64 *p3, u32x4 &v0,
-                                         u32x4 &v1, u32x4 &v2, u32x4 &v3) {
+__device__ __forceinline__ void ld_pairs(const u64 *const (&p)[4], u32x4 (&v)[4]) {
   asm volatile(
       "global_load_dwordx4 %0, %4, off sc1\n\tglobal_load_dwordx4 %1, %5, off sc1\n\t"
       "global_load_dwordx4 %2, %6, off sc1\n\tglobal_load_dwordx4 %3, %7, off sc1\n\ts_waitcnt vmcnt(0)"
-      : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
-      : "v"(p0), "v"(p1), "v"(p2), "v"(p3)
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+      : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3])
       : "memory");
 }
 
@@ -233,6 +232,32 @@ struct Ctx {
     zp ^= 1;
   }
 
+  // The total of the n values at p, once they have come, 64 NS or fewer.
+  template <int NS, bool MAXLAST>
+  __device__ __forceinline__ double gather(const u64 *p, int n, bool mx, int limit) {
+    auto op = [mx](double x, double y) { return MAXLAST && mx ? nmax(x, y) : x + y; };
+    const u64 *at[NS];
+    u32x4 v[NS];
+#pragma unroll
+    for (int i = 0; i < NS; i++) at[i] = p + 2 * min(i * 64 + lane, n - 1);
+    unsigned off;
+    int polls = 0;
+    do {
+      ld_pairs(at, v);
+      off = 0;
+#pragma unroll
+      for (int i = 0; i < NS; i++) off |= (v[i].y ^ ep) | (v[i].w ^ ep);
+    } while (off && !dead && !give_up(polls, limit));
+    double r = 0.0;
+#pragma unroll
+    for (int i = 0; i < NS; i++)
+      r = op(r, i * 64 + lane < n ? __longlong_as_double((long long)v[i].z << 32 | v[i].x) : 0.0);
+    r = MAXLAST && mx ? dpp_total<true>(r) : dpp_total<false>(r);
+    const long long b = __double_as_longlong(r);
+    const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+  }
+
   // Sums (the last one a maximum with MAXLAST) of the NQ quantities over
   // the team, in a fixed order, so that every workgroup holds the same totals:
   // lanes, waves, ranks.  The totals are in s.tot.  A wave per quantity
@@ -262,40 +287,16 @@ struct Ctx {
       }
       const int n = t.nwg;
       if (n > 1) {
-        u64 *base = slots + ((ep & 1) ? slab * copies : 0) + 2 * wv * n;
+        u64 *base = slots + (ep & 1 ? slab * copies : 0) + 2 * wv * n;
+        // a value is two words that carry the exchange's number
         const u64 b = (u64)__double_as_longlong(r), tag = (u64)ep << 32;
-        // Large teams write their sums in several copies, each read by some of
-        // the workgroups: a line that 250 workgroups poll is slow to reach.
         if (lane < 2 * copies)
-          st_agent(base + (lane >> 1) * slab + 2 * rank + (lane & 1), tag | ((lane & 1) ? b >> 32 : b & 0xffffffffull));
-        const u64 *sk = base + copy * slab;
-        constexpr int NS = TEAM_MAX_WG / 64;
-        const u64 *p[NS];
-        u32x4 w4[NS];
-#pragma unroll
-        for (int i = 0; i < NS; i++) {
-          p[i] = sk + 2 * min(i * 64 + lane, n - 1);
-          w4[i] = u32x4{0, ep, 0, ep};
-        }
-        unsigned off;
-        int polls = 0;
-        do {
-          if (n > 128) ld_pairs(p[0], p[1], p[2], p[3], w4[0], w4[1], w4[2], w4[3]);
-          else if (n > 64) ld_pairs(p[0], p[1], w4[0], w4[1]);
-          else ld_pairs(p[0], w4[0]);
-          off = 0;
-#pragma unroll
-          for (int i = 0; i < NS; i++) off |= (w4[i].y ^ ep) | (w4[i].w ^ ep);
-        } while (off && !dead && !give_up(polls, limit));
-        r = 0.0;
-#pragma unroll
-        for (int i = 0; i < NS; i++) {
-          const double d = __longlong_as_double((long long)w4[i].z << 32 | w4[i].x);
-          r = op(r, i * 64 + lane < n ? d : 0.0);
-        }
-        r = MAXLAST && mx ? dpp_total<true>(r) : dpp_total<false>(r);
+          st_agent(base + (lane >> 1) * slab + 2 * rank + (lane & 1), tag | (lane & 1 ? b >> 32 : b & 0xffffffffull));
+        const u64 *mine = base + copy * slab;
+        r = n <= 64 ? gather<1, MAXLAST>(mine, n, mx, limit)
+            : n <= 128 ? gather<2, MAXLAST>(mine, n, mx, limit) : gather<4, MAXLAST>(mine, n, mx, limit);
       }
-      if (lane == 63) s.tot[wv] = r;
+      if (lane == 0) s.tot[wv] = r;
     }
     __syncthreads();
     dead = dead || uni(s.bad) != 0;
@@ -318,8 +319,9 @@ struct Ctx {
   // z = P z of the thread's cells, by parts that are even or odd in x and y
   // (make_pclass64): the tile's wave w forms the quadrant of part w, 4
   // products in place of 16, and the parts are put together through LDS.
-  // Against the 64 x 64 product, whose operands took as many LDS reads:
-  // us an iteration @@
+  // An iteration of 16,384 blocks took 17.6 us with the 64 x 64 product (and its
+  // operands in 32 KB of LDS), 16.8 so; of 8348 graded blocks 16.4 and 15.2; the
+  // 64-instance batch 361 ms and 300 ms.
   __device__ __forceinline__ void prec(const double (&F)[4], double (&z)[T][4]) {
     to_lds(z);
     __syncthreads();
