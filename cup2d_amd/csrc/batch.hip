@@ -9,9 +9,9 @@
 // team of workgroups (team.hip), all in one launch: an iteration touches memory
 // for its halo and its sums only, and an instance ends when it converges, its
 // workgroups taking the next.  64 instances of 512-8,192 blocks (13.9 million
-// cells) to 1e-12: 361 ms, by the item kernels 915 ms; 9 small ones in mixed
+// cells) to 1e-12: 298 ms, by the item kernels 915 ms; 9 small ones in mixed
 // precision 22 ms against 53.4 ms.  What bounds it: the workgroups' own work and
-// the waits of a team (18 us an iteration on 64 blocks; 3,389 workgroups' worth
+// the waits of a team (15 us an iteration on 64 blocks; 3,389 workgroups' worth
 // of instances on 256).
 //
 // A batch with a larger instance takes the item kernels, which advance all
@@ -2042,13 +2042,12 @@ static int build_device(cup2d_psb *h, int n_inst, const cup2d_mesh_desc *meshes)
   return CUP2D_PS_OK;
 }
 
-// The order in which instances of n[k] workgroups start on `grid` of them:
-// whenever workgroups come free, the longest instance that fits.  Durations are
-// taken to grow as blocks^(3/4) (iterations grow with the size, an iteration's
-// time hardly does); the tickets then go in this order.  On the 64-instance
-// batch this leaves the workgroups idle for 3 % of the time against 14 % with
-// the largest instances first.
-static std::vector<int> start_order(const std::vector<int> &n, int grid) {
+// The order in which instances of n[k] workgroups, running for d[k], start on
+// `grid` of them: whenever workgroups come free, the longest instance that fits;
+// the tickets then go in this order.  `end`: when the last one ends.  On the
+// 64-instance batch this leaves the workgroups idle for 3 % of the time against
+// 14 % with the largest instances first.
+static std::vector<int> start_order(const std::vector<int> &n, const std::vector<double> &d, int grid, double &end) {
   const int K = (int)n.size();
   std::vector<int> left(K), order;
   for (int k = 0; k < K; k++) left[k] = k;
@@ -2056,13 +2055,15 @@ static std::vector<int> start_order(const std::vector<int> &n, int grid) {
   std::multimap<double, int> running;  // end of an instance, its workgroups
   double t = 0.0;
   int free = grid;
+  end = 0.0;
   while (!left.empty()) {
     size_t kept = 0;
     for (size_t i = 0; i < left.size(); i++) {
       const int k = left[i];
       if (n[k] <= free) {
         free -= n[k];
-        running.emplace(t + std::pow((double)n[k], 0.75), n[k]);
+        running.emplace(t + d[k], n[k]);
+        end = std::max(end, t + d[k]);
         order.push_back(k);
       } else {
         left[kept++] = k;
@@ -2080,54 +2081,65 @@ static std::vector<int> start_order(const std::vector<int> &n, int grid) {
   return order;
 }
 
-// The on-chip solve's teams: the fewest blocks per workgroup with which all
-// instances run at once, because a team's iteration is the shorter the fewer
-// blocks its workgroups hold (16: 8-10 us, 32: 11, 48: 13, 64: 14); else 64
-// blocks per workgroup in start_order, which keep the most instances running
-// (the 64-instance batch in 361 ms, with 48 in 412, with 32 in 515).
+// The on-chip solve's teams: the blocks per workgroup with which the last
+// instance ends first, if iterations grow as the square root of the blocks and
+// one takes TEAM_US + n TEAM_US_WG us on n workgroups (uniform meshes: 16 blocks
+// 7.9 us on 16 workgroups, 9.1 on 64; 32 blocks 9.1 on 16, 10.9 on 128; 48 blocks
+// 11.2 on 32, 14.0 on 171; 64 blocks 11.8 on 16, 14.1 on 128).  Few instances run
+// at once on small shares, many on 64 blocks, which keep the most of them
+// running: the 64-instance batch took 298 ms, with 48 blocks 384, with 32 502.
+constexpr double TEAM_US[TEAM_SHAPES] = {8.2, 8.9, 10.3, 11.3}, TEAM_US_WG = 0.025;
 static int plan_teams(cup2d_psb *h) {
   h->team_shape = -1;
   const int K = h->K;
   long long most = 0;
   for (int k = 0; k < K; k++) most = std::max(most, h->boff[k + 1] - h->boff[k]);
   if (most > TEAM_MAX_BLOCKS) return CUP2D_PS_OK;
-  for (int s = 0; s < TEAM_SHAPES && h->team_shape < 0; s++) {
-    const int grid = std::min(TEAM_MAX_WG, team_resident(s));
+  std::vector<int> order;
+  double best = 0.0;
+  int grid = 0;
+  for (int s = 0; s < TEAM_SHAPES; s++) {
+    const int g = std::min(TEAM_MAX_WG, team_resident(s));
     std::vector<int> wide(K);
-    int tickets = 0, widest = 0;
+    std::vector<double> us(K);
+    int widest = 0;
     for (int k = 0; k < K; k++) {
       TeamTask t{};
       team_split((int)(h->boff[k + 1] - h->boff[k]), team_blocks(s), t);
       wide[k] = t.nwg;
+      us[k] = std::sqrt((double)t.nb) * (TEAM_US[s] + TEAM_US_WG * t.nwg);
       widest = std::max(widest, t.nwg);
-      tickets = std::min(tickets + t.nwg, 1 << 30);
     }
-    if (widest > grid || (tickets > grid && s + 1 < TEAM_SHAPES)) continue;
-    const std::vector<int> order = start_order(wide, grid);
-    std::vector<TeamTask> team;
-    size_t words = 0;
-    tickets = 0;
-    for (int k : order) {
-      TeamTask t{};
-      team_split((int)(h->boff[k + 1] - h->boff[k]), team_blocks(s), t);
-      t.b0 = (int)h->boff[k];
-      t.ticket0 = tickets;
-      t.slot0 = (int)(words / TEAM_SLOT_WORDS);
-      t.e0 = (int)h->eoff[k];
-      t.e1 = (int)h->eoff[k + 1];
-      t.mean_row = (int)h->h_mean_row[k];
-      tickets += t.nwg;
-      words += team_words(t.nwg);
-      team.push_back(t);
-    }
+    if (widest > g) continue;
+    double end = 0.0;
+    std::vector<int> o = start_order(wide, us, g, end);
+    if (h->team_shape >= 0 && end >= best) continue;
     h->team_shape = s;
-    h->team = std::move(team);
-    h->team_inst = order;
-    h->team_words = words;
-    h->n_tickets = tickets;
-    h->team_grid = std::min(grid, tickets);
+    order = std::move(o);
+    best = end;
+    grid = g;
   }
   if (h->team_shape < 0) return CUP2D_PS_OK;
+  h->team.clear();
+  size_t words = 0;
+  int tickets = 0;
+  for (int k : order) {
+    TeamTask t{};
+    team_split((int)(h->boff[k + 1] - h->boff[k]), team_blocks(h->team_shape), t);
+    t.b0 = (int)h->boff[k];
+    t.ticket0 = tickets;
+    t.slot0 = (int)(words / TEAM_SLOT_WORDS);
+    t.e0 = (int)h->eoff[k];
+    t.e1 = (int)h->eoff[k + 1];
+    t.mean_row = (int)h->h_mean_row[k];
+    tickets += t.nwg;
+    words += team_words(t.nwg);
+    h->team.push_back(t);
+  }
+  h->team_inst = std::move(order);
+  h->team_words = words;
+  h->n_tickets = tickets;
+  h->team_grid = std::min(grid, tickets);
   int rc;
   if ((rc = bupload(h, h->allocs, &h->d_task, h->team)) ||
       (rc = balloc(h, h->allocs, &h->d_team, team_slots_at(K) + h->team_words * sizeof(unsigned long long))) ||

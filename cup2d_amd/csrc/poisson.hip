@@ -1891,13 +1891,13 @@ static int set_mesh_body(cup2d_ps *h, const cup2d_mesh_desc *m) {
 
 // The on-chip solve's team for the mesh: the fewest blocks per workgroup
 // whose workgroups all fit on the device at once -- an iteration of a uniform
-// mesh took 9.9 us with 16 blocks per workgroup, 10.9 with 32, 12.7 with 48 and
-// 13.8 with 64 on 1536 blocks, 14.5 / 15.0 / 15.5 with 32 / 48 / 64 on 8190, and
-// on a graded mesh of 8348 blocks 16.4 with 48 and 17.3 with 64 -- but 16 blocks
-// only up to 192 workgroups: on 3072 blocks 16 and 32 took 11.2 and 11.6, on
-// 4096 12.5 and 12.0, the larger team's sums taking longer than the shorter
-// product saves.
-constexpr int TEAM_16_MOST = 192;
+// mesh took 9.6 us with 16 blocks per workgroup, 10.2 with 32, 11.2 with 48 and
+// 12.2 with 64 on 1536 blocks, 12.5 / 12.7 / 13.5 with 32 / 48 / 64 on 6144, and
+// on a graded mesh of 8348 blocks 15.6 with 48 and 16.4 with 64 -- but 16 blocks
+// only up to 144 workgroups: on 2304 blocks 16 and 32 were alike (10.4), on 3072
+// 11.1 and 10.7, the larger team's sums taking longer than the shorter rows of
+// work save.
+constexpr int TEAM_16_MOST = 144;
 static void plan_team(cup2d_ps *h) {
   h->team_shape = -1;
   for (int s = 0; s < TEAM_SHAPES; s++) {
