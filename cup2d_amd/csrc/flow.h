@@ -50,7 +50,9 @@ struct FlowMesh {
 
 __device__ __forceinline__ double sqd(double x) { return x * x; }
 
-// advDiff.cpp:18-40 (pow(., 2) as a product)
+// advDiff.cpp:18-40 (pow(., 2) as a product).  The value for the other wind
+// (advDiff.cpp:42-62) is this one of the mirrored stencil: the same products,
+// the sums' operands exchanged, so the same in every bit.
 __device__ __forceinline__ double weno5_plus(double um2, double um1, double u, double up1, double up2) {
 #pragma clang fp contract(off)
   const double e = 1e-6;
@@ -67,28 +69,11 @@ __device__ __forceinline__ double weno5_plus(double um2, double um1, double u, d
   const double f3 = (1.0 / 3.0) * u + ((+5.0 / 6.0) * up1 - (1.0 / 6.0) * up2);
   return (w1 * f1 + w3 * f3) + w2 * f2;
 }
-// advDiff.cpp:42-62
-__device__ __forceinline__ double weno5_minus(double um2, double um1, double u, double up1, double up2) {
-#pragma clang fp contract(off)
-  const double e = 1e-6;
-  const double b1 = 13.0 / 12.0 * sqd((um2 + u) - 2 * um1) + 0.25 * sqd((um2 + 3 * u) - 4 * um1);
-  const double b2 = 13.0 / 12.0 * sqd((um1 + up1) - 2 * u) + 0.25 * sqd(um1 - up1);
-  const double b3 = 13.0 / 12.0 * sqd((u + up2) - 2 * up1) + 0.25 * sqd((3 * u + up2) - 4 * up1);
-  const double what1 = 0.3 / sqd(b1 + e);
-  const double what2 = 0.6 / sqd(b2 + e);
-  const double what3 = 0.1 / sqd(b3 + e);
-  const double aux = 1.0 / ((what1 + what3) + what2);
-  const double w1 = what1 * aux, w2 = what2 * aux, w3 = what3 * aux;
-  const double f1 = (1.0 / 3.0) * u + ((-1.0 / 6.0) * um2 + (5.0 / 6.0) * um1);
-  const double f2 = (5.0 / 6.0) * u + ((1.0 / 3.0) * um1 - (1.0 / 6.0) * up1);
-  const double f3 = (11.0 / 6.0) * u + ((-7.0 / 6.0) * up1 + (1.0 / 3.0) * up2);
-  return (w1 * f1 + w3 * f3) + w2 * f2;
-}
-// fp - fm, upwinded on the sign of U (advDiff.cpp:64-82)
-__device__ __forceinline__ double weno_diff(double U, const double (&s)[7]) {
-#pragma clang fp contract(off)
-  if (U > 0) return weno5_plus(s[1], s[2], s[3], s[4], s[5]) - weno5_plus(s[0], s[1], s[2], s[3], s[4]);
-  return weno5_minus(s[2], s[3], s[4], s[5], s[6]) - weno5_minus(s[1], s[2], s[3], s[4], s[5]);
+// The value at the face between the cells at o - st and o of a lab, upwinded for
+// a positive (plus) or another wind: one run of instructions for either.
+__device__ __forceinline__ double weno_face(const double *L, int o, int st, bool plus) {
+  const int a = plus ? o - 3 * st : o + 2 * st, k = plus ? st : -st;
+  return weno5_plus(L[a], L[a + k], L[a + 2 * k], L[a + 3 * k], L[a + 4 * k]);
 }
 
 // Value at the fine-frame point (X, Y) (fine units, the fine block's cell
@@ -163,12 +148,40 @@ __device__ __forceinline__ double ghost3(const FlowMesh &M, const double *__rest
   return 0.25 * ((fk[r0 * 8 + c0] + fk[r0 * 8 + c0 + 1]) + (fk[(r0 + 1) * 8 + c0] + fk[(r0 + 1) * 8 + c0 + 1]));
 }
 
-// tmp = the RHS of KernelAdvectDiffuse for every cell (u, v in; tu, tv out),
-// afac = -dt h, dfac = nu dt; the diffusive flux correction included.
-__global__ __launch_bounds__(WG) void kf_advdiff_rhs(FlowMesh M, const double *__restrict__ u,
-                                                     const double *__restrict__ v, double uinf_x,
-                                                     double uinf_y, double nu, double dt,
-                                                     double *__restrict__ tu, double *__restrict__ tv) {
+// Where ghost g of block b comes from at a wall or a same-level neighbour, and
+// its factors for the two velocity components (across a coarse-fine face: a
+// cell of the block, unused).
+__device__ __forceinline__ long ghost_cell(const int4 &n4, long b, int g, double &su, double &sv) {
+  const int fc = g / 24, d = (g % 24) / 8 + 1, t = g % 8;
+  const int nv = fc == 0 ? n4.x : fc == 1 ? n4.y : fc == 2 ? n4.z : n4.w;
+  su = nv == -1 && fc < 2 ? -1.0 : 1.0;
+  sv = nv == -1 && fc >= 2 ? -1.0 : 1.0;
+  const int k = nv >= 0 ? (fc & 1 ? d - 1 : BS - d) : fc & 1 ? BS - 1 : 0;  // along the face's normal
+  return (nv >= 0 ? (long)nv : b) * 64 + (fc < 2 ? t * 8 + k : k * 8 + t);
+}
+
+// One stage of advDiff::operator(): out = u0 + (t / 2) / h^2 (HALF: the first
+// stage) or u0 + t / h^2, t = the RHS of KernelAdvectDiffuse of (u, v) with
+// afac = -dt h, dfac = nu dt, the diffusive flux correction included.  u0 may be
+// out: a block's own values are read before they are written, and neighbours
+// are read of u and v alone.
+//
+// Bound by FP64 instructions: a WENO5 value is about 65 operations and 4
+// divisions.  A face's value serves the cells on both sides (fp - fm of
+// advDiff.cpp:64-82 is the value above minus the value below), so a lane forms
+// the four on its cell's low faces, for its own wind and, only where the lower
+// neighbour's has the other sign, for that one too; the low neighbour fetches
+// its value by a lane shuffle, and the 32 values on the block's high faces are
+// one more half-full pass: 4.5 values a cell instead of 8.  The stage's update is
+// done here.  The rare paths (coarse-fine ghosts, flux correction) are rolled
+// loops, so that 96 registers serve and five waves run on a SIMD (6 with spilled
+// ones were slower, 98 us).  1M cells, both stages and the call: 127 us as two
+// kernels a stage with 8 values a cell, 90 us so; 8348 graded blocks 90 and 71.
+template <bool HALF>
+__global__ __launch_bounds__(WG, 5) void kf_advdiff(FlowMesh M, const double *__restrict__ u,
+                                                 const double *__restrict__ v, double uinf_x, double uinf_y,
+                                                 double nu, double dt, const double *u0, const double *v0,
+                                                 double *uo, double *vo) {
 #pragma clang fp contract(off)
   __shared__ double lab[FWB][2][LW * LW];
   const int w = threadIdx.x >> 6, c = threadIdx.x & 63, ix = c & 7, iy = c >> 3;
@@ -177,15 +190,39 @@ __global__ __launch_bounds__(WG) void kf_advdiff_rhs(FlowMesh M, const double *_
     const bool ok = b < M.nb;
     double *LU = lab[w][0], *LV = lab[w][1];
     if (ok) {
-      LU[(LH + iy) * LW + LH + ix] = u[b * 64 + c];
-      LV[(LH + iy) * LW + LH + ix] = v[b * 64 + c];
-      for (int g = c; g < 96; g += 64) {
-        int gy, gx;
-        const double gu = ghost3(M, u, b, g, -1.0, 1.0, gy, gx);
-        const double gv = ghost3(M, v, b, g, 1.0, -1.0, gy, gx);
-        LU[gy * LW + gx] = gu;
-        LV[gy * LW + gx] = gv;
+      // every load is asked for before the first is awaited
+      const int4 n4 = M.nbr[b];
+      const double cu = u[b * 64 + c], cv = v[b * 64 + c];
+      double gu[2], gv[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int g = min(c + 64 * i, 95);
+        double su, sv;
+        const long src = ghost_cell(n4, b, g, su, sv);
+        gu[i] = su * u[src];
+        gv[i] = sv * v[src];
       }
+      LU[(LH + iy) * LW + LH + ix] = cu;
+      LV[(LH + iy) * LW + LH + ix] = cv;
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int g = c + 64 * i, fc = g / 24, d = (g % 24) / 8 + 1, t = g % 8;
+        const int n = fc & 1 ? LH + BS - 1 + d : LH - d;  // along the face's normal
+        if (g < 96) {
+          const int at = fc < 2 ? (LH + t) * LW + n : n * LW + LH + t;
+          LU[at] = gu[i];
+          LV[at] = gv[i];
+        }
+      }
+      if (n4.x == -2 || n4.y == -2 || n4.z == -2 || n4.w == -2)
+#pragma unroll 1
+        for (int k = 0; k < 4; k++) {
+          const int g = c + 64 * (k >> 1), fc = g / 24;
+          if (g >= 96 || (fc == 0 ? n4.x : fc == 1 ? n4.y : fc == 2 ? n4.z : n4.w) != -2) continue;
+          int gy, gx;
+          const double f = ghost3(M, k & 1 ? v : u, b, g, 1.0, 1.0, gy, gx);
+          (k & 1 ? LV : LU)[gy * LW + gx] = f;
+        }
     }
     __syncthreads();
     if (ok) {
@@ -193,19 +230,34 @@ __global__ __launch_bounds__(WG) void kf_advdiff_rhs(FlowMesh M, const double *_
       const double afac = -dt * h, dfac = nu * dt;
       const int o = (LH + iy) * LW + LH + ix;
       const double UU = LU[o] + uinf_x, VV = LV[o] + uinf_y;
-      double res[2];
-#pragma unroll
+      const double ih2 = 1.0 / (h * h);
+      double high = 0.0;  // lanes 8 (2 direction + component) + t: the value on the block's high face
+      if (c < 32) {
+        const int t = c & 7;
+        const bool xd = c < 16;
+        const int oh = xd ? (LH + t) * LW + LH + BS : (LH + BS) * LW + LH + t, st = xd ? 1 : LW;
+        const double wind = xd ? LU[oh - 1] + uinf_x : LV[oh - LW] + uinf_y;
+        high = weno_face(c & 8 ? LV : LU, oh, st, wind > 0);
+      }
+#pragma unroll 1
       for (int comp = 0; comp < 2; comp++) {
         const double *L = comp ? LV : LU;
-        double sx[7], sy[7];
-#pragma unroll
-        for (int k = 0; k < 7; k++) {
-          sx[k] = L[o + k - 3];
-          sy[k] = L[o + (k - 3) * LW];
+        double adv = 0.0;
+#pragma unroll 1
+        for (int dir = 0; dir < 2; dir++) {
+          const int st = dir ? LW : 1, at = dir ? iy : ix, t = dir ? ix : iy;
+          const double W = dir ? VV : UU;
+          const bool own = W > 0;
+          const bool low = at > 0 ? (dir ? LV[o - LW] + uinf_y : LU[o - 1] + uinf_x) > 0 : own;
+          const double fm = weno_face(L, o, st, own);
+          double fl = fm;
+          if (low != own) fl = weno_face(L, o, st, low);
+          const double next = __shfl(fl, (c + (dir ? BS : 1)) & 63), last = __shfl(high, 8 * (2 * dir + comp) + t);
+          const double a = W * ((at == BS - 1 ? last : next) - fm);
+          adv = dir ? adv + a : a;
         }
-        const double ddx = weno_diff(UU, sx), ddy = weno_diff(VV, sy);
-        const double lap = dfac * (((sx[4] + sx[2]) + (sy[4] + sy[2])) - 4 * sx[3]);
-        double t = afac * (UU * ddx + VV * ddy) + lap;
+        const double lap = dfac * (((L[o + 1] + L[o - 1]) + (L[o + LW] + L[o - LW])) - 4 * L[o]);
+        double t = afac * adv + lap;
         // diffusive flux correction on the faces with finer neighbours
         const int4 n4 = M.nbr[b];
 #pragma unroll 1
@@ -222,6 +274,7 @@ __global__ __launch_bounds__(WG) void kf_advdiff_rhs(FlowMesh M, const double *_
           const long fbk = tc >= BS / 2 ? fd.y : fd.x;
           const int t0 = (tc % (BS / 2)) * 2;
           const double *fld = comp ? v : u;
+#pragma unroll 1
           for (int hh = 0; hh < 2; hh++) {
             const int tf = t0 + hh;
             int fx, fy;
@@ -239,34 +292,11 @@ __global__ __launch_bounds__(WG) void kf_advdiff_rhs(FlowMesh M, const double *_
           }
           t = t + corr;
         }
-        res[comp] = t;
+        const double base = (comp ? v0 : u0)[b * 64 + c];
+        (comp ? vo : uo)[b * 64 + c] = base + (HALF ? 0.5 * t : t) * ih2;
       }
-      tu[b * 64 + c] = res[0];
-      tv[b * 64 + c] = res[1];
     }
     __syncthreads();  // the labs are refilled by the next pass
-  }
-}
-
-// out = base + (fac t) / h^2 (stage 1: fac = 0.5, (0.5 t) ih2; stage 2:
-// fac = 1, t ih2), for u and v.
-// (uo may be u0: each element is read before it is written)
-__global__ __launch_bounds__(WG) void kf_stage(FlowMesh M, const double *u0, const double *v0,
-                                               const double *__restrict__ tu,
-                                               const double *__restrict__ tv, int half, double *uo,
-                                               double *vo) {
-#pragma clang fp contract(off)
-  const long n = (long)M.nb * 64;
-  for (long i = (long)blockIdx.x * WG + threadIdx.x; i < n; i += (long)gridDim.x * WG) {
-    const double h = M.h[i >> 6];
-    const double ih2 = 1.0 / (h * h);
-    if (half) {
-      uo[i] = u0[i] + (0.5 * tu[i]) * ih2;
-      vo[i] = v0[i] + (0.5 * tv[i]) * ih2;
-    } else {
-      uo[i] = u0[i] + tu[i] * ih2;
-      vo[i] = v0[i] + tv[i] * ih2;
-    }
   }
 }
 
@@ -342,7 +372,7 @@ __global__ __launch_bounds__(WG) void kf_max_speed(long n, const double *__restr
 
 // score[b] = max over the block's cells of |omega|, omega = (0.5 / h)
 // ((u(x, y-1) - u(x, y+1)) + (v(x+1, y) - v(x-1, y))) (KernelVorticity,
-// Helpers.h:103-116, the velocity lab's ghosts as kf_advdiff_rhs); or 2 rtol
+// Helpers.h:103-116, the velocity lab's ghosts as kf_advdiff); or 2 rtol
 // when a cell of the block, or of its lab within `off` cells of it (2, 3 on
 // the finest level), has 0 < chi < 0.9 (GradChiOnTmp, AdaptTheMesh.cpp:
 // 11-71; chi clamped to [0, 1]; the lab is a cross, so the corner regions

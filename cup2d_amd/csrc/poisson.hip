@@ -2387,15 +2387,12 @@ static int advect_diffuse_body(cup2d_ps *h, double *d_u, double *d_v, double uin
   if (!(dt > 0) || !(nu >= 0)) return fail(h, CUP2D_PS_EINVAL, "dt must be positive and nu non-negative");
   HIPCHK(h, hipSetDevice(h->device));
   const FlowMesh M = flow_mesh(h);
-  // the solver's work vectors serve as the stage's work space: u1, v1 in
-  // p, nu; the right-hand sides in z1, z2
-  double *u1 = h->d_p, *v1 = h->d_nu, *tu = h->d_z1, *tv = h->d_z2;
-  const int Gf = flow_grid(h), Gc = cell_grid(h);
+  // the solver's work vectors p and nu hold the first stage
+  double *u1 = h->d_p, *v1 = h->d_nu;
+  const int G = flow_grid(h);
   hipStream_t s = h->stream;
-  kf_advdiff_rhs<<<Gf, WG, 0, s>>>(M, d_u, d_v, uinf_x, uinf_y, nu, dt, tu, tv);
-  kf_stage<<<Gc, WG, 0, s>>>(M, d_u, d_v, tu, tv, 1, u1, v1);
-  kf_advdiff_rhs<<<Gf, WG, 0, s>>>(M, u1, v1, uinf_x, uinf_y, nu, dt, tu, tv);
-  kf_stage<<<Gc, WG, 0, s>>>(M, d_u, d_v, tu, tv, 0, d_u, d_v);
+  kf_advdiff<true><<<G, WG, 0, s>>>(M, d_u, d_v, uinf_x, uinf_y, nu, dt, d_u, d_v, u1, v1);
+  kf_advdiff<false><<<G, WG, 0, s>>>(M, u1, v1, uinf_x, uinf_y, nu, dt, d_u, d_v, d_u, d_v);
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(s));
   return CUP2D_PS_OK;

@@ -49,6 +49,20 @@ def test_advect_diffuse_matches_oracle(name, on_device):
         assert np.array_equal(uo, ru) and np.array_equal(vo, rv), (name, uinf)
 
 
+@pytest.mark.parametrize("bx,by,px,py", [(1, 1, False, False), (1, 5, False, False), (3, 3, True, False), (5, 3, True, True)])
+def test_advect_diffuse_upwinds_every_face_by_its_cells(bx, by, px, py):
+    """Faces whose two cells have winds of either sign, or none at all (the sign test's other branch), on the
+    block's low and high sides."""
+    m = M.uniform(bx, by, 1.0, px, py)
+    rng = np.random.default_rng(bx * 10 + by)
+    u, v = (rng.integers(-1, 2, m.n) * rng.uniform(0.5, 1.5, m.n) for _ in range(2))
+    s = PS.Solver().set_mesh(m, on_device=True)
+    for uinf in ((0.0, 0.0), (1.0, -1.0)):
+        uo, vo = s.advect_diffuse(u, v, uinf, 1e-3, 1e-3)
+        ru, rv = FL.advect_diffuse(m, u, v, uinf, 1e-3, 1e-3)
+        assert np.array_equal(uo, ru) and np.array_equal(vo, rv)
+
+
 def test_penalize_chi_and_max_speed_match_oracle():
     m = W.cylinder_mesh(levels=3, target=300)
     s = PS.Solver().set_mesh(m)
