@@ -146,15 +146,16 @@ def adapt(mesh: Mesh, tags):
     lev, bx, by = (np.ascontiguousarray(a, dtype=np.int32) for a in (mesh.level, mesh.bx, mesh.by))
     args = (mesh.bpdx, mesh.bpdy, mesh.levels, int(mesh.periodic_x), int(mesh.periodic_y), mesh.n_blocks,
             lev.ctypes.data, bx.ctypes.data, by.ctypes.data, t.ctypes.data)
-    nb = lib.cup2d_mesh_adapt(*args, None, None, None, None, None, 0)
-    if nb < 0:
-        raise ValueError(lib.cup2d_mesh_last_error().decode())
-    nl, nx, ny = (np.empty(nb, np.int32) for _ in range(3))
-    kind = np.empty(nb, np.int32)
-    src = np.empty((nb, 4), np.int64)
-    nb2 = lib.cup2d_mesh_adapt(*args, nl.ctypes.data, nx.ctypes.data, ny.ctypes.data, kind.ctypes.data,
-                               src.ctypes.data, nb)
-    if nb2 != nb:
-        raise ValueError(lib.cup2d_mesh_last_error().decode())
+    cap = mesh.n_blocks + 6 * int((t > 0).sum()) + 64  # more where the balance splits many others: then once again
+    while True:
+        nl, nx, ny, kind = (np.empty(cap, np.int32) for _ in range(4))
+        src = np.empty((cap, 4), np.int64)
+        nb = lib.cup2d_mesh_adapt(*args, *(a.ctypes.data for a in (nl, nx, ny, kind, src)), cap)
+        if nb < 0:
+            raise ValueError(lib.cup2d_mesh_last_error().decode())
+        if nb <= cap:
+            break
+        cap = nb
+    nl, nx, ny, kind, src = (a[:nb] for a in (nl, nx, ny, kind, src))
     m = Mesh(mesh.bpdx, mesh.bpdy, mesh.levels, mesh.extent, nl, nx, ny, mesh.periodic_x, mesh.periodic_y)
     return m, kind, src

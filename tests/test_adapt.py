@@ -154,3 +154,81 @@ def test_adapt_rejects_bad_input():
     m2, kind, src = M.adapt(m, np.ones(m.n_blocks, np.int8))
     assert m2.n_blocks == m.n_blocks and (kind == 0).all()
     assert np.array_equal(src[:, 0], np.arange(m.n_blocks)) and (src[:, 1:] == -1).all()
+
+
+def _adapt_restated(m, tags):
+    """The rules of cup2d_mesh_adapt with sets of (level, x, y)."""
+    old = {k: b for b, k in enumerate(zip(m.level.tolist(), m.bx.tolist(), m.by.tolist()))}
+    leaves = set(old)
+
+    def split(k):
+        leaves.remove(k)
+        leaves.update((k[0] + 1, 2 * k[1] + q % 2, 2 * k[2] + q // 2) for q in range(4))
+
+    def covering(l, i, j):
+        return next((mm for mm in range(l, -1, -1) if (mm, i >> (l - mm), j >> (l - mm)) in leaves), -1)
+
+    def around(l, i, j):
+        nx, ny = m.bpdx << l, m.bpdy << l
+        for dj in (-1, 0, 1):
+            for di in (-1, 0, 1):
+                ni, nj = i + di, j + dj
+                if (di or dj) and (m.periodic_x or 0 <= ni < nx) and (m.periodic_y or 0 <= nj < ny):
+                    yield ni % nx, nj % ny
+
+    def balance():
+        while True:
+            for l, i, j in sorted(leaves):
+                far = [(covering(l - 1, ni >> 1, nj >> 1), ni, nj) for ni, nj in around(l, i, j)] if l > 1 else []
+                far = [(c, ni >> (l - c), nj >> (l - c)) for c, ni, nj in far if 0 <= c < l - 1]
+                if far:
+                    split(far[0])
+                    break
+            else:
+                return
+
+    for k, b in old.items():
+        if tags[b] > 0 and k[0] + 1 < m.levels:
+            split(k)
+    balance()
+    parents = {(l - 1, i >> 1, j >> 1) for (l, i, j), b in old.items() if tags[b] < 0 and l > 0}
+    for l, i, j in sorted(parents):
+        kids = [(l + 1, 2 * i + q % 2, 2 * j + q // 2) for q in range(4)]
+        if not all(k in leaves and k in old and tags[old[k]] < 0 for k in kids):
+            continue
+        if all(covering(l, ni, nj) >= 0 or all((l + 1, 2 * ni + q % 2, 2 * nj + q // 2) in leaves for q in range(4))
+               for ni, nj in around(l, i, j)):
+            leaves.difference_update(kids)
+            leaves.add((l, i, j))
+    balance()
+    plan = {}
+    for l, i, j in leaves:
+        up = [(mm, i >> (l - mm), j >> (l - mm)) for mm in range(l - 1, -1, -1)]
+        up = [k for k in up if k in old]
+        if (l, i, j) in old:
+            plan[l, i, j] = (0, old[l, i, j], -1, -1, -1)
+        elif up:
+            plan[l, i, j] = (1, old[up[0]], -1, -1, -1)
+        else:
+            plan[l, i, j] = (2, *(old[l + 1, 2 * i + q % 2, 2 * j + q // 2] for q in range(4)))
+    return plan
+
+
+@pytest.mark.parametrize("seed", range(12))
+def test_adapt_matches_its_rules(seed):
+    """Grids of every boundary, and meshes that come unbalanced, in any block order."""
+    rng = np.random.default_rng(seed)
+    bx, by, levels, px, py = 1 + seed % 3, 1 + seed // 4, 2 + seed % 4, bool(seed & 1), bool(seed & 2)
+    blocks = [(0, i, j) for j in range(by) for i in range(bx)]
+    for l in range(levels - 1):  # one block split at every level, its neighbours left alone
+        k = [b for b in blocks if b[0] == l][rng.integers(-2, 0) if l else -1]
+        blocks.remove(k)
+        blocks += [(l + 1, 2 * k[1] + q % 2, 2 * k[2] + q // 2) for q in range(4)]
+    m = M.from_blocks(bx, by, levels, 1.0, [blocks[k] for k in rng.permutation(len(blocks))], px, py)
+    for p in ((0.2, 0.5, 0.3), (0.8, 0.1, 0.1), (1.0, 0.0, 0.0), (0.0, 0.0, 1.0), (0.9, 0.1, 0.0)):
+        tags = rng.choice([-1, 0, 1], size=m.n_blocks, p=p)
+        plan = _adapt_restated(m, tags)
+        m2, kind, src = M.adapt(m, tags)
+        got = {(int(l), int(i), int(j)): (int(k), *map(int, s)) for l, i, j, k, s in zip(m2.level, m2.bx, m2.by, kind, src)}
+        assert got == plan and m2.n_blocks == len(plan)
+        m = m2
