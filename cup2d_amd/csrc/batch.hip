@@ -9,8 +9,8 @@
 // team of workgroups (team.hip), all in one launch: an iteration touches memory
 // for its halo and its sums only, and an instance ends when it converges, its
 // workgroups taking the next.  64 instances of 512-8,192 blocks (13.9 million
-// cells) to 1e-12: 298 ms, by the item kernels 915 ms; 9 small ones in mixed
-// precision 22 ms against 53.4 ms.  What bounds it: the workgroups' own work and
+// cells) to 1e-12: 290 ms, by the item kernels 915 ms; 9 small ones in mixed
+// precision 13 ms against 53.4 ms.  What bounds it: the workgroups' own work and
 // the waits of a team (15 us an iteration on 64 blocks; 3,389 workgroups' worth
 // of instances on 256).
 //
@@ -2087,7 +2087,7 @@ static std::vector<int> start_order(const std::vector<int> &n, const std::vector
 // 7.9 us on 16 workgroups, 9.1 on 64; 32 blocks 9.1 on 16, 10.9 on 128; 48 blocks
 // 11.2 on 32, 14.0 on 171; 64 blocks 11.8 on 16, 14.1 on 128).  Few instances run
 // at once on small shares, many on 64 blocks, which keep the most of them
-// running: the 64-instance batch took 298 ms, with 48 blocks 384, with 32 502.
+// running: the 64-instance batch took 290 ms, with 48 blocks 380, with 32 500.
 constexpr double TEAM_US[TEAM_SHAPES] = {8.2, 8.9, 10.3, 11.3}, TEAM_US_WG = 0.025;
 static int plan_teams(cup2d_psb *h) {
   h->team_shape = -1;

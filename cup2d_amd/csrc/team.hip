@@ -27,8 +27,8 @@
 //
 // Measured (us per iteration to a relative residual of 1e-12, against five
 // kernels per iteration replayed from a graph): 128 blocks 7.7 against 24.0,
-// 1448 blocks 10.8 against 27.9, 8348 blocks 15.5 against 49.9, 16,229 blocks
-// 19.4 against 64.8.  One workgroup of 64 blocks alone takes 7.4 us, of 16 4.3 us:
+// 1448 blocks 10.5 against 27.9, 8348 blocks 15.4 against 49.9, 16,229 blocks
+// 18.8 against 64.8.  One workgroup of 64 blocks alone takes 7.4 us, of 16 4.3 us:
 // the rest is the waits and the slowest of the workgroups.
 //
 // Teams form by tickets: a workgroup takes the next ticket, which names its
@@ -116,7 +116,7 @@ __device__ __forceinline__ double dpp_total(double v) {
 constexpr u64 EMPTY = 0x7ff4c2d0a11c0de5ull;
 
 constexpr int face_rows(int blocks) { return blocks * 28; }  // a block has 28 cells on its faces
-constexpr int ENT = 14;                                      // entries of an explicit row kept in LDS (13 occur)
+constexpr int ENT = 14, HALF = ENT / 2;                      // entries of an explicit row kept in LDS (13 occur)
 constexpr int TAB = 256;                                     // coefficients kept in LDS
 
 template <int WGS, int T>
@@ -124,7 +124,11 @@ struct Shared {
   static constexpr int BPW = WGS / 256 * T * TILE, NW = WGS / 64;
   static constexpr int GHOST0 = BPW * ZS, GHOSTS = BPW * 40;  // first, most cells of other workgroups
   static constexpr int ITEMS = BPW * 12;                      // a block's 4 faces and 8 rows
-  static constexpr int ROWS = BPW == 64 ? 512 : BPW == 48 ? 768 : face_rows(BPW);  // explicit rows kept in LDS
+  // Explicit rows kept in LDS, and those of more than HALF entries among them
+  // (a third of the rows; 300-625 and 100-280 occur on 64 blocks of small graded
+  // meshes, a row beyond them is read from memory: 9 such meshes took 19.7 ms
+  // when 512 rows were kept, 14.5 so, 32 of 400-1,600 blocks 29.2 and 17.4).
+  static constexpr int ROWS = BPW == 64 ? 704 : BPW == 48 ? 768 : face_rows(BPW), WIDE = BPW == 64 ? 288 : ROWS;
   double z[GHOST0 + GHOSTS];        // the workgroup's blocks (product inputs, then z), then the ghosts
   double part[GHOST0];              // P v of the blocks, by class
   double ye[face_rows(BPW)];        // A z of the explicit rows
@@ -135,14 +139,15 @@ struct Shared {
   int4 face[BPW];                   // where z across each face lies (Xm, Xp, Ym, Yp); the block's own cells
                                     // where no plain neighbour does (a wall's term vanishes)
   int ghost[GHOSTS];                // where in the halo buffer each ghost comes
-  unsigned ent[ENT][ROWS];          // entries of the explicit rows: LDS index, coefficient << 16
-  int erow[face_rows(BPW)];         // ELL slot of each explicit row
+  unsigned ent[HALF][ROWS];         // entries of the explicit rows: LDS index, coefficient << 16
+  unsigned wide[HALF][WIDE];        // those from HALF on
+  int erow[face_rows(BPW)];         // place in `wide` of each explicit row in LDS, ELL slot of the others
   int eoff[BPW + 1];                // first explicit row of each block
   unsigned char ewid[face_rows(BPW)];  // entries, | 64 with ghosts among them, | 192 read from memory
   int2 item[ITEMS];                 // what other workgroups read, 8 cells each: {first LDS index | stride 8 (bit
                                     // 16), place in the halo buffer}
   u64 tick, phase[TEAM_PHASES];     // of the profile: not in registers, which the loop needs
-  int ng, ni, nf, ticket, bad;      // ghosts, items, explicit rows with ghosts
+  int ng, ni, nf, nw, ticket, bad;  // ghosts, items, explicit rows with ghosts, wide ones
 };
 
 // The running workgroup: what its functions share.
@@ -384,13 +389,15 @@ struct Ctx {
       if ((how & 64) != kind) continue;
       double sum = 0.0;
       if (how < 128) {
-        for (int w0 = 0; w0 < width; w0 += ENT / 2) {
-          unsigned en[ENT / 2];
+        auto add = [&](const unsigned *from, int stride) __attribute__((always_inline)) {
+          unsigned en[HALF];
 #pragma unroll
-          for (int i = 0; i < ENT / 2; i++) en[i] = s.ent[w0 + i][k];
+          for (int i = 0; i < HALF; i++) en[i] = from[i * stride];
 #pragma unroll
-          for (int i = 0; i < ENT / 2; i++) sum += s.tab[en[i] >> 16] * s.z[en[i] & 0xffffu];
-        }
+          for (int i = 0; i < HALF; i++) sum += s.tab[en[i] >> 16] * s.z[en[i] & 0xffffu];
+        };
+        add(s.ent[0] + k, S::ROWS);
+        if (width > HALF) add(s.wide[0] + s.erow[k], S::WIDE);
       } else {
         const int e = s.erow[k];
         for (int i = 0; i < width; i++) {
@@ -477,7 +484,7 @@ struct Ctx {
 
   // Headers, ghosts and explicit rows of the workgroup's blocks.
   __device__ __forceinline__ void lay_out() {
-    if (tid == 0) s.ng = s.ni = s.nf = 0;
+    if (tid == 0) s.ng = s.ni = s.nf = s.nw = 0;
     __syncthreads();
     // LDS index of 8 cells of another workgroup, from `first` of the halo buffer on
     auto ghosts = [&](int first) -> int {
@@ -536,8 +543,7 @@ struct Ctx {
       const int row = a.A.erow[e], l = (row >> 6) - b0;
       if (l < 0 || l >= nb) continue;
       const int k = s.eoff[l] + __popcll(s.mask[l] & ((1ull << (row & 63)) - 1));
-      s.erow[k] = e;
-      int width = 0;
+      int width = 0, slot = 0;
       bool fits = k < S::ROWS && a.A.ell_w <= ENT, far = false;
 #pragma unroll 1
       for (int i = 0; i < a.A.ell_w; i++) {
@@ -546,8 +552,12 @@ struct Ctx {
         if (code) width = i + 1;
         fits = fits && code < TAB;
       }
+      if (fits && width > HALF) {
+        slot = atomicAdd(&s.nw, 1);
+        fits = slot < S::WIDE;
+      }
 #pragma unroll 1
-      for (int i = 0; i < ENT && fits; i++) {  // entries past the row's end: 0.0 times its own value
+      for (int i = 0; i < (width > HALF ? ENT : HALF) && fits; i++) {  // entries past the row's end: 0.0 times its own value
         const long at = (long)i * a.A.n_exc + e;
         const unsigned code = i < width ? a.A.ecode[at] : 0;
         const int col = i < width ? a.A.ecol[at] : row, lc = (col >> 6) - b0;
@@ -561,8 +571,9 @@ struct Ctx {
           if (fits) s.ghost[g] = place_of(row >> 6, col);
           idx = S::GHOST0 + g;
         }
-        if (fits) s.ent[i][k] = idx | code << 16;
+        if (fits) (i < HALF ? s.ent[i][k] : s.wide[i - HALF][slot]) = idx | code << 16;
       }
+      s.erow[k] = fits ? slot : e;
       if (far || !fits) atomicAdd(&s.nf, 1);
       s.ewid[k] = (unsigned char)(fits ? (far ? 64 : 0) + width : 192 + width);
     }
