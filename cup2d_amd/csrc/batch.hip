@@ -14,8 +14,8 @@
 // the waits of a team (15 us an iteration on 64 blocks; 3,389 workgroups' worth
 // of instances on 256).
 //
-// A batch with a larger instance takes the item kernels, which advance all
-// unfinished instances at once:
+// A batch with a larger instance, or in the mean-row form, takes the item
+// kernels, which advance all unfinished instances at once:
 //
 //  * work units: "items" (a run of up to `ib` blocks of one instance) for the
 //    SpMV and vector kernels, a workgroup per item; "tiles" (16 blocks of one
@@ -1655,7 +1655,7 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   a.n_tasks = K;
   a.n_tickets = h->n_tickets;
   a.start = h->mixed ? TEAM_ACCEPTS : TEAM_CHECKED;
-  a.mean_rows = h->cfg.mean_constraint != 0;
+  a.mean_rows = 0;
   a.norm_max = h->cfg.norm == CUP2D_PS_NORM_INF;
   a.form_polls = TEAM_POLLS << 5;  // a team forms when earlier tasks end
   a.st = h->d_st;
@@ -2094,7 +2094,10 @@ static int plan_teams(cup2d_psb *h) {
   const int K = h->K;
   long long most = 0;
   for (int k = 0; k < K; k++) most = std::max(most, h->boff[k + 1] - h->boff[k]);
-  if (most > TEAM_MAX_BLOCKS) return CUP2D_PS_OK;
+  // The mean-row form takes the item kernels: its runs are long, chaotic and full
+  // of restarts, and on chip one of 64 claimed convergence with a recurrence's
+  // residual 6x below the true one (theirs: within 1.1x).
+  if (most > TEAM_MAX_BLOCKS || h->cfg.mean_constraint) return CUP2D_PS_OK;
   std::vector<int> order;
   double best = 0.0;
   int grid = 0;
