@@ -830,6 +830,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           c.template exchange<KIND == PLAIN ? 2 : KIND == NORM_MAX ? 3 : 4, KIND == NORM_MAX>(v, TEAM_POLLS);
         }
         if (c.dead) break;
+        lap(3);
         if constexpr (KIND == MEAN_ROW) {
           if (mr) by_row = tot(3) * tot(2);
           put_mean_row();
@@ -855,7 +856,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           nu[tt][k] = y[tt][k];
         }
         c.clear();
-        lap(3);
+        lap(2);
         // t = A P s and omega
         c.place();
         CELLS z[tt][k] = r[tt][k];
@@ -879,6 +880,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           c.template exchange<4, false>(v, TEAM_POLLS);
         }
         if (c.dead) break;
+        lap(3);
         double ts = tot(0), tq = tot(1);
         if constexpr (KIND == MEAN_ROW) {
           if (mr) {
@@ -905,6 +907,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           c.place();
           c.template exchange<3, true>(f, TEAM_POLLS);
           if (c.dead) break;
+          lap(3);
           beta = uni((tot(1) / (rho + eps)) * aow);
           rho = tot(1);
           judge(tot(0), tot(l2 ? 0 : 2));
@@ -925,7 +928,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           c.clear();
         }
         CELLS p[tt][k] = r[tt][k] + beta * (p[tt][k] - omega * nu[tt][k]);
-        lap(3);
+        lap(2);
       }
       if (c.dead || done) break;
     }
