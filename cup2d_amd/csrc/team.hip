@@ -716,7 +716,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
     // The state at the top of an iteration (kernels.h evaluate: the same
     // rules, without the projection and the stall window); rho and beta are
     // the new ones.
-    auto judge = [&](double rr, double size) __attribute__((always_inline)) {
+    auto assess = [&](double rr, double size) __attribute__((always_inline)) {
       iter++;
       improved = size < size_opt;
       restart = replace = false;
@@ -805,10 +805,10 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
       lap(4);
       if (done) break;
       beta = 0.0;
-      bool pending = false;  // the last iteration's r is yet to be judged
+      bool pending = false;  // the last iteration's r is yet to be assessed
       for (;;) {
         // nu = A P p and alpha.  The size of r, by which the iteration before
-        // is judged, is summed with (rhat, nu), one exchange an iteration
+        // is assessed, is summed with (rhat, nu), one exchange an iteration
         // less; the mean row's own sums take its place there.
         c.place();
         CELLS z[tt][k] = p[tt][k];
@@ -835,7 +835,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           if (mr) by_row = tot(3) * tot(2);
           put_mean_row();
         } else if (pending) {
-          judge(tot(1), tot(l2 ? 1 : 2));
+          assess(tot(1), tot(l2 ? 1 : 2));
           if (__builtin_expect(done || replace || restart, 0)) {  // nothing of this pass is kept
             c.clear();
             if (!restart) {
@@ -910,7 +910,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           lap(3);
           beta = uni((tot(1) / (rho + eps)) * aow);
           rho = tot(1);
-          judge(tot(0), tot(l2 ? 0 : 2));
+          assess(tot(0), tot(l2 ? 0 : 2));
           c.clear();
           if (improved && !done && !replace) keep();
           if (!improved && (done || replace)) recall();

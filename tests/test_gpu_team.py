@@ -76,7 +76,7 @@ def test_block_orders_and_coarse_fine_rows(oracle, name, mc):
 @pytest.mark.parametrize("max_iter,breakdown_tol,max_restarts", [(1, 1e-14, 100), (2, 1e-14, 100), (3, 1e-14, 100),
                                                                  (12, 0.3, 100), (12, 0.3, 3), (12, 0.9, 100)])
 def test_last_iterations_and_restarts(norm, mc, max_iter, breakdown_tol, max_restarts):
-    """An iteration is judged when the next one's first sums arrive: the last one, and those that restart (a large
+    """An iteration is assessed when the next one's first sums arrive: the last one, and those that restart (a large
     breakdown tolerance: nearly all), end as the one-operation-per-launch solver's do."""
     m = W.graded_disk_mesh()
     b = W.vortex_rhs(m, 3)
