@@ -1298,9 +1298,10 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   HIPCHK(h, hipStreamSynchronize(h->stream));
   if (ctl[1]) return CUP2D_PS_OK;
   done = true;
-  HIPCHK(h, hipMemcpyAsync(d_out, h->d_x, h->op.n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
   const Scal &f = h->h_s[0];
+  // a refused solve leaves d_out as it was: nothing is queued that writes it
   if (h->mixed && f.err0 != f.err0) return fail(h, CUP2D_PS_EINVAL, "non-finite residual (NaN/Inf in b or x0)");
+  HIPCHK(h, hipMemcpyAsync(d_out, h->d_x, h->op.n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
   if (h->cfg.profile) {
     const auto *ph = reinterpret_cast<const unsigned long long *>(reinterpret_cast<unsigned char *>(ctl) + TEAM_PHASE_AT);
     for (int k = 0; k < TEAM_PHASES; k++) h->pms[k] += (double)ph[k] * TEAM_TICK_MS;
