@@ -38,13 +38,25 @@ __host__ __device__ constexpr int team_copies(int nwg) { return nwg <= 64 ? 1 : 
 // Exchange words of a team.
 constexpr size_t team_words(int nwg) { return (size_t)nwg * TEAM_SLOT_WORDS * team_copies(nwg); }
 
+// Places (words) in a task's part of a halo buffer, block b counted from the
+// task's first: the faces of every block (8 cells each, Xm, Xp, Ym, Yp), then
+// every block whole; 64 bytes that one workgroup writes and another reads lie
+// together.  Counted over a whole batch they would leave 32 bits from 22 million
+// blocks (of 33) on.
+constexpr int HALO_BLOCK = 96;
+__host__ __device__ constexpr int halo_face(int b, int f) { return 32 * b + 8 * f; }
+__host__ __device__ constexpr int halo_cell(int nb, int b) { return 32 * nb + 64 * b; }
+static_assert(halo_cell(TEAM_MAX_BLOCKS, TEAM_MAX_BLOCKS - 1) + 63 == (long long)HALO_BLOCK * TEAM_MAX_BLOCKS - 1 &&
+                  halo_face(TEAM_MAX_BLOCKS - 1, 3) + 7 == halo_cell(TEAM_MAX_BLOCKS, 0) - 1,
+              "places of the largest task");
+
 struct TeamArgs {
   OpView A;
   const int2 *fid;
   const double *pc;                     // FP64 MFMA fragments of P_inv's classes
   const double *b, *x0;
   double *out;
-  double *halo;                         // [3 n] what the workgroups read of each other
+  double *halo;                         // [3 n] what the workgroups read of each other (two buffers)
   double *xopt;                         // [n] work vector
   int n_codes;                          // entries of A.etab
   const TeamTask *task;                 // [n_tasks], or null: the one task `one`

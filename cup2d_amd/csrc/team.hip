@@ -145,7 +145,7 @@ struct Shared {
   int eoff[BPW + 1];                // first explicit row of each block
   unsigned char ewid[face_rows(BPW)];  // entries, | 64 with ghosts among them, | 192 read from memory
   int2 item[ITEMS];                 // what other workgroups read, 8 cells each: {first LDS index | stride 8 (bit
-                                    // 16), place in the halo buffer}
+                                    // 16), place in the halo buffer / 8}
   u64 tick, phase[TEAM_PHASES];     // of the profile: not in registers, which the loop needs
   int ng, ni, nf, nw, ticket, bad;  // ghosts, items, explicit rows with ghosts, wide ones
 };
@@ -160,6 +160,7 @@ struct Ctx {
   TeamTask t;
   int rank, b0, nb;                 // first block, blocks
   u64 *slots;
+  double *halo0;                    // the task's part of the halo buffer
   int copies, copy, slab;           // copies of the exchange words, the one read here, words of a copy
   unsigned ep, zp;                  // number of the exchange, parity of z's buffer
   int ni8, ng, nf;                  // words that others read, ghosts, explicit rows with ghosts
@@ -187,10 +188,8 @@ struct Ctx {
   __device__ __forceinline__ int lb(int tt) const { return (grp * T + tt) * TILE + j; }
   __device__ __forceinline__ bool ok(int tt) const { return lb(tt) < nb; }
   __device__ __forceinline__ long cell(int tt) const { return (long)(b0 + (ok(tt) ? lb(tt) : 0)) * 64 + c0; }
-  // the halo buffer of this z: the faces of every block (8 cells each, Xm, Xp,
-  // Ym, Yp), then every block whole; 64 bytes that one workgroup writes and
-  // another reads lie together
-  __device__ __forceinline__ double *halo() const { return a.halo + (zp ? 96l * a.A.nb : 0); }
+  // the task's halo buffer of this z (halo_face, halo_cell)
+  __device__ __forceinline__ double *halo() const { return halo0 + (zp ? (long)HALO_BLOCK * a.A.nb : 0); }
 
   // every 1024 polls: whether to give up (the launch failed, or the limit)
   __device__ __forceinline__ bool give_up(int &n, int limit) {
@@ -475,11 +474,11 @@ struct Ctx {
   __device__ __forceinline__ int place_of(int b, int col) const {
     const int4 n4 = a.A.nbr[b];
     const int blk = col >> 6, ix = col & 7, iy = (col >> 3) & 7;
-    if (n4.x == blk && ix == 7) return (4 * blk + 1) * 8 + iy;
-    if (n4.y == blk && ix == 0) return (4 * blk + 0) * 8 + iy;
-    if (n4.z == blk && iy == 7) return (4 * blk + 3) * 8 + ix;
-    if (n4.w == blk && iy == 0) return (4 * blk + 2) * 8 + ix;
-    return 32 * a.A.nb + col;
+    if (n4.x == blk && ix == 7) return halo_face(blk - t.b0, 1) + iy;
+    if (n4.y == blk && ix == 0) return halo_face(blk - t.b0, 0) + iy;
+    if (n4.z == blk && iy == 7) return halo_face(blk - t.b0, 3) + ix;
+    if (n4.w == blk && iy == 0) return halo_face(blk - t.b0, 2) + ix;
+    return halo_cell(t.nb, blk - t.b0) + (col & 63);
   }
 
   // Headers, ghosts and explicit rows of the workgroup's blocks.
@@ -503,7 +502,7 @@ struct Ctx {
       int at[4];
       bool whole = false;
       auto offer = [&](int base, bool column, int to) {
-        s.item[atomicAdd(&s.ni, 1)] = make_int2(l * ZS + base | (column ? 1 << 16 : 0), to);
+        s.item[atomicAdd(&s.ni, 1)] = make_int2(l * ZS + base | (column ? 1 << 16 : 0), to / 8);
       };
 #pragma unroll 1
       for (int f = 0; f < 4; f++) {
@@ -514,8 +513,8 @@ struct Ctx {
           if (nv >= b0 && nv < b0 + nb) {
             at[f] = (nv - b0) * ZS + (f == 0 ? 7 : f == 2 ? 56 : 0);  // the neighbour's facing row
           } else {
-            at[f] = ghosts((4 * nv + (f ^ 1)) * 8);
-            offer(f == 1 ? 7 : f == 3 ? 56 : 0, f < 2, 4 * b + f);
+            at[f] = ghosts(halo_face(nv - t.b0, f ^ 1));
+            offer(f == 1 ? 7 : f == 3 ? 56 : 0, f < 2, halo_face(b - t.b0, f));
           }
         } else if (nv == -2) {
           const int2 fd = a.fid[4 * (long)b + f];
@@ -525,7 +524,7 @@ struct Ctx {
       }
       if (whole)
 #pragma unroll 1
-        for (int i = 0; i < 8; i++) offer(8 * i, false, 4 * a.A.nb + 8 * b + i);
+        for (int i = 0; i < 8; i++) offer(8 * i, false, halo_cell(t.nb, b - t.b0) + 8 * i);
       s.face[l] = make_int4(at[0], at[1], at[2], at[3]);
     }
     __syncthreads();
@@ -637,6 +636,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
     c.b0 = t.b0 + c.rank * t.bpw;
     c.nb = min(t.bpw, t.nb - c.rank * t.bpw);
     c.slots = a.slots + (size_t)t.slot0 * TEAM_SLOT_WORDS;
+    c.halo0 = a.halo + (long)HALO_BLOCK * t.b0;
     c.copies = team_copies(t.nwg);
     c.copy = c.rank % c.copies;
     c.slab = 2 * TEAM_NQ * t.nwg;
