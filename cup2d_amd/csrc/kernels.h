@@ -354,6 +354,16 @@ __device__ __forceinline__ void tile_put(double (*tile)[TROW], int w, int lane, 
   for (int k = 0; k < 4; k++) tile[j][c0 + k] = ok ? v[k] : 0.0;
 }
 
+// Called on the results of FP64 matrix products before anything reads them.
+// v_mfma_f64_16x16x4 takes twice the cycles on gfx950 that it takes on gfx942.
+// Between it and a vector instruction that reads the result the compiler puts 19
+// wait states accordingly (11 on gfx942), but before an LDS or memory store of it
+// 18, as on gfx942: one fewer than the result takes.  (A first form of the on-chip
+// solve's product was seen to return an old high half of its first value.)  24
+// states here, of the at least 1024 cycles of a 64 x 64 product.
+__device__ __forceinline__ void settle(f64x4 &a) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(a)); }
+__device__ __forceinline__ void settle(f64x4 &a, f64x4 &b) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(a), "+v"(b)); }
+
 // z (the thread's four output cells) = rows 16 w + 4 q + v of P times block
 // j of the tile, after a workgroup barrier that published the tile
 __device__ __forceinline__ f64x4 tile_prec64(const double (*tile)[TROW], const PFrag64 &F,
@@ -365,6 +375,7 @@ __device__ __forceinline__ f64x4 tile_prec64(const double (*tile)[TROW], const P
   f64x4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int ks = 0; ks < 16; ks++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(F.a[ks], in[ks], acc, 0, 0, 0);
+  settle(acc);
   return acc;
 }
 __device__ __forceinline__ void st4(double *__restrict__ a, long i, const f64x4 &v) {

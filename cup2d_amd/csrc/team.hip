@@ -345,12 +345,8 @@ struct Ctx {
 #pragma unroll
       for (int k = 0; k < 4; k++) acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(F[k], in[k], acc[tt], 0, 0, 0);
     }
-    // The product's results are read 20 and more cycles after the last
-    // instruction: said here, because the compiler's own count once let the
-    // high half of the first result be read early (the product was kept in
-    // accumulation registers then).
-    if constexpr (T == 1) asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]));
-    else asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[T - 1]));
+    if constexpr (T == 1) settle(acc[0]);
+    else settle(acc[0], acc[T - 1]);
 #pragma unroll
     for (int tt = 0; tt < T; tt++) {
       double2 *d = reinterpret_cast<double2 *>(s.part + lb(tt) * ZS + c0);
