@@ -1,4 +1,4 @@
-"""ctypes binding of libcup2d_poisson.so (include/cup2d_poisson.h).
+"""ctypes binding of libcup2d_poisson.so (include/cup2d_poisson.h, include/cup2d_chip.h).
 
 Loading fails loudly when the library has not been built: the solver has no
 fallback path.
@@ -100,6 +100,14 @@ SIGNATURES = {
     "cup2d_psb_last_error": (ctypes.c_char_p, [_P]),
 }
 
+# ... and of include/cup2d_chip.h
+CHIP_SIGNATURES = {
+    "cup2d_ps_set_on_chip": (_I, [_P, _I, _I]),
+    "cup2d_ps_on_chip": (_I, [_P]),
+    "cup2d_psb_set_on_chip": (_I, [_P, _I, _I]),
+    "cup2d_psb_on_chip": (_I, [_P]),
+}
+
 _lib = None
 
 
@@ -110,7 +118,7 @@ def load():
             raise RuntimeError(f"{LIB_PATH} is missing: build it with __graft_entry__.build() "
                                "(the Poisson solver has no non-HIP fallback)")
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **CHIP_SIGNATURES}.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args

@@ -1180,6 +1180,7 @@ struct cup2d_psb {
   // too large for it), the instances' teams in launch order, device words
   int team_shape = -1;
   bool team_failed = false;
+  TeamUse chip;
   int n_codes = 0;                  // entries of etab
   std::vector<TeamTask> team;
   std::vector<int> team_inst;       // instance of each task
@@ -1623,7 +1624,9 @@ constexpr size_t TEAM_PHASE_AT = 64;
 size_t team_slots_at(int K) {
   return (TEAM_PHASE_AT + (size_t)K * TEAM_PHASES * sizeof(unsigned long long) + 127) / 128 * 128;
 }
-bool team_on(const cup2d_psb *h) { return h->team_shape >= 0 && !h->team_failed; }
+bool team_on(const cup2d_psb *h) {
+  return h->team_shape >= 0 && !h->team_failed && h->chip.mode != CUP2D_PS_CHIP_OFF;
+}
 
 // Every instance solved on chip (team.hip), a team of workgroups each, in one
 // launch: in start_order, the next instance as workgroups come free.
@@ -1657,13 +1660,14 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   a.start = h->mixed ? TEAM_ACCEPTS : TEAM_CHECKED;
   a.mean_rows = 0;
   a.norm_max = h->cfg.norm == CUP2D_PS_NORM_INF;
-  a.form_polls = TEAM_POLLS << 5;  // a team forms when earlier tasks end
+  a.form_polls = h->chip.polls != TEAM_POLLS ? h->chip.polls : TEAM_POLLS << 5;  // a team forms when earlier tasks end
   a.st = h->d_st;
   a.ctl = reinterpret_cast<int *>(h->d_team);
   a.phase = h->cfg.profile ? reinterpret_cast<unsigned long long *>(h->d_team + TEAM_PHASE_AT) : nullptr;
   a.slots = reinterpret_cast<unsigned long long *>(h->d_team + team_slots_at(K));
   BCHK(h, hipMemcpyAsync(h->d_st, st.data(), K * sizeof(Scal), hipMemcpyHostToDevice, h->stream));
-  BCHK(h, team_launch(a, h->team_shape, h->team_words, h->team_grid, h->stream));
+  const int grid = team_grid(h->chip, h->team_shape, h->team_grid, h->team[0].nwg);
+  BCHK(h, team_launch(a, h->team_shape, h->team_words, grid, h->stream));
   std::vector<unsigned char> words(team_slots_at(K));
   BCHK(h, hipMemcpyAsync(st.data(), h->d_st, K * sizeof(Scal), hipMemcpyDeviceToHost, h->stream));
   BCHK(h, hipMemcpyAsync(words.data(), h->d_team, words.size(), hipMemcpyDeviceToHost, h->stream));
@@ -1709,7 +1713,7 @@ int solve_b_body(cup2d_psb *h, const double *d_b, const double *d_x0, double *d_
     if ((rc = solve_b_team(h, d_b, d_x0, done))) return rc;
     h->team_failed = !done;
   }
-  const bool on_chip = done;
+  const bool on_chip = h->chip.ran = done;
   if (on_chip) {
     BCHK(h, hipMemcpyAsync(d_out, h->d_x, h->n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
   } else {
@@ -2191,6 +2195,13 @@ static int finish_meshes(cup2d_psb *h, int n_inst) {
   h->ready = true;
   return CUP2D_PS_OK;
 }
+
+int cup2d_psb_set_on_chip(cup2d_psb *h, int mode, int form_polls) {
+  if (!h) return bfail(nullptr, CUP2D_PS_EINVAL, "handle is NULL");
+  return team_use_set(h->chip, mode, form_polls) ? CUP2D_PS_OK : bfail(h, CUP2D_PS_EINVAL, "bad mode or poll count");
+}
+
+int cup2d_psb_on_chip(const cup2d_psb *h) { return h && h->chip.ran; }
 
 int cup2d_psb_offsets(const cup2d_psb *h, long long *offsets) {
   if (!h || !offsets) return CUP2D_PS_EINVAL;

@@ -906,6 +906,7 @@ struct cup2d_ps {
   // mesh is too large for it, or a launch failed) and its device words
   int team_shape = -1;
   bool team_failed = false;
+  TeamUse chip;
   TeamTask team{};
   unsigned char *d_team = nullptr;
   int G = 1;                             // workgroups of the SpMV / vector kernels
@@ -1249,7 +1250,9 @@ constexpr double TEAM_TICK_MS = 1e-5;  // wall_clock64: 100 MHz
 constexpr size_t TEAM_PHASE_AT = 64, TEAM_SLOTS_AT = 128;
 constexpr size_t TEAM_BYTES = TEAM_SLOTS_AT + team_words(TEAM_MAX_WG) * 8;
 
-bool team_on(const cup2d_ps *h) { return h->cfg.schedule == 0 && h->team_shape >= 0 && !h->team_failed; }
+bool team_on(const cup2d_ps *h) {
+  return h->cfg.schedule == 0 && h->team_shape >= 0 && !h->team_failed && h->chip.mode != CUP2D_PS_CHIP_OFF;
+}
 
 // The whole solve on chip (team.hip), in FP64.  A mixed handle's solve takes
 // it too -- vectors that never leave the registers gain nothing from FP32
@@ -1283,14 +1286,15 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   a.start = h->mixed ? TEAM_ACCEPTS : TEAM_PLAIN;
   a.mean_rows = h->op.mean_row >= 0;
   a.norm_max = h->cfg.norm == CUP2D_PS_NORM_INF;
-  a.form_polls = TEAM_POLLS;
+  a.form_polls = h->chip.polls;
   a.st = h->d_s;
   a.ctl = reinterpret_cast<int *>(h->d_team);
   a.phase = h->cfg.profile ? reinterpret_cast<unsigned long long *>(h->d_team + TEAM_PHASE_AT) : nullptr;
   a.slots = reinterpret_cast<unsigned long long *>(h->d_team + TEAM_SLOTS_AT);
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
   HIPCHK(h, hipMemcpyAsync(h->d_s, h->h_s, sizeof(Scal), hipMemcpyHostToDevice, h->stream));
-  HIPCHK(h, team_launch(a, h->team_shape, team_words(h->team.nwg), h->team.nwg, h->stream));
+  const int grid = team_grid(h->chip, h->team_shape, h->team.nwg, h->team.nwg);
+  HIPCHK(h, team_launch(a, h->team_shape, team_words(h->team.nwg), grid, h->stream));
   HIPCHK(h, hipEventRecord(h->ev1, h->stream));
   ptick(h, -1);
   HIPCHK(h, hipMemcpyAsync(h->h_s, h->d_s, sizeof(Scal), hipMemcpyDeviceToHost, h->stream));
@@ -1607,6 +1611,7 @@ int solve_impl(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
       if (rc) return rc;
       h->team_failed = !done;
     }
+    h->chip.ran = done;
     if (!done)
       rc = h->cfg.schedule == 1
                  ? solve_unfused(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st)
@@ -1732,6 +1737,7 @@ int solve_noalloc_body(cup2d_ps *h, const double *d_b, double *d_x, double tol_a
     int r = team_on(h) ? solve_team(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st, done) : CUP2D_PS_OK;
     if (r) return r;
     if (team_on(h)) h->team_failed = !done;
+    h->chip.ran = done;
     if (!done) r = solve_fp64(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st);
     if (r) return r;
     // true residual of the returned x: partials of |r|^2, |r|_inf, |b|^2,
@@ -2010,6 +2016,13 @@ static int set_mesh_on_device_body(cup2d_ps *h, const cup2d_mesh_desc *m) {
   h->d_csr_val = nullptr;
   return finish_mesh(h);
 }
+
+int cup2d_ps_set_on_chip(cup2d_ps *h, int mode, int form_polls) {
+  if (!h) return fail(nullptr, CUP2D_PS_EINVAL, "handle is NULL");
+  return team_use_set(h->chip, mode, form_polls) ? CUP2D_PS_OK : fail(h, CUP2D_PS_EINVAL, "bad mode or poll count");
+}
+
+int cup2d_ps_on_chip(const cup2d_ps *h) { return h && h->chip.ran; }
 
 int cup2d_ps_solve_device(cup2d_ps *h, const double *d_b, double *d_x, double tol_abs,
                           double tol_rel, int max_restarts, cup2d_ps_stats *st) {

@@ -7,6 +7,7 @@
 #include <string>
 #include <vector>
 
+#include "../../include/cup2d_chip.h"
 #include "kernels.h"
 
 namespace cup2d {
@@ -88,6 +89,25 @@ constexpr int TEAM_POLLS = 1 << 21;
 // Workgroups of a shape that this device runs at once (0: unknown; the
 // kernels' LDS size is allowed here, so a shape is asked for before its launch).
 int team_resident(int shape);
+
+// What a handle's cup2d_ps_set_on_chip says, and what came of its last solve.
+struct TeamUse {
+  int mode = CUP2D_PS_CHIP_AUTO;
+  int polls = TEAM_POLLS;   // for a team to form
+  bool ran = false;         // the last solve, on chip
+};
+inline bool team_use_set(TeamUse &u, int mode, int polls) {
+  if (mode < CUP2D_PS_CHIP_AUTO || mode > CUP2D_PS_CHIP_SHORT || polls < 0) return false;
+  u.mode = mode;
+  u.polls = polls > 0 ? polls : TEAM_POLLS;
+  return true;
+}
+// Workgroups to launch of a shape: `grid`, whose first team has nwg, or what the
+// mode asks for in their place.
+inline int team_grid(const TeamUse &u, int shape, int grid, int nwg) {
+  return u.mode == CUP2D_PS_CHIP_REFUSED ? team_resident(shape) + 1
+         : u.mode == CUP2D_PS_CHIP_SHORT && nwg > 1 ? nwg - 1 : grid;
+}
 
 // Splits nb blocks over a team of workgroups of at most `most` blocks.
 inline void team_split(int nb, int most, TeamTask &t) {

@@ -29,6 +29,7 @@ from .mesh import BLEN, Mesh
 
 FP64, MIXED = 0, 1
 NORM_INF, NORM_L2 = 0, 1
+CHIP_AUTO, CHIP_OFF, CHIP_REFUSED, CHIP_SHORT = 0, 1, 2, 3  # cup2d_ps_chip
 
 
 def _check(h, rc):
@@ -169,6 +170,16 @@ class Solver:
         return rp, col, val
 
     # -- solve -----------------------------------------------------------
+    def set_on_chip(self, mode=CHIP_AUTO, form_polls=0):
+        """Where solves run: on chip where the mesh fits (default), or by
+        launches per kernel (CHIP_OFF)."""
+        _check(self.h, _lib.load().cup2d_ps_set_on_chip(self.h, int(mode), int(form_polls)))
+        return self
+
+    def on_chip(self):
+        """Whether the last solve ran on chip."""
+        return bool(_lib.load().cup2d_ps_on_chip(self.h))
+
     def solve(self, b, x0=None, tol=0.0, rel_tol=1e-10, max_restarts=100):
         """Host arrays in, (x, stats) out; x is mean-free (ExpAMRSolver.cpp:383-415)."""
         b = np.ascontiguousarray(b, dtype=np.float64)
@@ -399,6 +410,15 @@ class BatchSolver:
         if a is not None:
             return DeviceArray.from_host(self.mem, a)
         return DeviceArray(self.mem, self.n if n is None else n)
+
+    def set_on_chip(self, mode=CHIP_AUTO, form_polls=0):
+        """As Solver.set_on_chip."""
+        _check_b(self.h, _lib.load().cup2d_psb_set_on_chip(self.h, int(mode), int(form_polls)))
+        return self
+
+    def on_chip(self):
+        """Whether the last solve ran on chip."""
+        return bool(_lib.load().cup2d_psb_on_chip(self.h))
 
     def solve(self, b, x0=None, tol=0.0, rel_tol=1e-10, max_restarts=100):
         b = np.ascontiguousarray(b, dtype=np.float64)

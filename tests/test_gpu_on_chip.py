@@ -1,12 +1,20 @@
-"""What a caller sees of the on-chip solve (csrc/team.hip) besides its solution: what a refused call leaves alone."""
+"""What a caller sees of the on-chip solve (csrc/team.hip) besides its solution: what a refused call leaves alone, who
+solves when a launch cannot run, and solves at the same time."""
+
+import ctypes
+import threading
 
 import numpy as np
 import pytest
 
+from cup2d_amd import _lib
+from cup2d_amd import mesh as M
 from cup2d_amd import poisson as PS
 from cup2d_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
+BOTH = pytest.mark.parametrize("precision", [PS.FP64, PS.MIXED])
+POLLS = 4096  # of a wait that is meant to end at its limit: some ms
 
 
 @pytest.mark.parametrize("where", ["b", "x0"])
@@ -25,3 +33,70 @@ def test_refused_mixed_solve_leaves_x(where):
     good = PS.DeviceArray.from_host(s, W.vortex_rhs(m, 2))
     d_x.upload(np.zeros(m.n))
     assert s.solve_device(good, d_x, rel_tol=1e-10)["converged"]
+
+
+def _hand_over(precision, mode, mc=0):
+    """A solve whose launch on chip does not run gives what CHIP_OFF gives, bit for bit, from the x0 it was given."""
+    m = W.graded_disk_mesh()
+    b, x0 = W.vortex_rhs(m, 6), np.random.default_rng(6).normal(size=m.n) * 1e-3
+    s = PS.Solver(norm=PS.NORM_L2, max_iter=4000, precision=precision, mean_constraint=mc).set_mesh(m, on_device=True)
+    ref, st0 = s.set_on_chip(PS.CHIP_OFF).solve(b, x0, rel_tol=1e-10)
+    x, st = s.set_on_chip(mode, POLLS).solve(b, x0, rel_tol=1e-10)
+    assert not s.on_chip() and st["converged"] and st["iterations"] == st0["iterations"]
+    assert np.array_equal(x, ref)
+
+
+def _hand_over_batch(precision, mode):
+    ms = [W.uniform_16x8_mesh(), W.graded_disk_mesh(), M.uniform(1, 1, 1.0)]
+    b = np.concatenate([W.vortex_rhs(m, 30 + k) for k, m in enumerate(ms)])
+    x0 = np.random.default_rng(8).normal(size=b.size) * 1e-3
+    s = PS.BatchSolver(PS.default_config(norm=PS.NORM_L2, max_iter=4000, precision=precision)).set_meshes(ms)
+    ref, st0 = s.set_on_chip(PS.CHIP_OFF).solve(b, x0, rel_tol=1e-10)
+    x, st = s.set_on_chip(mode, POLLS).solve(b, x0, rel_tol=1e-10)
+    assert not s.on_chip() and all(t["converged"] for t in st)
+    assert [t["iterations"] for t in st] == [t["iterations"] for t in st0]
+    assert np.array_equal(x, ref)
+
+
+@pytest.mark.parametrize("mc", [0, 1])
+@BOTH
+def test_short_launch_is_solved_per_kernel(precision, mc):
+    _hand_over(precision, PS.CHIP_SHORT, mc)
+
+
+@BOTH
+def test_short_batch_launch_is_solved_per_kernel(precision):
+    _hand_over_batch(precision, PS.CHIP_SHORT)
+
+
+def test_solves_at_the_same_time():
+    """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
+    ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
+
+    def single(k, mode=PS.CHIP_AUTO):
+        s = PS.Solver(norm=PS.NORM_L2, max_iter=300).set_mesh(ms[k], on_device=True).set_on_chip(mode)
+        b = W.vortex_rhs(ms[k], k)
+        return lambda: (s.solve(b, rel_tol=1e-30)[0], s.on_chip())
+
+    def batch():
+        s = PS.BatchSolver(PS.default_config(norm=PS.NORM_L2, max_iter=300)).set_meshes(ms)
+        b = np.concatenate([W.vortex_rhs(m, k) for k, m in enumerate(ms)])
+        return lambda: (s.solve(b, rel_tol=1e-30)[0], s.on_chip())
+
+    runs = [single(0), single(1), single(2), single(3, PS.CHIP_OFF), batch()]
+    alone = [run() for run in runs]
+    assert [c for _, c in alone] == [True, True, True, False, True]
+    wrong = []
+
+    def work(k):
+        for _ in range(6):
+            x, chip = runs[k]()
+            if not np.array_equal(x, alone[k][0]) or chip != alone[k][1]:
+                wrong.append((k, chip))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(runs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
