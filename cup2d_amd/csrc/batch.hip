@@ -1667,7 +1667,10 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   a.slots = reinterpret_cast<unsigned long long *>(h->d_team + team_slots_at(K));
   BCHK(h, hipMemcpyAsync(h->d_st, st.data(), K * sizeof(Scal), hipMemcpyHostToDevice, h->stream));
   const int grid = team_grid(h->chip, h->team_shape, h->team_grid, h->team[0].nwg);
-  BCHK(h, team_launch(a, h->team_shape, h->team_words, grid, h->stream));
+  if (team_launch(a, h->team_shape, h->team_words, grid, h->stream) != hipSuccess) {
+    (void)hipGetLastError();  // not the next call's: the caller falls back
+    return CUP2D_PS_OK;
+  }
   std::vector<unsigned char> words(team_slots_at(K));
   BCHK(h, hipMemcpyAsync(st.data(), h->d_st, K * sizeof(Scal), hipMemcpyDeviceToHost, h->stream));
   BCHK(h, hipMemcpyAsync(words.data(), h->d_team, words.size(), hipMemcpyDeviceToHost, h->stream));

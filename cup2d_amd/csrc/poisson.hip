@@ -1294,7 +1294,10 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
   HIPCHK(h, hipMemcpyAsync(h->d_s, h->h_s, sizeof(Scal), hipMemcpyHostToDevice, h->stream));
   const int grid = team_grid(h->chip, h->team_shape, h->team.nwg, h->team.nwg);
-  HIPCHK(h, team_launch(a, h->team_shape, team_words(h->team.nwg), grid, h->stream));
+  if (team_launch(a, h->team_shape, team_words(h->team.nwg), grid, h->stream) != hipSuccess) {
+    (void)hipGetLastError();  // not the next call's: the caller falls back
+    return CUP2D_PS_OK;
+  }
   HIPCHK(h, hipEventRecord(h->ev1, h->stream));
   ptick(h, -1);
   HIPCHK(h, hipMemcpyAsync(h->h_s, h->d_s, sizeof(Scal), hipMemcpyDeviceToHost, h->stream));

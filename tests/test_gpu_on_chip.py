@@ -69,6 +69,29 @@ def test_short_batch_launch_is_solved_per_kernel(precision):
     _hand_over_batch(precision, PS.CHIP_SHORT)
 
 
+@pytest.mark.parametrize("mc", [0, 1])
+@BOTH
+def test_refused_launch_is_solved_per_kernel(precision, mc):
+    _hand_over(precision, PS.CHIP_REFUSED, mc)
+
+
+@BOTH
+def test_refused_batch_launch_is_solved_per_kernel(precision):
+    _hand_over_batch(precision, PS.CHIP_REFUSED)
+
+
+def test_refused_noalloc_launch_is_solved_per_kernel():
+    m = W.uniform_16x8_mesh()
+    s = PS.Solver(norm=PS.NORM_L2, max_iter=4000).set_mesh(m, on_device=True).set_on_chip(PS.CHIP_REFUSED)
+    d_b = PS.DeviceArray.from_host(s, W.vortex_rhs(m, 2))
+    d_x, d_y = (PS.DeviceArray.from_host(s, np.zeros(m.n)) for _ in range(2))
+    st = _lib.Stats()
+    assert _lib.load().cup2d_ps_solve_device_noalloc(s.h, d_b.ptr, d_x.ptr, 0.0, 1e-10, 100, ctypes.byref(st)) == 0
+    assert st.converged and not s.on_chip()
+    s.set_on_chip(PS.CHIP_OFF).solve_device(d_b, d_y, rel_tol=1e-10)
+    assert np.array_equal(d_x.numpy(), d_y.numpy())
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
