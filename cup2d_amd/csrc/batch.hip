@@ -1179,7 +1179,6 @@ struct cup2d_psb {
   // the on-chip solve (team.hip): its launch shape (-1: a mesh of the batch is
   // too large for it), the instances' teams in launch order, device words
   int team_shape = -1;
-  bool team_failed = false;
   TeamUse chip;
   int n_codes = 0;                  // entries of etab
   std::vector<TeamTask> team;
@@ -1624,18 +1623,18 @@ constexpr size_t TEAM_PHASE_AT = 64;
 size_t team_slots_at(int K) {
   return (TEAM_PHASE_AT + (size_t)K * TEAM_PHASES * sizeof(unsigned long long) + 127) / 128 * 128;
 }
-bool team_on(const cup2d_psb *h) {
-  return h->team_shape >= 0 && !h->team_failed && h->chip.mode != CUP2D_PS_CHIP_OFF;
-}
 
 // Every instance solved on chip (team.hip), a team of workgroups each, in one
 // launch: in start_order, the next instance as workgroups come free.
 // FP64 throughout; a mixed handle keeps its stopping rule (convergence is
 // accepted on the recomputed FP64 residual).  h_st holds the marker states
 // (instance order) and receives the final ones; the mean-free solutions go to
-// h->d_x.  `done` is false when the launch could not run to its end.
+// h->d_x.  `done` is false when the launch could not run to its end, or is not
+// tried (TeamUse).
 int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done) {
-  done = false;
+  done = h->chip.ran = false;
+  if (h->team_shape < 0 || !h->chip.now()) return CUP2D_PS_OK;
+  h->chip.tried(false);
   const int K = h->K;
   std::vector<Scal> st(K);
   for (int i = 0; i < K; i++) {
@@ -1676,7 +1675,8 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   BCHK(h, hipMemcpyAsync(words.data(), h->d_team, words.size(), hipMemcpyDeviceToHost, h->stream));
   BCHK(h, hipStreamSynchronize(h->stream));
   if (reinterpret_cast<const int *>(words.data())[1]) return CUP2D_PS_OK;
-  done = true;
+  done = h->chip.ran = true;
+  h->chip.tried(true);
   for (int i = 0; i < K; i++) h->h_st[h->team_inst[i]] = st[i];
   if (h->cfg.profile) {
     // the launch's time, split as its teams spent theirs
@@ -1710,13 +1710,9 @@ int solve_b_body(cup2d_psb *h, const double *d_b, const double *d_x0, double *d_
   std::vector<int> iters(K, 0), restarts(K, 0), reps(K, 0), conv(K, 0);
   std::vector<double> err0(K, -1.0), errf(K, 0.0);
   for (int k = 0; k < K; k++) h->h_st[k] = marker_b(h, k, tol_abs, tol_rel, max_restarts, max_iter);
-  int rc = CUP2D_PS_OK;
-  bool done = false;
-  if (team_on(h)) {
-    if ((rc = solve_b_team(h, d_b, d_x0, done))) return rc;
-    h->team_failed = !done;
-  }
-  const bool on_chip = h->chip.ran = done;
+  bool on_chip = false;
+  int rc = solve_b_team(h, d_b, d_x0, on_chip);
+  if (rc) return rc;
   if (on_chip) {
     BCHK(h, hipMemcpyAsync(d_out, h->d_x, h->n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
   } else {
@@ -2098,6 +2094,7 @@ static std::vector<int> start_order(const std::vector<int> &n, const std::vector
 constexpr double TEAM_US[TEAM_SHAPES] = {8.2, 8.9, 10.3, 11.3}, TEAM_US_WG = 0.025;
 static int plan_teams(cup2d_psb *h) {
   h->team_shape = -1;
+  h->chip.new_mesh();
   const int K = h->K;
   long long most = 0;
   for (int k = 0; k < K; k++) most = std::max(most, h->boff[k + 1] - h->boff[k]);

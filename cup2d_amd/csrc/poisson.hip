@@ -903,9 +903,8 @@ struct cup2d_ps {
   double *d_p2 = nullptr, *d_p4 = nullptr, *d_p5 = nullptr, *d_pm = nullptr, *d_pfin = nullptr;
   Scal *h_s = nullptr;                   // pinned copy of the state slots, then of the team's control words
   // the on-chip solve (team.hip): its launch shape for this mesh (-1: the
-  // mesh is too large for it, or a launch failed) and its device words
+  // mesh is too large for it) and its device words
   int team_shape = -1;
-  bool team_failed = false;
   TeamUse chip;
   TeamTask team{};
   unsigned char *d_team = nullptr;
@@ -1250,18 +1249,17 @@ constexpr double TEAM_TICK_MS = 1e-5;  // wall_clock64: 100 MHz
 constexpr size_t TEAM_PHASE_AT = 64, TEAM_SLOTS_AT = 128;
 constexpr size_t TEAM_BYTES = TEAM_SLOTS_AT + team_words(TEAM_MAX_WG) * 8;
 
-bool team_on(const cup2d_ps *h) {
-  return h->cfg.schedule == 0 && h->team_shape >= 0 && !h->team_failed && h->chip.mode != CUP2D_PS_CHIP_OFF;
-}
-
 // The whole solve on chip (team.hip), in FP64.  A mixed handle's solve takes
 // it too -- vectors that never leave the registers gain nothing from FP32
 // storage -- and keeps its stopping rule: convergence is accepted on the
 // recomputed FP64 residual only.  `done` is false when the launch could not
-// run to its end (the caller falls back to the launch-per-kernel solve).
+// run to its end, or is not tried (TeamUse): the caller falls back to the
+// launch-per-kernel solve.
 int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out, double tol_abs,
                double tol_rel, int max_restarts, cup2d_ps_stats *st, bool &done) {
-  done = false;
+  done = h->chip.ran = false;
+  if (h->cfg.schedule != 0 || h->team_shape < 0 || !h->chip.now()) return CUP2D_PS_OK;
+  h->chip.tried(false);
   Scal m = marker_state(h, tol_abs, tol_rel, max_restarts, h->cfg.max_iter);
   m.project = m.stall = 0;
   // A replacement only where convergence is claimed: in a mixed solve, and with
@@ -1304,7 +1302,8 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   HIPCHK(h, hipMemcpyAsync(ctl, h->d_team, TEAM_SLOTS_AT, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   if (ctl[1]) return CUP2D_PS_OK;
-  done = true;
+  done = h->chip.ran = true;
+  h->chip.tried(true);
   const Scal &f = h->h_s[0];
   // a refused solve leaves d_out as it was: nothing is queued that writes it
   if (h->mixed && f.err0 != f.err0) return fail(h, CUP2D_PS_EINVAL, "non-finite residual (NaN/Inf in b or x0)");
@@ -1607,14 +1606,9 @@ int solve_impl(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   HIPCHK(h, hipSetDevice(h->device));
   return guarded(h, [&]() -> int {
     pstart(h);
-    int rc = CUP2D_PS_OK;
     bool done = false;
-    if (team_on(h)) {
-      rc = solve_team(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st, done);
-      if (rc) return rc;
-      h->team_failed = !done;
-    }
-    h->chip.ran = done;
+    int rc = solve_team(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st, done);
+    if (rc) return rc;
     if (!done)
       rc = h->cfg.schedule == 1
                  ? solve_unfused(h, d_b, d_x0, d_out, tol_abs, tol_rel, max_restarts, st)
@@ -1737,10 +1731,8 @@ int solve_noalloc_body(cup2d_ps *h, const double *d_b, double *d_x, double tol_a
   h->cfg.profile = 0;
   int rc = guarded(h, [&]() -> int {
     bool done = false;
-    int r = team_on(h) ? solve_team(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st, done) : CUP2D_PS_OK;
+    int r = solve_team(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st, done);
     if (r) return r;
-    if (team_on(h)) h->team_failed = !done;
-    h->chip.ran = done;
     if (!done) r = solve_fp64(h, d_b, d_x, d_x, tol_abs, tol_rel, max_restarts, st);
     if (r) return r;
     // true residual of the returned x: partials of |r|^2, |r|_inf, |b|^2,
@@ -1913,6 +1905,7 @@ static int set_mesh_body(cup2d_ps *h, const cup2d_mesh_desc *m) {
 constexpr int TEAM_16_MOST = 144;
 static void plan_team(cup2d_ps *h) {
   h->team_shape = -1;
+  h->chip.new_mesh();
   for (int s = 0; s < TEAM_SHAPES; s++) {
     TeamTask t{};
     team_split((int)std::min<long long>(h->op.nb, 1 << 30), team_blocks(s), t);

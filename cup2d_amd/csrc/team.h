@@ -90,11 +90,30 @@ constexpr int TEAM_POLLS = 1 << 21;
 // kernels' LDS size is allowed here, so a shape is asked for before its launch).
 int team_resident(int shape);
 
-// What a handle's cup2d_ps_set_on_chip says, and what came of its last solve.
+// What a handle's cup2d_ps_set_on_chip says, and what came of its last solves.
 struct TeamUse {
   int mode = CUP2D_PS_CHIP_AUTO;
   int polls = TEAM_POLLS;   // for a team to form
   bool ran = false;         // the last solve, on chip
+  int wait = 0, next = 1;   // solves until the chip is tried again, and after the next failure
+
+  // Whether to try the chip for this solve.  After a launch that could not run
+  // (another process's workgroups in the way: a second or two are lost) it is
+  // left out for one solve, then for twice as many each time it fails again: the
+  // cause may pass, and where it stays the attempts become few.
+  bool now() {
+    if (mode == CUP2D_PS_CHIP_OFF) return false;
+    if (wait > 0) {
+      wait--;
+      return false;
+    }
+    return true;
+  }
+  void tried(bool done) {
+    wait = done ? 0 : next;
+    next = done ? 1 : next < 1024 ? 2 * next : next;
+  }
+  void new_mesh() { wait = 0, next = 1; }
 };
 inline bool team_use_set(TeamUse &u, int mode, int polls) {
   if (mode < CUP2D_PS_CHIP_AUTO || mode > CUP2D_PS_CHIP_SHORT || polls < 0) return false;

@@ -92,6 +92,30 @@ def test_refused_noalloc_launch_is_solved_per_kernel():
     assert np.array_equal(d_x.numpy(), d_y.numpy())
 
 
+@pytest.mark.parametrize("mode", [PS.CHIP_SHORT, PS.CHIP_REFUSED])
+def test_a_launch_that_cannot_run_is_not_the_last(mode):
+    """After a launch that could not run the next solve takes the kernels, and then the chip is tried again, after
+    twice as many solves each time it fails; a mesh change tries it at once."""
+    m = W.graded_disk_mesh()
+    b = W.vortex_rhs(m, 6)
+    s = PS.Solver(norm=PS.NORM_L2, max_iter=4000).set_mesh(m)
+    bs = PS.BatchSolver(PS.default_config(norm=PS.NORM_L2, max_iter=4000)).set_meshes([m])
+
+    def on_chip(h, mode=PS.CHIP_AUTO):
+        h.set_on_chip(mode, POLLS).solve(b, rel_tol=1e-10)
+        return h.on_chip()
+
+    for h in (s, bs):
+        assert not on_chip(h, mode)
+        assert [on_chip(h) for _ in range(3)] == [False, True, True]
+        assert not on_chip(h, mode) and not on_chip(h) and not on_chip(h, mode)
+        assert [on_chip(h) for _ in range(3)] == [False, False, True]
+    assert not on_chip(s, mode) and not on_chip(bs, mode)
+    s.set_mesh(m, on_device=True)
+    bs.set_meshes([m], on_device=True)
+    assert on_chip(s) and on_chip(bs)
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
