@@ -1659,7 +1659,7 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   a.start = h->mixed ? TEAM_ACCEPTS : TEAM_CHECKED;
   a.mean_rows = 0;
   a.norm_max = h->cfg.norm == CUP2D_PS_NORM_INF;
-  a.form_polls = h->chip.polls != TEAM_POLLS ? h->chip.polls : TEAM_POLLS << 5;  // a team forms when earlier tasks end
+  a.form_polls = h->chip.polls;
   a.st = h->d_st;
   a.ctl = reinterpret_cast<int *>(h->d_team);
   a.phase = h->cfg.profile ? reinterpret_cast<unsigned long long *>(h->d_team + TEAM_PHASE_AT) : nullptr;
@@ -2139,6 +2139,7 @@ static int plan_teams(cup2d_psb *h) {
     t.e0 = (int)h->eoff[k];
     t.e1 = (int)h->eoff[k + 1];
     t.mean_row = (int)h->h_mean_row[k];
+    t.order = (int)h->team.size();
     tickets += t.nwg;
     words += team_words(t.nwg);
     h->team.push_back(t);

@@ -21,7 +21,7 @@ struct TeamTask {
   int slot0;          // first of the team's exchange words, in units of TEAM_SLOT_WORDS
   int e0, e1;         // explicit rows (ELL slots) of these blocks
   int mean_row;       // replaced row, or -1
-  int pad;
+  int order;          // tasks before this one
 };
 
 constexpr int TEAM_MAX_WG = 256;        // workgroups of a team: at most one per CU
@@ -65,10 +65,10 @@ struct TeamArgs {
   int n_tasks, n_tickets;
   int start;                            // TeamStart
   int mean_rows, norm_max;              // a mean row among the tasks, the infinity norm
-  int form_polls;                       // polls before the wait for a team to form fails
+  int form_polls;                       // polls before the wait for a team to form fails, earlier tasks ended
   Scal *st;                             // [n_tasks] marker state in, final state out
   unsigned long long *slots;            // exchange words of all teams, zero at launch
-  int *ctl;                             // {next ticket, failure}, zero at launch
+  int *ctl;                             // {next ticket, failure, ended tasks}, zero at launch
   unsigned long long *phase;            // [n_tasks][TEAM_PHASES] ticks of 10 ns, or null
 };
 

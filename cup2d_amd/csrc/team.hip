@@ -36,7 +36,9 @@
 // taken in order by running workgroups, so the lowest unfinished task always
 // has or gets its whole team (a cooperative launch: no more workgroups than
 // fit) and every wait ends; a wait beyond its limit marks the launch as
-// failed and every workgroup leaves.
+// failed and every workgroup leaves.  Workgroups that wait for a team to form
+// wait for earlier tasks, however long those run; their limit is for a launch
+// that did not get its workgroups.
 
 #include "team.h"
 
@@ -191,9 +193,15 @@ struct Ctx {
   // the task's halo buffer of this z (halo_face, halo_cell)
   __device__ __forceinline__ double *halo() const { return halo0 + (zp ? (long)HALO_BLOCK * a.A.nb : 0); }
 
-  // every 1024 polls: whether to give up (the launch failed, or the limit)
+  // every 1024 polls: whether to give up (the launch failed, or the limit; a
+  // negative one is that of the wait for the team to form, which counts from the
+  // end of the tasks before it: their workgroups are the ones awaited)
   __device__ __forceinline__ bool give_up(int &n, int limit) {
     if (((++n) & 1023) != 0) return false;
+    if (limit < 0) {
+      limit = -limit;
+      if (__hip_atomic_load(a.ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < t.order) n = 0;
+    }
     if (n < limit && !__hip_atomic_load(a.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
     __hip_atomic_store(a.ctl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s.bad = 1;
@@ -677,7 +685,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
       c.clear();
       c.clear();
       double v[2] = {0.0, 0.0};
-      c.template exchange<2, false>(v, a.form_polls);
+      c.template exchange<2, false>(v, -a.form_polls);
     }
 
     // y = A z; the mean row: sum h^2 z in v[2], the other factor's value there in v[3]
@@ -958,6 +966,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
       o->err = o->err_opt = l2 ? sqrt(size_opt) : size_opt;
       o->err_rep = err_rep;
       o->mean = mean;
+      __hip_atomic_fetch_add(a.ctl + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (prof)
         for (int k = 0; k < TEAM_PHASES; k++) a.phase[(size_t)id * TEAM_PHASES + k] = s.phase[k];
     }
@@ -1004,7 +1013,7 @@ int team_resident(int shape) {
 hipError_t team_launch(const TeamArgs &a, int shape, size_t n_words, int grid, hipStream_t stream) {
   TeamArgs args = a;
   hipError_t e = hipMemsetAsync(a.slots, 0, n_words * sizeof(u64), stream);
-  if (e == hipSuccess) e = hipMemsetAsync(a.ctl, 0, 2 * sizeof(int), stream);
+  if (e == hipSuccess) e = hipMemsetAsync(a.ctl, 0, 3 * sizeof(int), stream);
   if (e != hipSuccess) return e;
   void *params[] = {&args};
   return hipLaunchCooperativeKernel(shape_kernel(shape, a.mean_rows ? MEAN_ROW : a.norm_max ? NORM_MAX : PLAIN), dim3(grid), dim3(shape_threads(shape)),

@@ -116,6 +116,18 @@ def test_a_launch_that_cannot_run_is_not_the_last(mode):
     assert on_chip(s) and on_chip(bs)
 
 
+def test_a_team_waits_for_the_solves_before_it():
+    """Workgroups of a later instance wait as long as earlier ones run, however short the wait for a team is set (an
+    instance of 16,384 blocks and 3000 iterations runs for 50 ms, 4096 polls take a few)."""
+    ms = [M.uniform(128, 128, 16.0), M.uniform(128, 127, 16.0), M.uniform(16, 8, 2.0)]
+    s = PS.BatchSolver(PS.default_config(norm=PS.NORM_L2, max_iter=3000)).set_meshes(ms, on_device=True)
+    b = np.concatenate([W.vortex_rhs(m, k) for k, m in enumerate(ms)])
+    ref = s.solve(b, rel_tol=1e-30)[0]
+    assert s.on_chip()
+    x = s.set_on_chip(PS.CHIP_AUTO, POLLS).solve(b, rel_tol=1e-30)[0]
+    assert s.on_chip() and np.array_equal(x, ref)
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
