@@ -732,7 +732,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           else converged = done = true;
         }
       }
-      if (iter >= max_iter) done = true;
+      if (iter >= max_iter && !replace) done = true;  // a claim made in the last iteration is still confirmed
       const bool breakdown = rho * rho < bd_tol * rr * hh || !(fabs(beta) < 1e30);
       if (__builtin_expect(breakdown && !done && !replace && max_restarts > 0, 0)) {
         restarts++;
@@ -743,7 +743,6 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           hh = rho = rr;  // rhat = r
         }
       }
-      replace = replace && !done;
     };
 
     // Residuals r = b - A x (the start, and the confirmations of a mixed

@@ -128,6 +128,19 @@ def test_a_team_waits_for_the_solves_before_it():
     assert s.on_chip() and np.array_equal(x, ref)
 
 
+@pytest.mark.parametrize("precision,mc", [(PS.MIXED, 0), (PS.MIXED, 1), (PS.FP64, 1), (PS.FP64, 0)])
+@pytest.mark.parametrize("norm", [PS.NORM_L2, PS.NORM_INF])
+def test_converging_in_the_last_iteration_allowed(precision, mc, norm):
+    """Where convergence is confirmed on the residual, that is done after the last iteration too."""
+    m = W.graded_disk_mesh()
+    b = W.vortex_rhs(m, 6)
+    cfg = dict(norm=norm, precision=precision, mean_constraint=mc)
+    x, st = PS.Solver(max_iter=4000, **cfg).set_mesh(m).solve(b, rel_tol=1e-6)
+    assert st["converged"]
+    y, sy = PS.Solver(max_iter=st["iterations"], **cfg).set_mesh(m).solve(b, rel_tol=1e-6)
+    assert sy["converged"] and sy["iterations"] == st["iterations"] and np.array_equal(x, y)
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
