@@ -1251,8 +1251,8 @@ constexpr size_t TEAM_BYTES = TEAM_SLOTS_AT + team_words(TEAM_MAX_WG) * 8;
 
 // The whole solve on chip (team.hip), in FP64.  A mixed handle's solve takes
 // it too -- vectors that never leave the registers gain nothing from FP32
-// storage -- and keeps its stopping rule: convergence is accepted on the
-// recomputed FP64 residual only.  `done` is false when the launch could not
+// storage -- and keeps its rules (solve_mixed): passes of at most max_restarts
+// restarts, convergence on the recomputed FP64 residual only.  `done` is false when the launch could not
 // run to its end, or is not tried (TeamUse): the caller falls back to the
 // launch-per-kernel solve.
 int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out, double tol_abs,
@@ -1281,7 +1281,7 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
   a.one = h->team;
   a.n_tasks = 1;
   a.n_tickets = h->team.nwg;
-  a.start = h->mixed ? TEAM_ACCEPTS : TEAM_PLAIN;
+  a.start = h->mixed ? TEAM_REFINES : TEAM_PLAIN;
   a.mean_rows = h->op.mean_row >= 0;
   a.norm_max = h->cfg.norm == CUP2D_PS_NORM_INF;
   a.form_polls = h->chip.polls;
@@ -1319,7 +1319,7 @@ int solve_team(cup2d_ps *h, const double *d_b, const double *d_x0, double *d_out
     st->converged = f.converged;
     st->refinements = h->mixed ? f.n_rep : 0;
     st->err_init = f.err0;
-    st->err_final = f.rep_factor > 0.0 && f.converged && f.n_rep > 0 ? f.err_rep : f.err_opt;
+    st->err_final = h->mixed || (f.converged && f.n_rep > 0) ? f.err_rep : f.err_opt;
     float ms = 0;
     HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
     st->ms = ms;

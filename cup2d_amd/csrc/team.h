@@ -77,6 +77,9 @@ enum TeamStart {
   TEAM_PLAIN = 0,     // nothing (the FP64 single solve: evaluate alone)
   TEAM_CHECKED = 1,   // a non-finite residual ends the solve, a zero one is convergence
   TEAM_ACCEPTS = 2,   // ... and a start within the tolerance is convergence too
+  TEAM_REFINES = 3,   // ... and the solve is a sequence of passes (iterative refinement): max_restarts
+                      // holds for each, and whatever ends one -- the recurrence's claim, its restarts, the
+                      // iteration cap -- is followed by the residual of the best iterate
 };
 
 // Blocks per workgroup of a launch shape.

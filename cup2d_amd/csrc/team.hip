@@ -150,6 +150,7 @@ struct Shared {
                                     // 16), place in the halo buffer / 8}
   u64 tick, phase[TEAM_PHASES];     // of the profile: not in registers, which the loop needs
   int ng, ni, nf, nw, ticket, bad;  // ghosts, items, explicit rows with ghosts, wide ones
+  int restarts;                     // of the passes before this one
 };
 
 // The running workgroup: what its functions share.
@@ -487,7 +488,7 @@ struct Ctx {
 
   // Headers, ghosts and explicit rows of the workgroup's blocks.
   __device__ __forceinline__ void lay_out() {
-    if (tid == 0) s.ng = s.ni = s.nf = s.nw = 0;
+    if (tid == 0) s.ng = s.ni = s.nf = s.nw = s.restarts = 0;
     __syncthreads();
     // LDS index of 8 cells of another workgroup, from `first` of the halo buffer on
     auto ghosts = [&](int first) -> int {
@@ -732,12 +733,13 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
           else converged = done = true;
         }
       }
-      if (iter >= max_iter && !replace) done = true;  // a claim made in the last iteration is still confirmed
+      // (a claim made in the last iteration is still confirmed)
+      if (iter >= max_iter && !replace) (a.start == TEAM_REFINES ? replace : done) = true;
       const bool breakdown = rho * rho < bd_tol * rr * hh || !(fabs(beta) < 1e30);
       if (__builtin_expect(breakdown && !done && !replace && max_restarts > 0, 0)) {
         restarts++;
         if (restarts >= max_restarts) {
-          done = true;
+          (a.start == TEAM_REFINES ? replace : done) = true;
         } else {
           restart = true;
           hh = rho = rr;  // rhat = r
@@ -782,6 +784,10 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
       err = uni(norm_of(size));
       if (replace) {
         n_rep++;
+        if (a.start == TEAM_REFINES) {  // the next pass counts its own
+          if (tid == 0) s.restarts += restarts;
+          restarts = 0;
+        }
       } else {
         err0 = err;
         // sizes above this have not converged (the test itself is exact)
@@ -798,7 +804,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
         if (err != err || err > 1.79e308) {
           done = true;
           converged = false;
-        } else if (!replace && (err == 0.0 || (a.start == TEAM_ACCEPTS && (err <= tol_abs || tol_rel >= 1.0)))) {
+        } else if (!replace && (err == 0.0 || (a.start >= TEAM_ACCEPTS && (err <= tol_abs || tol_rel >= 1.0)))) {
           converged = done = true;
         }
       }
@@ -956,7 +962,7 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
     if (c.rank == 0 && tid == 0) {
       Scal *o = a.st + id;
       o->iter = iter;
-      o->restarts = restarts;
+      o->restarts = s.restarts + restarts;
       o->n_rep = n_rep;
       o->converged = converged;
       o->improved = improved;

@@ -141,6 +141,29 @@ def test_converging_in_the_last_iteration_allowed(precision, mc, norm):
     assert sy["converged"] and sy["iterations"] == st["iterations"] and np.array_equal(x, y)
 
 
+def test_mixed_solve_recomputes_the_residual_at_its_end():
+    m = W.graded_disk_mesh()
+    b = W.vortex_rhs(m, 6)
+    for mode in (PS.CHIP_OFF, PS.CHIP_AUTO):
+        s = PS.Solver(norm=PS.NORM_L2, precision=PS.MIXED, max_iter=25).set_mesh(m).set_on_chip(mode)
+        x, st = s.solve(b, rel_tol=1e-10)
+        assert st["iterations"] == 25 and not st["converged"] and st["refinements"] >= 1
+        assert abs(st["err_final"] - st["true_rel2"] * np.linalg.norm(b)) <= 1e-9 * st["err_final"]
+
+
+@pytest.mark.parametrize("breakdown_tol,max_restarts", [(1e-2, 20), (1e-6, 5), (1e-8, 2)])
+def test_mixed_restarts_are_counted_by_pass(breakdown_tol, max_restarts):
+    """A mixed solve that has used up its restarts recomputes the residual and goes on (64 passes at most), on chip as
+    by launches per kernel."""
+    m = W.graded_disk_mesh()
+    b = W.vortex_rhs(m, 3)
+    for mode in (PS.CHIP_OFF, PS.CHIP_AUTO):
+        s = PS.Solver(norm=PS.NORM_L2, precision=PS.MIXED, breakdown_tol=breakdown_tol, max_iter=4000).set_mesh(m)
+        x, st = s.set_on_chip(mode).solve(b, rel_tol=1e-10, max_restarts=max_restarts)
+        assert st["restarts"] > max_restarts
+        assert st["refinements"] == 64 or (st["converged"] and st["true_rel2"] <= 1.05e-10)
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
