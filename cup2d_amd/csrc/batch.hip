@@ -1187,7 +1187,6 @@ struct cup2d_psb {
   int team_grid = 0, n_tickets = 0;
   TeamTask *d_task = nullptr;
   unsigned char *d_team = nullptr;  // control words, phase times [K], exchange words
-  double *d_halo = nullptr;         // [3 n]
   int *d_all_done = nullptr;
   int *h_all_done = nullptr;        // pinned
   std::vector<Scal> h_st;
@@ -1650,7 +1649,7 @@ int solve_b_team(cup2d_psb *h, const double *d_b, const double *d_x0, bool &done
   a.b = d_b;
   a.x0 = d_x0;
   a.out = h->d_x;
-  a.halo = h->d_halo;
+  a.halo = (double *)h->v_r;  // the Krylov vectors of the item kernels: 7 n values, 3 n doubles and more
   a.xopt = h->d_xopt;
   a.n_codes = h->n_codes;
   a.task = h->d_task;
@@ -2150,8 +2149,7 @@ static int plan_teams(cup2d_psb *h) {
   h->team_grid = std::min(grid, tickets);
   int rc;
   if ((rc = bupload(h, h->allocs, &h->d_task, h->team)) ||
-      (rc = balloc(h, h->allocs, &h->d_team, team_slots_at(K) + h->team_words * sizeof(unsigned long long))) ||
-      (rc = balloc(h, h->allocs, &h->d_halo, 3 * (size_t)h->n)))
+      (rc = balloc(h, h->allocs, &h->d_team, team_slots_at(K) + h->team_words * sizeof(unsigned long long))))
     return rc;
   return CUP2D_PS_OK;
 }
@@ -2173,10 +2171,11 @@ static int finish_meshes(cup2d_psb *h, int n_inst) {
   for (double **v : dv)
     if ((rc = balloc(h, pool, v, n))) return rc;
   void **kv[] = {&h->v_r, &h->v_rhat, &h->v_p, &h->v_nu, &h->v_z1, &h->v_z2, &h->v_t};
+  char *krylov = nullptr;  // one buffer: the on-chip solve's halo takes it
+  if ((rc = balloc(h, pool, &krylov, 7 * n * es))) return rc;
   for (void **v : kv) {
-    char *p = nullptr;
-    if ((rc = balloc(h, pool, &p, n * es))) return rc;
-    *v = p;
+    *v = krylov;
+    krylov += n * es;
   }
   if ((rc = balloc(h, pool, &h->d_st, (size_t)n_inst)) || (rc = balloc(h, pool, &h->d_all_done, 1)) ||
       (rc = balloc(h, pool, &h->d_rt, 4 * (size_t)n_inst)))

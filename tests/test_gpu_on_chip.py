@@ -164,6 +164,25 @@ def test_mixed_restarts_are_counted_by_pass(breakdown_tol, max_restarts):
         assert st["refinements"] == 64 or (st["converged"] and st["true_rel2"] <= 1.05e-10)
 
 
+def _free():
+    """Free bytes of the device, by the HIP runtime that the library has loaded."""
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("precision,bound", [(PS.FP64, 96), (PS.MIXED, 68)])
+def test_batch_memory(precision, bound):
+    """Device memory per unknown: b, x, the best iterate, the host interface's copy and seven Krylov vectors (8 or 4
+    bytes), and the operator (1-2 bytes on a uniform mesh)."""
+    ms = [M.uniform(128, 128, 16.0)] * 16
+    s = PS.BatchSolver(PS.default_config(precision=precision))
+    free = _free()
+    s.set_meshes(ms)
+    assert free - _free() <= bound * s.n
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
