@@ -113,8 +113,7 @@ __device__ __forceinline__ double dpp_total(double v) {
 }
 
 // A word of z that has not arrived: a signalling NaN, which no arithmetic
-// returns (an x0 that holds this very one fails the launch, not the solve:
-// the launch-per-kernel path takes over).
+// returns.
 constexpr u64 EMPTY = 0x7ff4c2d0a11c0de5ull;
 
 constexpr int face_rows(int blocks) { return blocks * 28; }  // a block has 28 cells on its faces
@@ -677,7 +676,8 @@ __global__ __launch_bounds__(WGS, WGS > 512 ? WGS / 256 : 2) void k_team(TeamArg
 #pragma unroll
     for (int tt = 0; tt < T; tt++) {
 #pragma unroll
-      for (int k = 0; k < 4; k++) x[tt][k] = a.x0[c.cell(tt) + k];  // the caller's arrays: 8-byte aligned
+      for (int k = 0; k < 4; k++)  // the caller's arrays: 8-byte aligned; x0's NaNs are made quiet (EMPTY is none)
+        x[tt][k] = __builtin_canonicalize(a.x0[c.cell(tt) + k]);
       if (c.ok(tt)) st4(a.xopt, c.cell(tt), x[tt]);
       else x[tt][0] = x[tt][1] = x[tt][2] = x[tt][3] = 0.0;
     }

@@ -183,6 +183,15 @@ def test_batch_memory(precision, bound):
     assert free - _free() <= bound * s.n
 
 
+def test_x0_of_marker_words():
+    """x0 may hold any word, also the NaN that marks halo words which have not arrived."""
+    m = W.uniform_16x8_mesh()
+    x0 = np.full(m.n, 0x7ff4c2d0a11c0de5, np.uint64).view(np.float64)
+    s = PS.Solver(norm=PS.NORM_L2, max_iter=50).set_mesh(m)
+    x, st = s.solve(W.vortex_rhs(m, 2), x0, rel_tol=1e-10)
+    assert s.on_chip() and not st["converged"]
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
