@@ -101,7 +101,8 @@ struct TeamUse {
   int wait = 0, next = 1;   // solves until the chip is tried again, and after the next failure
 
   // Whether to try the chip for this solve.  After a launch that could not run
-  // (another process's workgroups in the way: a second or two are lost) it is
+  // (the runtime refuses cooperative launches while another process makes them,
+  // which takes it some ms; a wait that ends at its limit takes a second) it is
   // left out for one solve, then for twice as many each time it fails again: the
   // cause may pass, and where it stays the attempts become few.
   bool now() {

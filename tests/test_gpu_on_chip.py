@@ -2,6 +2,9 @@
 solves when a launch cannot run, and solves at the same time."""
 
 import ctypes
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -223,3 +226,27 @@ def test_solves_at_the_same_time():
     for t in threads:
         t.join()
     assert not wrong
+
+
+PROCESS = """
+import numpy as np
+from cup2d_amd import mesh as M, poisson as PS, workloads as W
+bx, by = %d, %d
+m = M.uniform(bx, by, extent=max(bx, by) / 8.0)
+s = PS.Solver(norm=PS.NORM_L2, max_iter=4000).set_mesh(m, on_device=True)
+b = W.vortex_rhs(m, 1)
+for k in range(20):
+    x, st = s.solve(b, rel_tol=1e-10)
+    assert st["converged"] and st["true_rel2"] <= 1.05e-10, st
+print("solved")
+"""
+
+
+def test_processes_at_the_same_time():
+    """The runtime may refuse a process's launches on chip while another one has them (an error of state): its solves
+    run by launches per kernel then."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    ps = [subprocess.Popen([sys.executable, "-c", PROCESS % g], cwd=root, stdout=subprocess.PIPE,
+                           stderr=subprocess.STDOUT, text=True) for g in ((16, 8), (64, 64), (91, 90), (128, 96))]
+    out = [p.communicate(timeout=100)[0] for p in ps]
+    assert all(p.returncode == 0 and "solved" in o for p, o in zip(ps, out)), out
