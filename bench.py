@@ -9,19 +9,24 @@ the 64x64 block-Jacobi preconditioner, b and x resident in HBM.  `value` is
 FP64 solves per second over the timed steps.  Prints one JSON line.
 
 Also measured in the same run (all in `config`):
-* the same batch in mixed precision (FP32 Krylov vectors, BF16 MFMA
-  preconditioner, FP64 residual replacement), and the like-for-like
-  mixed / FP64 batched ratio;
+* the same batch in mixed precision, and the like-for-like mixed / FP64
+  batched ratio (`on_chip` true: both are the FP64 kernel that solves an
+  instance in registers, the mixed handle with its own stopping rule; false:
+  FP32 Krylov vectors, BF16 MFMA preconditioner, FP64 residual replacement);
 * the same 64 solves one after another with the single-solve FP64 solver,
-  fused (graph-replayed) and unfused (one operation per launch, the
-  reference GPU loop's structure): the denominators of the batch speedups;
+  fused (on chip) and unfused (one operation per launch, the reference GPU
+  loop's structure): the denominators of the batch speedups;
 * every instance's FP64 true residual, and the error of the FP64 and the
   mixed solutions against the oracle's FP64 solve on a sample of instances;
 * the single-mesh workloads (3-level graded mesh, 1448 blocks; 6-level
   mesh, 16,229 blocks) in FP64 and mixed precision;
-* `roofline`: the dominant batched FP64 iteration kernel, timed live with
-  HIP events on the solver's stream, with the counted HBM traffic of the
-  committed rocprofv3 summary; the batched SpMV on its minimal bytes;
+* `roofline`: the dominant batched FP64 iteration kernel of the batches that
+  are not solved on chip (an instance beyond 16,384 blocks, the mean-row form),
+  timed live with HIP events on the solver's stream, with the counted HBM
+  traffic of the committed rocprofv3 summary; the batched SpMV on its minimal
+  bytes.  `fp64_iteration_kernels`, `mixed_iteration_kernels`, `item_blocks`,
+  `xcd_run`, `ms_per_iteration_tuned` and `work_proportional_ms` are of that path
+  too, and `graph` applies to it alone;
 * `cpu_baseline`: the oracle's restatement of the reference CPU solver
   (pipelined BiCGSTAB with the block-Cholesky preconditioner,
   AMRSolver.cpp:149-490) on a bounded sample of the same instances, OpenMP
@@ -255,7 +260,7 @@ def timed_batch(PS, meshes, b, precision, steps, warmup, use_graph, profile=0):
     w_its = float(np.dot(its, nbk) / nbk.sum())
     res = {"solves_per_s": len(meshes) * steps / tot, "ms_per_batch": tot * 1e3 / steps,
            "ms_per_batch_median": float(np.median(t)) * 1e3,
-           "set_meshes_ms_device_assembly": setup_ms, "item_blocks": ib, "xcd_run": bs.xcd_run(),
+           "on_chip": bs.on_chip(), "set_meshes_ms_device_assembly": setup_ms, "item_blocks": ib, "xcd_run": bs.xcd_run(),
            "ms_per_iteration_tuned": ms_it,
            "iterations_max": int(its.max()), "iterations_mean": float(its.mean()),
            "iterations_mean_weighted_by_blocks": w_its,
@@ -268,7 +273,7 @@ def timed_batch(PS, meshes, b, precision, steps, warmup, use_graph, profile=0):
 
 def sequential(PS, meshes, rhs, schedule, use_graph):
     """The batch's solves one after another with the single-solve FP64
-    solver (schedule 0: fused, graph-replayed; 1: one operation per launch,
+    solver (schedule 0: fused, on chip; 1: one operation per launch,
     the reference GPU loop's structure).  One warm-up solve per mesh."""
     s = PS.Solver(norm=PS.NORM_L2, max_iter=4000, use_graph=use_graph, schedule=schedule)
     tot, iters, conv = 0.0, [], True
@@ -277,7 +282,7 @@ def sequential(PS, meshes, rhs, schedule, use_graph):
         d_b = PS.DeviceArray.from_host(s, bb)
         d_x = PS.DeviceArray(s, m.n)
         d_x.upload(np.zeros(m.n))
-        s.solve_device(d_b, d_x, rel_tol=1e-10)  # warm-up (graph capture)
+        s.solve_device(d_b, d_x, rel_tol=1e-10)  # warm-up
         d_x.upload(np.zeros(m.n))
         t0 = time.perf_counter()
         st = s.solve_device(d_b, d_x, rel_tol=1e-10)
@@ -314,7 +319,7 @@ def bench_single(PS, W, mesh, b, steps, use_graph):
         xs[name] = d_x.numpy()
         out[name] = {"solves_per_s": 1.0 / sec, "ms_per_solve": sec * 1e3, "set_mesh_ms": setup_ms,
                      "iterations": st["iterations"], "refinements": st["refinements"],
-                     "restarts": st["restarts"], "converged": st["converged"],
+                     "restarts": st["restarts"], "converged": st["converged"], "on_chip": s.on_chip(),
                      "true_rel2_residual": st["true_rel2"]}
         if name == "fp64":
             out["fp64"]["kernel_ms"] = [s.kernel_time(k, reps=100) for k in range(5)]
@@ -442,7 +447,7 @@ def cylinder_flow(PS, W, steps, precision, cpu_steps=0, adapt_every=0):
             "rel_l2_v": float(np.linalg.norm(gv - v) / np.linalg.norm(v)),
             "rel_l2_p": float(np.linalg.norm(gp - p) / np.linalg.norm(p))}
     flow = FLOW.CylinderFlow(m, precision=precision, rel_tol=1e-10, adapt_every=adapt_every)
-    flow.step()  # untimed first step (graph capture of the solver's iteration chunks)
+    flow.step()  # untimed first step
     its, nbs = [], []
     t0 = time.perf_counter()
     for _ in range(steps):
@@ -547,16 +552,51 @@ def kernel_only(PS, W, which, reps):
                           "bytes_read": s.n * 8, "bytes_written": s.n * 8,
                           "GB_per_s": 16 * s.n / (ms * 1e-3) / 1e9}))
         return
+    if which == "on_chip":
+        # `reps` solves on chip of 400 iterations each, on five meshes and the
+        # 64-instance batch in this order: us per iteration, and of the profiled
+        # solves the first workgroup's time in each phase
+        from cup2d_amd import mesh as M
+        out = []
+        for m in (W.uniform_16x8_mesh(), W.graded_disk_mesh(), M.uniform(96, 64, 12.0), W.cylinder_mesh(),
+                  W.four_disk_amr6_mesh()):
+            b = W.workload_rhs(m, 3)
+            for profile in (0, 1):
+                s = PS.Solver(norm=PS.NORM_L2, max_iter=400, profile=profile).set_mesh(m, on_device=True)
+                d_b, d_x = PS.DeviceArray.from_host(s, b), PS.DeviceArray(s, m.n)
+                ms = []
+                for _ in range(reps):
+                    d_x.upload(np.zeros(m.n))
+                    st = s.solve_device(d_b, d_x, rel_tol=1e-30)
+                    ms.append(st["ms"])
+                assert s.on_chip()
+                us = 1e3 / st["iterations"]
+                if not profile:
+                    out.append({"blocks": m.n_blocks, "iterations": st["iterations"], "us_per_iteration": min(ms) * us})
+                else:
+                    out[-1]["us_by_phase"] = {k: v * us for k, v in st["ms_phase"].items()}
+        meshes = W.batch64_meshes()
+        b = np.concatenate([W.workload_rhs(m, 400 + k) for k, m in enumerate(meshes)])
+        bs = PS.BatchSolver(PS.default_config(norm=PS.NORM_L2, max_iter=400)).set_meshes(meshes, on_device=True)
+        d_b, d_x = bs.device_array(b), bs.device_array()
+        for _ in range(reps):
+            d_x.upload(np.zeros_like(b))
+            st = bs.solve_device(d_b, d_x, rel_tol=1e-30)
+        assert bs.on_chip()
+        out.append({"blocks": bs.n // 64, "instances": len(meshes), "iterations": max(s["iterations"] for s in st),
+                    "ms": st[0]["ms"]})
+        print(json.dumps({"kernel": "k_team", "solves": out}))
+        return
     if which in ("batch_fp64", "batch_mixed"):
-        # 64 iterations of the batched solve (every instance running), plain
-        # stream launches so that each kernel is traced: the batched iteration
-        # kernels at their real shape
+        # 64 iterations of the batched solve (every instance running) by the item
+        # kernels, plain stream launches so that each is traced: the batched
+        # iteration kernels at their real shape
         meshes = W.batch64_meshes()
         b = np.concatenate([W.workload_rhs(m, 400 + k) for k, m in enumerate(meshes)])
         cfg = PS.default_config(precision=PS.FP64 if which == "batch_fp64" else PS.MIXED,
                                 max_iter=64, norm=PS.NORM_L2, use_graph=0)
         cfg.item_blocks = 32
-        bs = PS.BatchSolver(cfg).set_meshes(meshes)
+        bs = PS.BatchSolver(cfg).set_meshes(meshes).set_on_chip(PS.CHIP_OFF)
         d_b = bs.device_array(b)
         d_x = bs.device_array(np.zeros_like(b))
         st = bs.solve_device(d_b, d_x, rel_tol=1e-14)
@@ -618,16 +658,18 @@ def main():
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline and oracle-error legs")
     ap.add_argument("--spmv-reps", type=int, default=50)
     ap.add_argument("--graph", type=int, default=1,
-                    help="1: replay iteration chunks from a hipGraph; 0: plain stream launches")
+                    help="1: replay iteration chunks from a hipGraph; 0: plain stream launches "
+                         "(solves that do not run on chip)")
     ap.add_argument("--no-extra", action="store_true",
                     help="skip the sequential solves and the single-mesh workloads")
-    modes = ["spmv", "batch_spmv", "batch_fp64", "batch_mixed", "copy", "assembly", "projection", "flow"]
+    modes = ["spmv", "batch_spmv", "batch_fp64", "batch_mixed", "copy", "assembly", "projection", "flow", "on_chip"]
     modes += [f"{p}iter{k}" for p in ("", "x", "a", "b", "m") for k in range(5)]
     ap.add_argument("--kernel-only", choices=modes, default=None,
                     help="profiling aid: launch only this kernel --steps times and exit "
                          "(spmv: operator on the 3-level mesh; batch_spmv: batched operator on the "
                          "64-instance batch; batch_fp64 / batch_mixed: 64 iterations of the "
-                         "batched solve, every kernel launched from the stream; iterK: iteration "
+                         "batched solve by the item kernels, launched from the stream; on_chip: solves of "
+                         "400 iterations on chip, five meshes and the batch; iterK: iteration "
                          "kernel K of the 3-level mesh's solve (xiterK: mixed; aiterK: FP64 on the 6-level mesh); biterK / miterK: batched FP64 / "
                          "mixed iteration kernel K with every instance iterating; copy: the "
                          "library's streaming copy over 13,881,344 doubles, the bandwidth ceiling "
@@ -722,6 +764,7 @@ def main():
             "algorithmic_bytes": kern[dom]["algorithmic_bytes"],
             "ms_per_launch": kern[dom]["ms_per_launch"],
             "profile": "profiles/roofline_batch.md, profiles/pmc_traffic.txt",
+            "on_chip": False,  # the timed solves run k_team instead: profiles/team_kernel.md
         },
         "roofline_spmv": batch_spmv_roofline(PS, meshes, args.spmv_reps),
     }

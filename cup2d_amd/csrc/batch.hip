@@ -2098,8 +2098,8 @@ static int plan_teams(cup2d_psb *h) {
   long long most = 0;
   for (int k = 0; k < K; k++) most = std::max(most, h->boff[k + 1] - h->boff[k]);
   // The mean-row form takes the item kernels: its runs are long, chaotic and full
-  // of restarts, and on chip one of 64 claimed convergence with a recurrence's
-  // residual 6x below the true one (theirs: within 1.1x).
+  // of restarts, the recurrence's residual may drift from the true one (solve_team
+  // in poisson.hip), and FP64 batches have no confirmation of it.
   if (most > TEAM_MAX_BLOCKS || h->cfg.mean_constraint) return CUP2D_PS_OK;
   std::vector<int> order;
   double best = 0.0;

@@ -195,6 +195,18 @@ def test_x0_of_marker_words():
     assert s.on_chip() and not st["converged"]
 
 
+@pytest.mark.parametrize("rel_tol", [1e-13, 1e-14, 1e-15])
+def test_mean_row_below_the_attainable_residual(rel_tol):
+    """FP64 convergence is the recurrence's (as BiCGSTAB.cu:572-593), also where rounding keeps the residual itself
+    from following: on chip as by launches per kernel, and with no larger residual there."""
+    for m in (W.uniform_16x8_mesh(), W.graded_disk_mesh(), W.batch64_meshes()[0]):
+        b = W.vortex_rhs(m, 3)
+        st = [PS.Solver(norm=PS.NORM_L2, mean_constraint=1, max_iter=4000).set_mesh(m, on_device=True)
+              .set_on_chip(mode).solve(b, rel_tol=rel_tol)[1] for mode in (PS.CHIP_OFF, PS.CHIP_AUTO)]
+        assert st[0]["converged"] and st[1]["converged"]
+        assert st[1]["true_rel2"] <= st[0]["true_rel2"]
+
+
 def test_solves_at_the_same_time():
     """Handles on threads of their own, on chip and not, a batch among them: what each gives alone."""
     ms = [M.uniform(16, 8, 2.0), M.uniform(128, 96, 16.0), W.graded_disk_mesh(), M.uniform(91, 90, 12.0)]
