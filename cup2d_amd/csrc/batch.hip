@@ -42,6 +42,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -2051,30 +2052,25 @@ static int build_device(cup2d_psb *h, int n_inst, const cup2d_mesh_desc *meshes)
 // 14 % with the largest instances first.
 static std::vector<int> start_order(const std::vector<int> &n, const std::vector<double> &d, int grid, double &end) {
   const int K = (int)n.size();
-  std::vector<int> left(K), order;
-  for (int k = 0; k < K; k++) left[k] = k;
-  std::stable_sort(left.begin(), left.end(), [&](int a, int b) { return n[a] > n[b]; });
+  std::vector<int> order;
+  std::map<int, std::vector<int>, std::greater<int>> left;  // by workgroups, each in reverse
+  for (int k = K - 1; k >= 0; k--) left[n[k]].push_back(k);
   std::multimap<double, int> running;  // end of an instance, its workgroups
   double t = 0.0;
   int free = grid;
   end = 0.0;
   while (!left.empty()) {
-    size_t kept = 0;
-    for (size_t i = 0; i < left.size(); i++) {
-      const int k = left[i];
-      if (n[k] <= free) {
-        free -= n[k];
-        running.emplace(t + d[k], n[k]);
+    for (auto w = left.lower_bound(free); w != left.end() && free > 0;) {
+      while (!w->second.empty() && w->first <= free) {
+        const int k = w->second.back();
+        w->second.pop_back();
+        free -= w->first;
+        running.emplace(t + d[k], w->first);
         end = std::max(end, t + d[k]);
         order.push_back(k);
-      } else {
-        left[kept++] = k;
       }
-      if (free == 0) {
-        for (i++; i < left.size(); i++) left[kept++] = left[i];
-      }
+      w = w->second.empty() ? left.erase(w) : std::next(w);
     }
-    left.resize(kept);
     if (running.empty()) break;  // an instance wider than the grid: the caller has ruled it out
     t = running.begin()->first;
     free += running.begin()->second;
