@@ -1160,10 +1160,12 @@ struct cup2d_psb {
   unsigned long long *d_mask = nullptr;
   int *d_erow = nullptr, *d_ecol = nullptr;
   uint16_t *d_ecode = nullptr;
-  double *d_etab = nullptr, *d_h2 = nullptr, *d_P = nullptr;
-  double *d_pc = nullptr;           // MFMA fragments of P_inv's classes (make_pclass64)
+  double *d_etab = nullptr, *d_h2 = nullptr;
   std::vector<uint8_t> elen;        // [n_exc] entries of each explicit row
   int ell_w = 0;
+  // the handle's copy of P_inv, whatever the meshes (one buffer): FP64 MFMA
+  // fragments, those of its classes (make_pclass64), BF16 ones
+  double *d_P = nullptr, *d_pc = nullptr;
   bf16x8 *d_pfrag = nullptr;
   long long *d_mean_row = nullptr;
   double *d_h = nullptr;            // [nb] cell size per block
@@ -1856,6 +1858,7 @@ int cup2d_psb_destroy(cup2d_psb *h) {
   bfree_pool(h->unit_allocs);
   bfree_pool(h->allocs);
   bfree_pool(h->spare);
+  if (h->d_P) (void)hipFree(h->d_P);
   if (h->h_all_done) (void)hipHostFree(h->h_all_done);
   for (hipEvent_t e : h->pev) (void)hipEventDestroy(e);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
@@ -2158,10 +2161,14 @@ static int finish_meshes(cup2d_psb *h, int n_inst) {
   static const std::vector<double> P = make_pinv();  // the same for every mesh
   static const std::vector<uint16_t> pf = make_pfrag(P);
   static const std::vector<double> pf64 = make_pfrag64(P), pc64 = make_pclass64(P);
-  if ((rc = bupload(h, pool, &h->d_P, pf64)) || (rc = bupload(h, pool, &h->d_pc, pc64)) || (rc = bupload(h, pool, &h->d_mean_row, h->h_mean_row)))
-    return rc;
-  if ((rc = balloc(h, pool, &h->d_pfrag, pf.size() / 8))) return rc;
-  BCHK(h, hipMemcpy(h->d_pfrag, pf.data(), pf.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  if (!h->d_P) {  // ... and this handle's copy on the device is made once
+    double *d = nullptr;
+    BCHK(h, upload_pinv(pf64, pc64, pf, d));
+    h->d_P = d;
+    h->d_pc = d + pf64.size();
+    h->d_pfrag = reinterpret_cast<bf16x8 *>(h->d_pc + pc64.size());
+  }
+  if ((rc = bupload(h, pool, &h->d_mean_row, h->h_mean_row))) return rc;
   const size_t n = (size_t)h->n, es = h->mixed ? sizeof(float) : sizeof(double);
   double **dv[] = {&h->d_x, &h->d_xopt, &h->d_b, &h->d_xio};
   for (double **v : dv)

@@ -885,6 +885,7 @@ struct cup2d_ps {
   bool has_csr = false;                  // plain CSR copy present (host-assembled meshes)
   int *d_csr_rp = nullptr, *d_csr_col = nullptr;
   double *d_csr_val = nullptr;
+  // the handle's copy of P_inv, whatever the mesh (one buffer)
   double *d_P = nullptr;                 // FP64 MFMA fragments of P_inv (make_pfrag64)
   double *d_pc = nullptr;                // of its classes (make_pclass64)
   bf16x8 *d_pf = nullptr;                // BF16 MFMA fragments of P_inv
@@ -1829,6 +1830,7 @@ int cup2d_ps_destroy(cup2d_ps *h) {
   free_mesh(h);
   for (const DevBuf &b : h->spare) (void)hipFree(b.p);
   h->spare.clear();
+  if (h->d_P) (void)hipFree(h->d_P);
   if (h->h_s) (void)hipHostFree(h->h_s);
   for (hipEvent_t e : h->pev) (void)hipEventDestroy(e);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
@@ -1930,8 +1932,13 @@ static int finish_mesh(cup2d_ps *h) {
   static const std::vector<double> P = make_pinv();  // the same for every mesh
   static const std::vector<uint16_t> pf = make_pfrag(P);
   static const std::vector<double> pf64 = make_pfrag64(P), pc64 = make_pclass64(P);
-  if ((rc = upload(h, &h->d_P, pf64)) || (rc = upload(h, &h->d_pc, pc64)) || (rc = dalloc(h, &h->d_pf, 8 * 64))) return rc;
-  HIPCHK(h, hipMemcpy(h->d_pf, pf.data(), pf.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  if (!h->d_P) {  // ... and this handle's copy on the device is made once
+    double *d = nullptr;
+    HIPCHK(h, upload_pinv(pf64, pc64, pf, d));
+    h->d_P = d;
+    h->d_pc = d + pf64.size();
+    h->d_pf = reinterpret_cast<bf16x8 *>(h->d_pc + pc64.size());
+  }
   const size_t n = op.n;
   double **vecs[] = {&h->d_x, &h->d_xopt, &h->d_r, &h->d_rhat, &h->d_p, &h->d_nu, &h->d_b, &h->d_xio};
   for (double **v : vecs)

@@ -4,7 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
-#include <string>
+#include <cstdint>
+#include <cstring>
 #include <vector>
 
 #include "../../include/cup2d_chip.h"
@@ -138,6 +139,23 @@ inline void team_split(int nb, int most, TeamTask &t) {
   t.nwg = (nb + most - 1) / most;
   t.bpw = (nb + t.nwg - 1) / t.nwg;
   t.nwg = (nb + t.bpw - 1) / t.bpw;
+}
+
+// The fragments of P_inv (make_pfrag64, make_pclass64, make_pfrag) in one new
+// buffer on the device, in this order; nothing is left of it where that fails.
+inline hipError_t upload_pinv(const std::vector<double> &f64, const std::vector<double> &c64,
+                              const std::vector<uint16_t> &f16, double *&out) {
+  std::vector<double> all(f64);
+  all.insert(all.end(), c64.begin(), c64.end());
+  const size_t n = all.size(), bytes = n * sizeof(double) + f16.size() * sizeof(uint16_t);
+  all.resize((bytes + sizeof(double) - 1) / sizeof(double));
+  std::memcpy(all.data() + n, f16.data(), f16.size() * sizeof(uint16_t));
+  double *d = nullptr;
+  hipError_t e = hipMalloc((void **)&d, bytes);
+  if (e == hipSuccess) e = hipMemcpy(d, all.data(), bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess) out = d;
+  else if (d) (void)hipFree(d);
+  return e;
 }
 
 // Launches the solves on `stream` with `grid` workgroups, no more than
