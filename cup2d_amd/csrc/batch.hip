@@ -11,11 +11,12 @@
 // workgroups taking the next.  64 instances of 512-8,192 blocks (13.9 million
 // cells) to 1e-12: 290 ms, by the item kernels 915 ms; 9 small ones in mixed
 // precision 13 ms against 53.4 ms.  What bounds it: the workgroups' own work and
-// the waits of a team (15 us an iteration on 64 blocks; 3,389 workgroups' worth
+// the waits of a team (15 us an iteration on 64 blocks; 3,418 workgroups' worth
 // of instances on 256).
 //
-// A batch with a larger instance, or in the mean-row form, takes the item
-// kernels, which advance all unfinished instances at once:
+// A batch with a larger instance, or in the mean-row form, or whose launch on
+// chip could not run, takes the item kernels, which advance all unfinished
+// instances at once:
 //
 //  * work units: "items" (a run of up to `ib` blocks of one instance) for the
 //    SpMV and vector kernels, a workgroup per item; "tiles" (16 blocks of one
@@ -28,7 +29,7 @@
 //    workgroup per instance re-reduces that instance's item partials in a
 //    fixed order and advances its scalar recurrence (deterministic, no
 //    atomics or fences).
-//  * the item size `ib` is picked by a timing autotuner and cached per
+//  * the item size `ib` can be picked by a timing autotuner and is cached per
 //    batch shape.
 //
 // Precisions of the item kernels: FP64, or FP32-stored Krylov vectors with

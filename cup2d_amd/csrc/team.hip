@@ -23,7 +23,10 @@
 // explicit row needs lies in LDS, and the addresses of a thread's halo words
 // in registers.  What is the same in every lane is kept in scalar registers
 // (uni): in vector ones the vectors were spilled to memory (64 blocks per
-// workgroup: 20.5 us on 16,384 blocks, 17.6 without).
+// workgroup: 20.5 us on 16,384 blocks, 17.6 without).  There are too many of
+// them: 129-184 scalar registers are spilled to lanes of vector ones, whose
+// reloads lie in the loop, and 8-24 bytes a lane of flags to memory; of the
+// vectors the 48-block shape spills 2 registers (12 with the infinity norm).
 //
 // Measured (us per iteration to a relative residual of 1e-12, against five
 // kernels per iteration replayed from a graph): 128 blocks 7.7 against 24.0,

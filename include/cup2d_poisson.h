@@ -55,7 +55,10 @@ typedef struct {
 
 typedef struct {
   int device;             /* HIP device ordinal */
-  int precision;          /* cup2d_ps_precision */
+  int precision;          /* cup2d_ps_precision.  CUP2D_PS_MIXED: FP32 Krylov vectors and a BF16
+                             preconditioner inside FP64 iterative refinement; a solve on chip
+                             (cup2d_chip.h) is FP64 throughout and keeps the refinement's rules:
+                             passes, convergence on the recomputed FP64 residual */
   int mean_constraint;    /* bMeanConstraint (SimulationData.h:98): 0 = post-hoc mean removal only,
                              nonzero = the (0,0) row of the corner block is replaced by
                              sum h^2 x = 0 (BiCGSTAB.cu:393-409) */
@@ -71,7 +74,8 @@ typedef struct {
                              elsewhere kernels are launched one by one between HIP events;
                              0 = off */
   int item_blocks;        /* batch handles: blocks per work item, 1..256; 0 = the value tuned in
-                             this process for the batch's shape, else 8 */
+                             this process for the batch's shape, else 8 (batches that are not
+                             solved on chip, as xcd_run) */
   int schedule;           /* 0 = fused kernels (default); 1 = one operation per launch with a
                              host check of the stopping norm every iteration, the structure of the
                              reference GPU loop (BiCGSTAB.cu:412-620), FP64 single solves only: the
@@ -85,7 +89,8 @@ typedef struct {
   double breakdown_tol;   /* restart when rho^2 < breakdown_tol |r|^2 |rhat|^2 (BiCGSTAB.cu:483) */
   double inner_tol;       /* mixed precision: the FP32 recurrence residual may fall to inner_tol
                              times the last FP64 residual before the residual is recomputed in
-                             FP64 and BiCGSTAB restarts from the best iterate; 0 = 1e-2 */
+                             FP64 and BiCGSTAB restarts from the best iterate; 0 = 1e-2
+                             (not on chip: there is no FP32 recurrence) */
   double reserved_d[5];
 } cup2d_ps_config;
 
@@ -95,7 +100,8 @@ typedef struct {
   int converged;          /* 1 when the stopping test was met; 0 returns the best iterate x_opt */
   int refinements;        /* FP64 residual updates (mixed precision) */
   double err_init;        /* stopping norm of r0 = b - A x0 */
-  double err_final;       /* stopping norm of the returned iterate (recurrence residual) */
+  double err_final;       /* stopping norm of the returned iterate (recurrence residual; single
+                             mixed solves: the residual recomputed after the last pass) */
   double ms;              /* wall time of the solve on the handle's stream, ms */
   double true_rel2;       /* |b - A x|_2 / |b|_2 of the returned x, recomputed in FP64 on the device
                              after the solve (b's mean row taken as 0 with mean_constraint) */
@@ -389,7 +395,8 @@ int cup2d_psb_solve_device(cup2d_psb *h, const double *d_b, double *d_x, double 
  * (plain order, or runs of 4 .. 32 consecutive items per XCD) -- on
  * right-hand side d_b, keeps the fastest (also for later handles of this
  * process with the same precision and batch shape) and reports its item
- * size and ms per iteration.  No counterpart in the reference. */
+ * size and ms per iteration.  Of use to batches that are not solved on chip
+ * (cup2d_chip.h).  No counterpart in the reference. */
 int cup2d_psb_autotune(cup2d_psb *h, const double *d_b, int *item_blocks, double *ms_per_iter);
 /* Blocks per work item in use. */
 int cup2d_psb_item_blocks(const cup2d_psb *h);
