@@ -23,8 +23,9 @@ typedef enum {
                                 the others' wait for it ends at its limit */
 } cup2d_ps_chip;
 
-/* Sets the mode of a handle's solves from now on.  form_polls: polls (0.5 us and
- * more each) a workgroup waits for the others to be there; 0 = the default, 2^21. */
+/* Sets the mode of a handle's solves from now on.  form_polls: polls (0.15-0.25 us
+ * each) a workgroup waits for the others to be there, once the instances of a batch
+ * before its own have ended; 0 = the default, 2^21. */
 int cup2d_ps_set_on_chip(cup2d_ps *h, int mode, int form_polls);
 int cup2d_psb_set_on_chip(cup2d_psb *h, int mode, int form_polls);
 
