@@ -17,7 +17,7 @@ from cup2d_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 BOTH = pytest.mark.parametrize("precision", [PS.FP64, PS.MIXED])
-POLLS = 4096  # of a wait that is meant to end at its limit: some ms
+POLLS = 4096  # of a wait that is meant to end at its limit: 1 ms
 
 
 @pytest.mark.parametrize("where", ["b", "x0"])
@@ -120,9 +120,9 @@ def test_a_launch_that_cannot_run_is_not_the_last(mode):
 
 
 def test_a_team_waits_for_the_solves_before_it():
-    """Workgroups of a later instance wait as long as earlier ones run, however short the wait for a team is set (an
-    instance of 16,384 blocks and 3000 iterations runs for 50 ms, 4096 polls take a few)."""
-    ms = [M.uniform(128, 128, 16.0), M.uniform(128, 127, 16.0), M.uniform(16, 8, 2.0)]
+    """The first instance takes 200 of 256 workgroups for 3000 iterations, 50 ms; the others take tickets of the second,
+    which has 100, and wait for the rest however short the wait for a team is set (4096 polls: 1 ms)."""
+    ms = [M.uniform(128, 100, 16.0), M.uniform(80, 80, 10.0), M.uniform(16, 8, 2.0)]
     s = PS.BatchSolver(PS.default_config(norm=PS.NORM_L2, max_iter=3000)).set_meshes(ms, on_device=True)
     b = np.concatenate([W.vortex_rhs(m, k) for k, m in enumerate(ms)])
     ref = s.solve(b, rel_tol=1e-30)[0]
